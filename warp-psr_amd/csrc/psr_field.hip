@@ -43,45 +43,111 @@ __global__ void k_cumulative(FieldIndex f, int d, const T* __restrict__ coef, T*
 
 template <class T> PSR_HD int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-// field.py:371-393 (add_level)
-template <class T>
-__device__ __forceinline__ void add_level(const FieldIndex& f, const T* coef, T p0, T p1, T p2, int d, T* res) {
-  const int n = 1 << d;
-  const T t[3] = {p0 * T(n), p1 * T(n), p2 * T(n)};
-  int cell[3], base[3];
+// Node words of levels 0..word_depth from the concatenated sorted keys: the
+// first key of each word (a key whose predecessor lies in another word)
+// collects the word's following keys, at most 32, so no two threads write one
+// word.  Words without keys keep the cleared value (no bits).
+__global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int word_depth, NodeWord* __restrict__ words) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t key = keys[i];
+  const int d = key_d(key);
+  if (d > word_depth) return;
+  if (i > 0 && (keys[i - 1] >> 5) == (key >> 5)) return;  // z is the key's lowest field
+  uint32_t bits = 0;
+  for (int64_t j = i; j < n && (keys[j] >> 5) == (key >> 5); ++j) bits |= 1u << (int)(keys[j] & 31);
+  const int dim = (1 << d) + 1;
+  words[word_base(d) + (uint32_t)(key_x(key) * dim + key_y(key)) * (uint32_t)word_columns(d) + (uint32_t)(key_z(key) >> 5)] =
+      NodeWord{bits, (int32_t)i};
+}
+
+// One level's eight trilinear corners of a cube point: cell, weights and
+// coefficient indices (-1 absent or left of the point's floor).
+template <class T> struct Corners {
+  int idx[8];
   T fr[3];
+  bool up[3];  // cell + 1 > floor: the upper corner has weight fr, else 1 - fr
+};
+
+// field.py:371-393 (add_level), lookups only
+template <class T, bool WORDS>
+__device__ __forceinline__ void find_corners(const FieldIndex& f, const T* p, int d, Corners<T>& c) {
+  const int n = 1 << d;
+  int cell[3], base[3];
+#pragma unroll
   for (int a = 0; a < 3; ++a) {
-    cell[a] = clampi<T>((int)ceil(t[a]) - 1, 0, n - 1);
-    base[a] = (int)floor(t[a]);
-    fr[a] = t[a] - T(base[a]);
+    const T t = p[a] * T(n);
+    cell[a] = clampi<T>((int)ceil(t) - 1, 0, n - 1);
+    base[a] = (int)floor(t);
+    c.fr[a] = t - T(base[a]);
+    c.up[a] = cell[a] + 1 > base[a];
   }
-  int64_t found[2][2][2];
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) level_run<2>(f, d, cell[0] + a, cell[1] + b, cell[2], 2, found[a][b]);
-  for (int corner = 0; corner < 8; ++corner) {
-    const int node[3] = {cell[0] + corner / 4, cell[1] + (corner / 2) % 2, cell[2] + corner % 2};
-    if (imin(imin(node[0] - base[0], node[1] - base[1]), node[2] - base[2]) < 0) continue;
-    const int64_t idx = found[corner / 4][(corner / 2) % 2][corner % 2];
-    if (idx < 0) continue;
-    T h[3], sg[3];
-    for (int a = 0; a < 3; ++a) {
-      h[a] = T(1) - fr[a];
-      sg[a] = T(-1);
-      if (node[a] > base[a]) { h[a] = fr[a]; sg[a] = T(1); }
+  if constexpr (WORDS) {
+    const int wc = word_columns(d);
+    const NodeWord* at = f.words + word_base(d) + (uint32_t)(cell[0] * (n + 1) + cell[1]) * (uint32_t)wc + (uint32_t)(cell[2] >> 5);
+    // the upper node's word: the same one, except at a word's end (then the
+    // next word of the column, which exists because cell + 1 <= 2^d)
+    const int next = ((cell[2] + 1) >> 5) - (cell[2] >> 5);
+    NodeWord lo[4], hi[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const NodeWord* w = at + (k / 2 * (n + 1) + k % 2) * wc;
+      lo[k] = w[0];
+      hi[k] = w[next];
     }
-    const T c = coef[idx];
-    res[0] = res[0] + c * h[0] * h[1] * h[2];
-    res[1] = res[1] + c * T(n) * sg[0] * h[1] * h[2];
-    res[2] = res[2] + c * T(n) * h[0] * sg[1] * h[2];
-    res[3] = res[3] + c * T(n) * h[0] * h[1] * sg[2];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      c.idx[2 * k] = node_in_word(lo[k], cell[2]);
+      c.idx[2 * k + 1] = node_in_word(hi[k], cell[2] + 1);
+    }
+  } else {
+    for (int a = 0; a < 2; ++a)
+      for (int b = 0; b < 2; ++b) {
+        int64_t found[2];
+        level_run<2>(f, d, cell[0] + a, cell[1] + b, cell[2], 2, found);
+        c.idx[4 * a + 2 * b] = (int)found[0];
+        c.idx[4 * a + 2 * b + 1] = (int)found[1];
+      }
+  }
+  // a corner left of the point's floor (a knot owned by the left cell) does not count
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+    if (imin(imin(cell[0] + k / 4 - base[0], cell[1] + k / 2 % 2 - base[1]), cell[2] + k % 2 - base[2]) < 0) c.idx[k] = -1;
+}
+
+// field.py:371-393 (add_level), sums only, corners in order.  An absent
+// corner enters as the coefficient +0: its products are zeros of either sign,
+// and a sum that starts at +0 is never -0, so adding them changes no bit.
+template <class T>
+__device__ __forceinline__ void blend_corners(const Corners<T>& c, const T* v, int d, T* res) {
+  const T n = T(1 << d);
+  T h[3][2], sg[3][2];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {  // lower corner: node <= floor, upper corner: by `up`
+    h[a][0] = T(1) - c.fr[a];
+    sg[a][0] = T(-1);
+    h[a][1] = c.up[a] ? c.fr[a] : T(1) - c.fr[a];
+    sg[a][1] = c.up[a] ? T(1) : T(-1);
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int x = k / 4, y = k / 2 % 2, z = k % 2;
+    res[0] = res[0] + v[k] * h[0][x] * h[1][y] * h[2][z];
+    res[1] = res[1] + v[k] * n * sg[0][x] * h[1][y] * h[2][z];
+    res[2] = res[2] + v[k] * n * h[0][x] * sg[1][y] * h[2][z];
+    res[3] = res[3] + v[k] * n * h[0][x] * h[1][y] * sg[2][z];
   }
 }
 
-// field.py:395-420 (reference evaluation kernel)
-template <class T>
-__global__ void k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth, const T* __restrict__ queries, int64_t m, Affine<T> A,
-                           int point_div_mode, const T* __restrict__ divisors, T* __restrict__ values, T* __restrict__ grads,
-                           int* __restrict__ valid) {
+// field.py:395-420 (reference evaluation kernel).  WORDS: every level has
+// node words, so the three dependent steps (leaf words, the three blended
+// levels' words, their coefficients) each issue all their loads at once; the
+// general form searches level by level.
+template <class T, bool WORDS>
+__global__ void __launch_bounds__(256) k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth,
+                                                  const T* __restrict__ queries, int64_t m, Affine<T> A, int point_div_mode,
+                                                  const T* __restrict__ divisors, T* __restrict__ values, T* __restrict__ grads,
+                                                  int* __restrict__ valid) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= m) return;
   T q0 = queries[3 * i], q1 = queries[3 * i + 1], q2 = queries[3 * i + 2];
@@ -100,29 +166,66 @@ __global__ void k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __
     return;
   }
   int leaf = 0;
-  for (int d = depth; d >= 0; --d) {
-    const int n = 1 << d;
-    const int c0 = clampi<T>((int)ceil(p[0] * T(n)) - 1, 0, n - 1);
-    const int c1 = clampi<T>((int)ceil(p[1] * T(n)) - 1, 0, n - 1);
-    const int c2 = clampi<T>((int)ceil(p[2] * T(n)) - 1, 0, n - 1);
-    int64_t idx;
-    level_run<1>(f, d, c0, c1, c2, 1, &idx);
-    if (idx >= 0) { leaf = d; break; }
+  if constexpr (WORDS) {
+    // the cell at level d is the finest cell >> (depth - d): scaling by a
+    // power of two is exact and ceil(ceil(m) / 2^k) = ceil(m / 2^k)
+    const int nf = 1 << depth;
+    int cf[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) cf[a] = clampi<T>((int)ceil(p[a] * T(nf)) - 1, 0, nf - 1);
+    constexpr int AHEAD = 4;  // levels whose words are loaded together
+    bool found = false;
+    for (int top = depth; top >= 0 && !found; top -= AHEAD) {
+      NodeWord w[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) {
+        const int d = imax(top - k, 0), up = depth - d;
+        const int x = cf[0] >> up, y = cf[1] >> up, z = cf[2] >> up;
+        w[k] = f.words[word_base(d) + (uint32_t)(x * ((1 << d) + 1) + y) * (uint32_t)word_columns(d) + (uint32_t)(z >> 5)];
+      }
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) {
+        const int d = imax(top - k, 0);
+        if (!found && ((w[k].bits >> ((cf[2] >> (depth - d)) & 31)) & 1u)) { leaf = d; found = true; }
+      }
+    }
+  } else {
+    for (int d = depth; d >= 0; --d) {
+      const int n = 1 << d;
+      const int c0 = clampi<T>((int)ceil(p[0] * T(n)) - 1, 0, n - 1);
+      const int c1 = clampi<T>((int)ceil(p[1] * T(n)) - 1, 0, n - 1);
+      const int c2 = clampi<T>((int)ceil(p[2] * T(n)) - 1, 0, n - 1);
+      int64_t idx;
+      level_run<1>(f, d, c0, c1, c2, 1, &idx);
+      if (idx >= 0) { leaf = d; break; }
+    }
   }
   for (int a = 0; a < 3; ++a) {
     if (p[a] == T(0)) p[a] = T(1e-6);
     else if (p[a] == T(1)) p[a] = T(1.0 - 1e-6);
   }
+  const bool lower = leaf > 0, upper = leaf < depth;
+  Corners<T> c0, c1, c2;
+  find_corners<T, WORDS>(f, p, leaf, c0);
+  find_corners<T, WORDS>(f, p, imax(leaf - 1, 0), c1);
+  find_corners<T, WORDS>(f, p, imin(leaf + 1, depth), c2);
+  T v0[8], v1[8], v2[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    v0[k] = c0.idx[k] >= 0 ? coef[c0.idx[k]] : T(0);
+    v1[k] = lower && c1.idx[k] >= 0 ? cum[c1.idx[k]] : T(0);
+    v2[k] = upper && c2.idx[k] >= 0 ? coef[c2.idx[k]] : T(0);
+  }
   T res[4] = {T(0), T(0), T(0), T(0)};
-  add_level(f, coef, p[0], p[1], p[2], leaf, res);
-  if (leaf > 0) {
+  blend_corners(c0, v0, leaf, res);
+  if (lower) {
     T r2[4] = {T(0), T(0), T(0), T(0)};
-    add_level(f, cum, p[0], p[1], p[2], leaf - 1, r2);
+    blend_corners(c1, v1, leaf - 1, r2);
     for (int a = 0; a < 4; ++a) res[a] = res[a] + r2[a];
   }
-  if (leaf < depth) {
+  if (upper) {
     T r2[4] = {T(0), T(0), T(0), T(0)};
-    add_level(f, coef, p[0], p[1], p[2], leaf + 1, r2);
+    blend_corners(c2, v2, leaf + 1, r2);
     for (int a = 0; a < 4; ++a) res[a] = res[a] + r2[a];
   }
   values[i] = res[0];
@@ -286,16 +389,37 @@ template <class T> void reference_inverse(const T* m, T* out) {
 
 
 template <class T>
+static void launch_evaluate(const Result<T>& r, const T* queries, int64_t m, const Affine<T>& A, int point_div_mode,
+                            const T* divisors, T* values, T* grads, int* valid, hipStream_t s) {
+  if (m <= 0) return;
+  const int depth = r.prm.depth;
+  auto kernel = r.word_depth >= depth ? k_evaluate<T, true> : k_evaluate<T, false>;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(m, 256)), dim3(256), 0, s, field_index(r), (const T*)r.coefficients.data(),
+                     (const T*)r.cumulative.data(), depth, queries, m, A, point_div_mode, divisors, values, grads, valid);
+  KERNEL_CHECK();
+}
+
+template <class T>
 void evaluate_field(const Result<T>& r, const T* queries, int64_t m, const T* linear, const T* translation, T* values, T* grads,
                     int* valid, hipStream_t s) {
   if (m <= 0) return;
   Affine<T> A;
   for (int k = 0; k < 9; ++k) A.L[k] = linear[k];
   for (int k = 0; k < 3; ++k) A.t[k] = translation[k];
-  hipLaunchKernelGGL(k_evaluate<T>, dim3(blocks_for(m, 256)), dim3(256), 0, s, field_index(r),
-                     (const T*)r.coefficients.data(), (const T*)r.cumulative.data(), r.prm.depth,
-                     queries, m, A, 0, (const T*)nullptr, values, grads, valid);
-  KERNEL_CHECK();
+  launch_evaluate(r, queries, m, A, 0, (const T*)nullptr, values, grads, valid, s);
+}
+
+// Deepest level with node words: the lookup-table limits' dense one (depth 9
+// by default; word_base is defined up to there), at most the field's depth.
+static int field_word_depth(int depth) {
+  const int64_t cells = dense_index_max_cells();
+  int d = -1;
+  for (int e = 0; e <= imin(depth, 9); ++e) {
+    const int64_t dim = ((int64_t)1 << e) + 1;
+    if (dim * dim * dim > cells) break;
+    d = e;
+  }
+  return d;
 }
 
 template <class T> void stage_field(Result<T>& r) {
@@ -321,7 +445,21 @@ template <class T> void stage_field(Result<T>& r) {
   }
   r.offsets_dev.reset(D + 2, s);
   HIP_CHECK(hipMemcpyAsync(r.offsets_dev.data(), r.level_offsets.data(), sizeof(int) * (D + 2), hipMemcpyHostToDevice, s));
-  if (D <= field_table_max_depth() && K) {
+  // lookup tables: node words for the levels within the dense limit, column
+  // tables where deeper levels remain, else searches of the keys
+  const bool tables = D <= field_table_max_depth() && K;
+  r.word_depth = tables ? field_word_depth(D) : -1;
+  if (r.word_depth >= 0) {
+    r.node_words.reset(word_base(r.word_depth) + ((size_t)1 + ((size_t)1 << r.word_depth)) * ((1 << r.word_depth) + 1) *
+                                                     word_columns(r.word_depth), s);
+    r.node_words.zero();
+    hipLaunchKernelGGL(k_field_words, dim3(blocks_for(K, 256)), dim3(256), 0, s, (const int64_t*)r.keys.data(), K, r.word_depth,
+                       r.node_words.data());
+    KERNEL_CHECK();
+  } else {
+    r.node_words.free();
+  }
+  if (tables && r.word_depth < D) {
     const size_t cells = (size_t)column_base(D + 1);
     r.column_start.reset(cells, s);
     r.column_end.reset(cells, s);
@@ -350,11 +488,8 @@ template <class T> void stage_field(Result<T>& r) {
   Affine<T> I;
   for (int k = 0; k < 9; ++k) I.L[k] = (k % 4 == 0) ? T(1) : T(0);
   for (int k = 0; k < 3; ++k) I.t[k] = T(0);
-  hipLaunchKernelGGL(k_evaluate<T>, dim3(blocks_for(G, 256)), dim3(256), 0, s, f, (const T*)r.coefficients.data(),
-                     (const T*)r.cumulative.data(), D,
-                     (const T*)r.position_sums.data(), (int64_t)G, I, 1, (const T*)r.weights.data(), r.centroid_values.data(),
-                     (T*)nullptr, (int*)nullptr);
-  KERNEL_CHECK();
+  launch_evaluate(r, (const T*)r.position_sums.data(), (int64_t)G, I, 1, (const T*)r.weights.data(), r.centroid_values.data(),
+                  (T*)nullptr, (int*)nullptr, s);
   DArray<T> iso(1, s);
   compute_isovalue((const T*)r.centroid_values.data(), (const T*)r.weights.data(), (int64_t)G, iso.data(), s);
   read_bytes(&r.iso, iso.data(), sizeof(T), s);

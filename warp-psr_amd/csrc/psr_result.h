@@ -6,6 +6,14 @@
 
 namespace psr {
 
+// Presence of 32 z-consecutive nodes of one (x, y) column of a level and the
+// concatenated index of the word's first present node: a lookup is one 8-byte
+// load and a population count, because keys are sorted with z fastest.
+struct NodeWord {
+  uint32_t bits;
+  int32_t first;
+};
+
 struct Params {
   int depth = 6, full_depth = 3, base_depth = 3, solve_depth = 6, kernel_depth = 4;
   double samples_per_node = 1.5, scale = 1.1, point_weight = 2.0;
@@ -106,8 +114,14 @@ template <class T> struct Result {
   DArray<T> coefficients, cumulative, centroid_values;
   std::vector<int> level_offsets;  // concatenated key offsets per depth
   DArray<int> offsets_dev;         // the same on the device
+  // node words of levels 0..word_depth of keys, level after level, x-major
+  // (2^d + 1)^2 columns of ceil((2^d + 1) / 32) words each: 41 MB at depth 9,
+  // deeper levels have none (see field_word_depth)
+  DArray<NodeWord> node_words;
+  int word_depth = -1;
   // (x, y) column runs of every level of keys (absolute indices), laid out
-  // level after level with (2^d + 1)^2 cells each; empty above depth 11
+  // level after level with (2^d + 1)^2 cells each; only for fields with
+  // levels beyond word_depth, empty above depth 11
   DArray<int> column_start, column_end;
   T iso;
   T cube_to_model[16], model_to_cube[16];
