@@ -1422,16 +1422,17 @@ __device__ __forceinline__ int ring_of(int v, int t0, int ts) {
 
 // Tiles of row j's slice whose ring-4 region holds it: flags (FLAG), counts,
 // or the sort keys (compact tile << 3 | category) and values (j) from
-// count[j] on (EMIT).
+// count[j] on (EMIT).  flip = 3 files colour 3 - c as category c: the tables
+// of the reverse sweeps, which update the colours in the opposite order.
 template <int MODE>  // 0 flag, 1 count, 2 emit
-__global__ void k_tile_members(const int* __restrict__ order, const int64_t* __restrict__ keys, int R, int ts, int nt,
+__global__ void k_tile_members(const int* __restrict__ order, const int64_t* __restrict__ keys, int R, int ts, int nt, int flip,
                                int* __restrict__ flags, const int* __restrict__ compact, int* __restrict__ count,
                                uint32_t* __restrict__ out_keys, int* __restrict__ out_vals) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= R) return;
   const int64_t k = keys[order[j]];
   const int x = key_x(k), y = key_y(k), z = key_z(k);
-  const int colour = (x & 1) + 2 * (y & 1);
+  const int colour = ((x & 1) + 2 * (y & 1)) ^ flip;
   const int tx0 = max(0, (x - 4) / ts), tx1 = min(nt - 1, (x + 4) / ts);
   const int ty0 = max(0, (y - 4) / ts), ty1 = min(nt - 1, (y + 4) / ts);
   int c = 0, pos = MODE == 2 ? count[j] : 0;
@@ -1532,7 +1533,7 @@ struct TileCell {
 
 template <bool EMIT>
 __device__ __forceinline__ TileCell tile_cell(const int* __restrict__ dense, int dim, int n, int z, int ox, int oy, int ts,
-                                              int g, int w, const int* __restrict__ inv) {
+                                              int g, int w, int flip, const int* __restrict__ inv) {
   TileCell c{0, 0, -1, false};
   if (w >= g * g) return c;
   const int lx = w / g, ly = w - (w / g) * g;
@@ -1542,7 +1543,7 @@ __device__ __forceinline__ TileCell tile_cell(const int* __restrict__ dense, int
   if (i < 0) return c;
   c.present = true;
   const int r = max(ring_of(x, ox + 4, ts), ring_of(y, oy + 4, ts));
-  const int colour = (x & 1) + 2 * (y & 1);
+  const int colour = ((x & 1) + 2 * (y & 1)) ^ flip;
   c.cat = r <= 3 - colour ? colour : -1;
   if (EMIT) {
     c.j = inv[i];
@@ -1553,7 +1554,7 @@ __device__ __forceinline__ TileCell tile_cell(const int* __restrict__ dense, int
 
 __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int* __restrict__ dense, int dim, int n,
                                                                         const int* __restrict__ dense_of, int nt, int ts,
-                                                                        int* __restrict__ counts) {
+                                                                        int flip, int* __restrict__ counts) {
   __shared__ int total[5];
   const int t = blockIdx.x, tid = threadIdx.x;
   if (tid < 5) total[tid] = 0;
@@ -1563,7 +1564,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int
   const int ox = tx * ts - 4, oy = ty * ts - 4, g = ts + 8;
   int cnt[5] = {0, 0, 0, 0, 0};
   for (int w = tid; w < g * g; w += TILE_SCAN_THREADS) {
-    const TileCell c = tile_cell<false>(dense, dim, n, z, ox, oy, ts, g, w, nullptr);
+    const TileCell c = tile_cell<false>(dense, dim, n, z, ox, oy, ts, g, w, flip, nullptr);
     if (!c.present) continue;
     if (c.cat >= 0) ++cnt[c.cat];
     ++cnt[4];
@@ -1577,7 +1578,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int
 
 __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_emit(const int* __restrict__ dense, int dim, int n,
                                                                        const int* __restrict__ dense_of, int nt, int ts,
-                                                                       const int* __restrict__ inv, const int* __restrict__ offs,
+                                                                       int flip, const int* __restrict__ inv, const int* __restrict__ offs,
                                                                        int2* __restrict__ entries) {
   constexpr int WAVES = TILE_SCAN_THREADS / 64;
   __shared__ int base[5];
@@ -1590,7 +1591,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_emit(const int*
   const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
   __syncthreads();
   for (int w0 = 0; w0 < g * g; w0 += TILE_SCAN_THREADS) {
-    const TileCell c = tile_cell<true>(dense, dim, n, z, ox, oy, ts, g, w0 + tid, inv);
+    const TileCell c = tile_cell<true>(dense, dim, n, z, ox, oy, ts, g, w0 + tid, flip, inv);
     int pre[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -1663,6 +1664,28 @@ template <class T, class V> struct TiledArgs {
   int g;  // grid side, ts + 8
 };
 
+// What one wave of the tiled sweeps computes.  RELAX: a relaxation wave.
+// SNAP: the same, each new x also written to snap[visit R + position].
+// REVERSE: a wave of the sweeps' adjoint.  Row i's update
+// x_i += (b_i - sum_c A_ic x_c) / A_ii has the adjoint r_i = g_i / A_ii,
+// g_c -= A_ic r_i for every c (i too) and gb_i += r_i, in the opposite order
+// of the updates.  Gathered instead of scattered: between two reverse updates
+// of row i each neighbour c was reversed exactly once, so
+//   g_i = h_i - sum_{c != i} A_ci r_c,  r_i = g_i / A_ii,  h_i = g_i - A_ii r_i
+// with the latest r of every neighbour (h starts as the gradient of the final
+// x, r as 0).  That is a relaxation wave over r with the transposed operator,
+// visits, slices and colours all counted from the other end; h moves between
+// two buffers with r, because neighbouring tiles recompute a row's r from the
+// h that its own tile replaces.
+enum { TILED_RELAX = 0, TILED_SNAP = 1, TILED_REVERSE = 2 };
+
+template <class T, class V> struct TiledSnapArgs : TiledArgs<T, V> {
+  T* snap;          // visit-major, R values a visit: x (SNAP) or r (REVERSE)
+  T* h0;            // REVERSE: h by schedule position, in the buffers' order
+  T* h1;
+  int R, first;     // the wave's slice s is at visit first + s
+};
+
 // The slices of one wave: tiles [start[s], end[s]) of slice z0 + 2s; bit s of
 // flip selects buffer 1 as the slice's read buffer.
 struct WaveTiles {
@@ -1698,25 +1721,27 @@ __device__ __forceinline__ void tiled_place(int2 en, int gh, TiledRow<T, V>& w) 
 
 // Row w.j's record and right-hand side.
 template <class T, class V>
-__device__ __forceinline__ void tiled_load(const TiledArgs<T, V>& a, TiledRow<T, V>& w) {
+__device__ __forceinline__ void tiled_load(const TiledArgs<T, V>& a, const T* b, TiledRow<T, V>& w) {
   RowRecordWords<T, V> u;
   const record_word* src = (const record_word*)(a.records + (unsigned)w.j);
 #pragma unroll
   for (int i = 0; i < (int)(sizeof(u.q) / sizeof(record_word)); ++i) u.q[i] = src[i];
   w.op = u.r;
-  w.b = a.b[(unsigned)w.j];
+  w.b = b[(unsigned)w.j];
 }
 
 // The update of a row of colour C (x parity C & 1, y parity C >> 1):
 // neighbour (dx, dy, dz) sits in layer dz + 1, plane of parities
 // ((C & 1) + dx, (C >> 1) + dy), at base + ((px + dx) >> 1) * gh + ((py + dy) >> 1).
-template <int C, class T, class V>
-__device__ __forceinline__ void tiled_update(T* grid, int gh, T* Q, const TiledRow<T, V>& w) {
+// REVERSE leaves the row's own entry (slot 13) out of the sum and keeps h.
+template <int C, int MODE, class T, class V>
+__device__ __forceinline__ void tiled_update(T* grid, int gh, T* Q, T* H, T* snap, const TiledRow<T, V>& w) {
   constexpr int px = C & 1, py = C >> 1;
   const int pl = gh * gh, layer = 4 * pl;
   T r = w.b;
 #pragma unroll
   for (int k = 0; k < 27; ++k) {
+    if (MODE == TILED_REVERSE && k == 13) continue;
     const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
     const int qx = px + dx + 2, qy = py + dy + 2;  // shifted to stay nonnegative
     const int plane = ((qy & 1) << 1) | (qx & 1);
@@ -1724,10 +1749,19 @@ __device__ __forceinline__ void tiled_update(T* grid, int gh, T* Q, const TiledR
     r = r - grid[off + w.base] * T(w.op.v[k]);
   }
   const int self = layer + (py * 2 + px) * pl + w.base;
-  const T xi = grid[self];
-  const T nv = w.op.has ? xi + r * w.op.inv : xi;
+  T nv;
+  if constexpr (MODE == TILED_REVERSE) {
+    nv = w.op.has ? r * w.op.inv : T(0);
+    if (w.interior) H[w.j] = r - nv * T(w.op.v[13]);
+  } else {
+    const T xi = grid[self];
+    nv = w.op.has ? xi + r * w.op.inv : xi;
+  }
   grid[self] = nv;
-  if (w.interior) Q[w.j] = nv;
+  if (w.interior) {
+    Q[w.j] = nv;
+    if constexpr (MODE != TILED_RELAX) snap[w.j] = nv;
+  }
 }
 
 // BS threads per tile: thread i computes the tile's i-th row (rows of colour
@@ -1737,24 +1771,38 @@ __device__ __forceinline__ void tiled_update(T* grid, int gh, T* Q, const TiledR
 // BS computed rows take further passes for the rest.
 constexpr int TILED_STAGE_UNROLL = 4;
 
-template <class T, class V>
-__device__ __forceinline__ void tiled_phase(int phase, T* grid, int gh, T* Q, const TiledRow<T, V>& w) {
+template <int MODE, class T, class V>
+__device__ __forceinline__ void tiled_phase(int phase, T* grid, int gh, T* Q, T* H, T* snap, const TiledRow<T, V>& w) {
+  constexpr int F = MODE == TILED_REVERSE ? 3 : 0;  // category c holds colour c, or 3 - c
   switch (phase) {
-    case 0: tiled_update<0>(grid, gh, Q, w); break;
-    case 1: tiled_update<1>(grid, gh, Q, w); break;
-    case 2: tiled_update<2>(grid, gh, Q, w); break;
-    default: tiled_update<3>(grid, gh, Q, w); break;
+    case 0: tiled_update<0 ^ F, MODE>(grid, gh, Q, H, snap, w); break;
+    case 1: tiled_update<1 ^ F, MODE>(grid, gh, Q, H, snap, w); break;
+    case 2: tiled_update<2 ^ F, MODE>(grid, gh, Q, H, snap, w); break;
+    default: tiled_update<3 ^ F, MODE>(grid, gh, Q, H, snap, w); break;
   }
 }
 
 // One tile of slice s of a wave: the bx-th tile of the slice's range.
-template <class T, class V, int BS>
-__device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveTiles& wv, int bx, int s, T* grid) {
+template <class T, class V, int BS, int MODE = TILED_RELAX>
+__device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveTiles& wv, int bx, int s, T* grid,
+                                           const TiledSnapArgs<T, V>* m = nullptr) {
   const int tile = wv.start[s] + bx;
   if (tile >= wv.end[s]) return;
   const bool flip = (wv.flip >> s) & 1u;
   const T* P = flip ? a.x1 : a.x0;
   T* Q = flip ? a.x0 : a.x1;
+  // a row's constant term: b, or (reverse) h from the read buffer
+  const T* B = a.b;
+  T* H = nullptr;
+  T* snap = nullptr;
+  if constexpr (MODE != TILED_RELAX) snap = m->snap + (size_t)(m->first + s) * (size_t)m->R;
+  if constexpr (MODE == TILED_REVERSE) {
+    B = flip ? m->h1 : m->h0;
+    H = flip ? m->h0 : m->h1;
+  }
+  // the layer of the slice that this wave's visit count has reached: z + 1
+  // (layer 2), or z - 1 (layer 0) when the slices run the other way
+  constexpr int AHEAD = MODE == TILED_REVERSE ? 0 : 2;
   const int4 d0 = *(const int4*)(a.desc + TILE_DESC_INTS * tile);
   const int4 d1 = *(const int4*)(a.desc + TILE_DESC_INTS * tile + 4);
   const int4 d2 = *(const int4*)(a.desc + TILE_DESC_INTS * tile + 8);
@@ -1762,7 +1810,7 @@ __device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveT
   if (c0 == stage0) return;  // no interior rows: staged data for the neighbouring slices only
   const int tid = (int)threadIdx.x, gh = a.g >> 1, layer = 4 * gh * gh;
   // staged values: this slice [d1.x, d1.y) (layer 1), slice z + 1 [d1.z, d1.w)
-  // (layer 2, read buffer of the write side) and slice z - 1 [d2.x, d2.y)
+  // (layer 2, from the write side's buffer unless reversed) and slice z - 1 [d2.x, d2.y)
   // (layer 0), as one index range
   const int n_own = d1.y - d1.x, n_up = d1.w - d1.z, n_all = n_own + n_up + (d2.y - d2.x);
   const int e = c0 + tid;
@@ -1790,7 +1838,7 @@ __device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveT
   };
   auto stage_values = [&]() {
 #pragma unroll
-    for (int u = 0; u < TILED_STAGE_UNROLL; ++u) sval[u] = (slay[u] == 2 ? (const T*)Q : P)[(unsigned)sen[u].x];
+    for (int u = 0; u < TILED_STAGE_UNROLL; ++u) sval[u] = (slay[u] == AHEAD ? (const T*)Q : P)[(unsigned)sen[u].x];
   };
   auto stage_store = [&]() {
 #pragma unroll
@@ -1804,7 +1852,7 @@ __device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveT
   const int2 en2 = a.entries[e + BS < stage0 ? e + BS : c0];
   stage_values();
   tiled_place(en, gh, w);
-  tiled_load(a, w);
+  tiled_load(a, B, w);
   for (int i = tid; i < 3 * layer; i += BS) grid[i] = T(0);
   __syncthreads();  // grid cleared
   stage_store();
@@ -1819,12 +1867,12 @@ __device__ __forceinline__ void relax_tile(const TiledArgs<T, V>& a, const WaveT
   // registers once it is done.
   const int cstart[5] = {c0, c1, c2, c3, stage0};
   for (int phase = 0; phase < 4; ++phase) {
-    if (have && colour == phase) tiled_phase(phase, grid, gh, Q, w);
+    if (have && colour == phase) tiled_phase<MODE>(phase, grid, gh, Q, H, snap, w);
     for (int e2 = e + BS; e2 < stage0; e2 += BS) {
       if (e2 < cstart[phase] || e2 >= cstart[phase + 1]) continue;
       tiled_place(e2 == e + BS ? en2 : a.entries[e2], gh, w);
-      tiled_load(a, w);
-      tiled_phase(phase, grid, gh, Q, w);
+      tiled_load(a, B, w);
+      tiled_phase<MODE>(phase, grid, gh, Q, H, snap, w);
     }
     __syncthreads();
   }
@@ -1834,6 +1882,12 @@ template <class T, class V, int BS>
 __global__ void __launch_bounds__(BS) k_relax_tiled(TiledArgs<T, V> a, WaveTiles wv) {
   extern __shared__ unsigned char lds_raw[];
   relax_tile<T, V, BS>(a, wv, (int)blockIdx.x, (int)blockIdx.y, (T*)lds_raw);
+}
+
+template <class T, class V, int BS, int MODE>
+__global__ void __launch_bounds__(BS) k_tiled_snap(TiledSnapArgs<T, V> a, WaveTiles wv) {
+  extern __shared__ unsigned char lds_raw[];
+  relax_tile<T, V, BS, MODE>(a, wv, (int)blockIdx.x, (int)blockIdx.y, (T*)lds_raw, &a);
 }
 
 // Several reconstructions' tiles of the same wave in one launch: members'
@@ -2125,9 +2179,9 @@ static int relax_tile_size(int requested, int depth) {
 
 // With the level's dense z-major index (level_dense, side dim) the entries
 // come tile by tile from the index (k_tile_scan_*); without it, row by row
-// and a sort of the (tile, category) keys.
+// and a sort of the (tile, category) keys.  flip: see k_tile_members.
 static void build_tile_table(const int64_t* keys, const int* order, int R, int depth, int ts, const int* level_dense,
-                             int dim, TileTable& tt, hipStream_t s) {
+                             int dim, TileTable& tt, hipStream_t s, int flip = 0) {
   const int n = 1 << depth;
   tt.ts = ts;
   tt.nt = (n + 1 + ts - 1) / ts;
@@ -2136,7 +2190,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
   if (ndense + 1 > INT32_MAX) throw PsrError(1, "tiled relaxation: too many tiles");
   DArray<int> flags(ndense + 1, s), compact(ndense + 1, s), total(1, s);
   flags.zero();
-  hipLaunchKernelGGL(k_tile_members<0>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flags.data(),
+  hipLaunchKernelGGL(k_tile_members<0>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flip, flags.data(),
                      (const int*)nullptr, (int*)nullptr, (uint32_t*)nullptr, (int*)nullptr);
   KERNEL_CHECK();
   scan_exclusive_i32(flags.data(), compact.data(), ndense + 1, total.data(), s);
@@ -2153,7 +2207,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
     HIP_CHECK(hipMemsetAsync(offs.data() + 5 * (size_t)tiles, 0, sizeof(int), s));
     if (tiles) {
       hipLaunchKernelGGL(k_tile_scan_count, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, level_dense, dim, n,
-                         (const int*)dense_of.data(), tt.nt, ts, offs.data());
+                         (const int*)dense_of.data(), tt.nt, ts, flip, offs.data());
       KERNEL_CHECK();
     }
     scan_exclusive_i32(offs.data(), offs.data(), 5 * (int64_t)tiles + 1, etotal.data(), s);
@@ -2165,7 +2219,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
     tt.desc.reset(TILE_DESC_INTS * (size_t)std::max(tiles, 1), s);
     if (tiles) {
       hipLaunchKernelGGL(k_tile_scan_emit, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, level_dense, dim, n,
-                         (const int*)dense_of.data(), tt.nt, ts, (const int*)inv.data(), (const int*)offs.data(),
+                         (const int*)dense_of.data(), tt.nt, ts, flip, (const int*)inv.data(), (const int*)offs.data(),
                          tt.entries.data());
       KERNEL_CHECK();
       hipLaunchKernelGGL(k_tile_desc_offs, dim3(blocks_for(tiles, 256)), dim3(256), 0, s, (const int*)offs.data(), tiles,
@@ -2186,7 +2240,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
     return;
   }
   DArray<int> count(R + 1, s), pos(R + 1, s), etotal(1, s);
-  hipLaunchKernelGGL(k_tile_members<1>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flags.data(),
+  hipLaunchKernelGGL(k_tile_members<1>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flip, flags.data(),
                      (const int*)compact.data(), count.data(), (uint32_t*)nullptr, (int*)nullptr);
   KERNEL_CHECK();
   HIP_CHECK(hipMemsetAsync(count.data() + R, 0, sizeof(int), s));
@@ -2200,7 +2254,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
   tt.entries_count = E;
   DArray<uint32_t> skeys(std::max(E, 1), s);
   DArray<int> svals(std::max(E, 1), s);
-  hipLaunchKernelGGL(k_tile_members<2>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flags.data(),
+  hipLaunchKernelGGL(k_tile_members<2>, dim3(blocks_for(R, 256)), dim3(256), 0, s, order, keys, R, ts, tt.nt, flip, flags.data(),
                      (const int*)compact.data(), pos.data(), skeys.data(), svals.data());
   KERNEL_CHECK();
   sort_pairs_u32(skeys.data(), svals.data(), E, bits_for((uint64_t)tt.tiles * 8), s);
@@ -3943,6 +3997,91 @@ __global__ void __launch_bounds__(256) k_gs_reverse(const int* __restrict__ orde
   }
 }
 
+// Row records of a finished level from its schedule-ordered operator (the
+// relaxation's own, or the transposed one of the reverse sweeps: row i's slot
+// k holds A_ci of its neighbour c, which is c's slot 26 - k, because the
+// stencils of one level are symmetric in structure).  Absent slots hold +0.
+template <class T, class S, class V>
+__global__ void __launch_bounds__(256) k_row_records(const int* __restrict__ order, const int* __restrict__ inv, int transposed,
+                                                     int R, const int* __restrict__ cols, const V* __restrict__ vals,
+                                                     RowRecord<T, V>* __restrict__ records) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= R) return;
+  int at[27];
+#pragma unroll
+  for (int k = 0; k < 27; ++k) at[k] = cols[(int64_t)k * R + j];
+  if (transposed) {
+#pragma unroll
+    for (int k = 0; k < 27; ++k) at[k] = at[k] >= 0 ? inv[at[k]] : -1;
+  }
+  RowRecordWords<T, V> rec;
+#pragma unroll
+  for (int k = 0; k < 27; ++k)
+    rec.r.v[k] = at[k] < 0 ? V(0) : transposed ? vals[(int64_t)(26 - k) * R + at[k]] : vals[(int64_t)k * R + j];
+  const S diagonal = S(rec.r.v[13]);  // slot 13 is the row itself
+  rec.r.has = diagonal != S(0);
+  rec.r.inv = T(diagonal != S(0) ? S(1) / diagonal : S(0));
+  record_word* dst = (record_word*)(records + j);
+#pragma unroll
+  for (int q = 0; q < (int)(sizeof(rec.q) / sizeof(record_word)); ++q) dst[q] = rec.q[q];
+}
+
+// After the reverse sweeps, at schedule position j: the right-hand side's
+// gradient sum over visits of r (last visit first, as it was reversed) at the
+// canonical row, and with gvals the operator's, -sum over visits r x_seen per
+// slot.  Row i at visit t saw x_c of visit t for neighbours updated earlier
+// in the visit (the slice above, or an earlier colour of its own slice), of
+// visit t - 1 otherwise; the diagonal entry also carries -r (x_new - x_old)
+// through 1/A_ii, so it saw visit t.  rsnap's visit v is visit iters - 1 - v.
+// One pass over the snapshots after the chain of waves: the sums are not part
+// of any wave's dependency chain.
+constexpr int VISIT_CHUNK = 8;
+
+template <class T>
+__global__ void __launch_bounds__(256) k_sliced_grads(const int* __restrict__ order, const int* __restrict__ inv,
+                                                      const int64_t* __restrict__ keys, const int* __restrict__ cols, int R,
+                                                      int iters, const double* __restrict__ rsnap, const T* __restrict__ xsnap,
+                                                      double* __restrict__ grhs, double* __restrict__ gvals) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= R) return;
+  const int i = order[j];
+  const int64_t key = keys[i];
+  const int px = key_x(key) & 1, py = key_y(key) & 1;
+  double sum = 0.0;
+  for (int v0 = 0; v0 < iters; v0 += VISIT_CHUNK) {
+    double r[VISIT_CHUNK];  // visits iters - 1 - v0, ... downwards
+#pragma unroll
+    for (int u = 0; u < VISIT_CHUNK; ++u) r[u] = v0 + u < iters ? rsnap[(int64_t)(v0 + u) * R + j] : 0.0;
+#pragma unroll
+    for (int u = 0; u < VISIT_CHUNK; ++u) sum += r[u];
+    if (!gvals) continue;
+    for (int k = 0; k < 27; ++k) {
+      const int c = cols[(int64_t)k * R + j];
+      double g = 0.0;
+      if (c >= 0) {
+        const int cj = inv[c];
+        const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
+        const bool earlier = dz > 0 || (dz == 0 && ((px + dx) & 1) + 2 * ((py + dy) & 1) < px + 2 * py) || k == 13;
+        T x[VISIT_CHUNK];
+#pragma unroll
+        for (int u = 0; u < VISIT_CHUNK; ++u) {
+          const int t = iters - 1 - v0 - u - (earlier ? 0 : 1);
+          x[u] = t >= 0 ? xsnap[(int64_t)t * R + cj] : T(0);
+        }
+#pragma unroll
+        for (int u = 0; u < VISIT_CHUNK; ++u) g -= r[u] * double(x[u]);
+      }
+      gvals[(int64_t)k * R + j] = v0 ? gvals[(int64_t)k * R + j] + g : g;
+    }
+  }
+  grhs[i] = sum;
+}
+
+__global__ void k_gather_d(const int* __restrict__ order, int R, const double* __restrict__ g, double* __restrict__ out) {
+  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+  if (j < R) out[j] = g[order[j]];
+}
+
 // ---- matrix-value gradients (relaxation_adjoint.py:29-73, multigrid_adjoint.py,
 // assembly_adjoint.py:44-91): the reverse sweeps need the x each row saw, so
 // the forward relaxations are replayed once with x snapshots.
@@ -4414,13 +4553,120 @@ void stencil_scatter(const int* order, const Stencil<V>& m, int slots, const dou
   KERNEL_CHECK();
 }
 
-// One finer level backwards: gx (w.r.t. its correction, consumed) gives the
-// right-hand-side gradient grhs and adds to gcum_prev (w.r.t. the cumulative
-// solution of the level below).
+// One wave after another of a tiled sweep sequence with snapshots (SNAP,
+// REVERSE), as tiled_prepare's graph runs RELAX; `buffers` is the state of
+// iters % 2's read buffers on entry.  REVERSE counts slices from the other
+// end: its slice z is the level's slice 2^depth - z.
+template <class T, class V, int BS, int MODE>
+static void tiled_waves(const TileTable& tt, TiledSnapArgs<T, V> a, int depth, int iters, hipStream_t s) {
+  const int n = 1 << depth;
+  const size_t lds = sizeof(T) * 3 * (size_t)a.g * a.g;
+  for (int q = 0; q <= n + 2 * (iters - 1); ++q) {
+    const int first = std::max(0, floordiv(q - n + 1, 2));
+    const int last = std::min(iters - 1, q / 2);
+    if (last < first) continue;
+    const int slices = last - first + 1;
+    WaveTiles wv;
+    wv.flip = 0;
+    int most = 0;
+    for (int k = 0; k < RELAX_MAX_SLICES; ++k) wv.start[k] = wv.end[k] = 0;
+    for (int k = 0; k < slices; ++k) {
+      const int zw = n - q + 2 * first + 2 * k, z = MODE == TILED_REVERSE ? n - zw : zw;
+      wv.start[k] = tt.slice_start[z];
+      wv.end[k] = tt.slice_start[z + 1];
+      most = std::max(most, wv.end[k] - wv.start[k]);
+      if ((iters - (first + k)) % 2) wv.flip |= 1u << k;
+    }
+    if (!most) continue;
+    a.first = first;
+    hipLaunchKernelGGL((k_tiled_snap<T, V, BS, MODE>), dim3((unsigned)most, (unsigned)slices), dim3(BS), lds, s, a, wv);
+  }
+  KERNEL_CHECK();
+}
+
+template <class T, class V, int MODE>
+static void tiled_sweeps(const TileTable& tt, const TiledSnapArgs<T, V>& a, int depth, int iters, hipStream_t s) {
+  if (iters > RELAX_MAX_SLICES) throw PsrError(1, "tiled relaxation supports at most 16 sweeps");
+  switch (tiled_width(tt)) {
+    case 64: return tiled_waves<T, V, 64, MODE>(tt, a, depth, iters, s);
+    case 128: return tiled_waves<T, V, 128, MODE>(tt, a, depth, iters, s);
+    default: return tiled_waves<T, V, 256, MODE>(tt, a, depth, iters, s);
+  }
+}
+
+// The sliced relaxation of one finer level backwards on tile tables: gx
+// (canonical) -> grhs and, with gA, the operator's gradient (the relaxation
+// is replayed from zero for the x each visit saw, relaxation_adjoint.py:29-46).
 template <class T, class V>
-void finer_backward(Result<T>& r, int d, const Stencil<V>& Aop, const Stencil<V>& Cop, DArray<double>& gx, DArray<double>& grhs,
-                    DArray<double>& gcum_prev, hipStream_t s, DArray<double>* gA = nullptr, DArray<double>* gC = nullptr,
-                    const T* cum_prev = nullptr) {
+void tiled_backward(Result<T>& r, int d, int ts, const Stencil<V>& Aop, const double* gx, double* grhs, double* gA, hipStream_t s) {
+  LevelState<T>& L = r.levels[d];
+  const int R = L.basis_count, iters = r.prm.iters;
+  const int* ord = L.order.data();
+  const int* cols = Aop.cols.data();
+  const V* vals = Aop.vals.data();
+  const unsigned blocks = blocks_for(R, 256);
+  DArray<int> dense, inv(R, s);
+  const int64_t dim = (1 << d) + 1;
+  const bool dense_ok = dim * dim * dim <= dense_index_max_cells();
+  if (dense_ok) {
+    dense.reset((size_t)(dim * dim * dim), s);
+    HIP_CHECK(hipMemsetAsync(dense.data(), 0xff, sizeof(int) * dense.size(), s));  // -1
+    hipLaunchKernelGGL(k_dense_fill, dim3(blocks), dim3(256), 0, s, (const int64_t*)L.basis_keys.data(), R, (int)dim, dense.data());
+    KERNEL_CHECK();
+  }
+  const int* level_dense = dense_ok ? (const int*)dense.data() : (const int*)nullptr;
+  hipLaunchKernelGGL(k_inverse_permutation, dim3(blocks), dim3(256), 0, s, ord, R, inv.data());
+  KERNEL_CHECK();
+  DArray<T> xsnap;
+  if (gA) {
+    TileTable tt;
+    build_tile_table(L.basis_keys.data(), ord, R, d, ts, level_dense, (int)dim, tt, s);
+    DArray<RowRecord<T, V>> records(R, s);
+    hipLaunchKernelGGL((k_row_records<T, T, V>), dim3(blocks), dim3(256), 0, s, ord, (const int*)inv.data(), 0, R, cols, vals,
+                       records.data());
+    KERNEL_CHECK();
+    DArray<T> x0(R, s), x1(R, s);
+    (iters % 2 ? x1 : x0).zero();
+    xsnap.reset((size_t)iters * R, s);
+    TiledSnapArgs<T, V> a;
+    static_cast<TiledArgs<T, V>&>(a) = TiledArgs<T, V>{tt.entries.data(), tt.desc.data(), records.data(), L.rhs.data(), x0.data(),
+                                                       x1.data(), ts + 8};
+    a.snap = xsnap.data();
+    a.h0 = a.h1 = nullptr;
+    a.R = R;
+    a.first = 0;
+    tiled_sweeps<T, V, TILED_SNAP>(tt, a, d, iters, s);
+  }
+  TileTable tt;
+  build_tile_table(L.basis_keys.data(), ord, R, d, ts, level_dense, (int)dim, tt, s, 3);
+  DArray<RowRecord<double, V>> records(R, s);
+  hipLaunchKernelGGL((k_row_records<double, T, V>), dim3(blocks), dim3(256), 0, s, ord, (const int*)inv.data(), 1, R, cols, vals,
+                     records.data());
+  KERNEL_CHECK();
+  DArray<double> r0(R, s), r1(R, s), h0(R, s), h1(R, s), rsnap((size_t)iters * R, s);
+  (iters % 2 ? r1 : r0).zero();
+  hipLaunchKernelGGL(k_gather_d, dim3(blocks), dim3(256), 0, s, ord, R, gx, (iters % 2 ? h1 : h0).data());
+  KERNEL_CHECK();
+  TiledSnapArgs<double, V> a;
+  static_cast<TiledArgs<double, V>&>(a) = TiledArgs<double, V>{tt.entries.data(), tt.desc.data(), records.data(),
+                                                               (const double*)nullptr, r0.data(), r1.data(), ts + 8};
+  a.snap = rsnap.data();
+  a.h0 = h0.data();
+  a.h1 = h1.data();
+  a.R = R;
+  a.first = 0;
+  tiled_sweeps<double, V, TILED_REVERSE>(tt, a, d, iters, s);
+  hipLaunchKernelGGL(k_sliced_grads<T>, dim3(blocks), dim3(256), 0, s, ord, (const int*)inv.data(),
+                     (const int64_t*)L.basis_keys.data(), cols, R, iters, (const double*)rsnap.data(), (const T*)xsnap.data(), grhs,
+                     gA);
+  KERNEL_CHECK();
+}
+
+// The same launch by launch and colour by colour, scattering with atomics:
+// runs of more than RELAX_MAX_SLICES sweeps, and the colour-per-launch form.
+template <class T, class V>
+void launched_backward(Result<T>& r, int d, const Stencil<V>& Aop, DArray<double>& gx, DArray<double>& grhs, DArray<double>* gA,
+                       hipStream_t s) {
   LevelState<T>& L = r.levels[d];
   const int R = L.basis_count;
   Schedule<T> sc = make_schedule<T>(L.basis_keys, R, d, true, s);
@@ -4467,6 +4713,25 @@ void finer_backward(Result<T>& r, int d, const Stencil<V>& Aop, const Stencil<V>
                            gx.data(), grhs.data(), gA->data());
       }
     KERNEL_CHECK();
+  }
+}
+
+// One finer level backwards: gx (w.r.t. its correction, consumed) gives the
+// right-hand-side gradient grhs and adds to gcum_prev (w.r.t. the cumulative
+// solution of the level below).
+template <class T, class V>
+void finer_backward(Result<T>& r, int d, const Stencil<V>& Aop, const Stencil<V>& Cop, DArray<double>& gx, DArray<double>& grhs,
+                    DArray<double>& gcum_prev, hipStream_t s, DArray<double>* gA = nullptr, DArray<double>* gC = nullptr,
+                    const T* cum_prev = nullptr) {
+  LevelState<T>& L = r.levels[d];
+  const int R = L.basis_count;
+  const int ts = relax_tile_size(r.prm.relax_tile, d);
+  if (ts && R && r.prm.iters <= RELAX_MAX_SLICES) {
+    grhs.reset(R, s);
+    if (gA) gA->reset(27 * (size_t)R, s);
+    tiled_backward<T, V>(r, d, ts, Aop, (const double*)gx.data(), grhs.data(), gA ? gA->data() : (double*)nullptr, s);
+  } else {
+    launched_backward<T, V>(r, d, Aop, gx, grhs, gA, s);
   }
   // b = rhs - cross * cumulative(d-1); the cross operator has canonical rows
   stencil_scatter<V>((const int*)nullptr, Cop, 27, (const double*)grhs.data(), -1.0, gcum_prev.data(), s);
