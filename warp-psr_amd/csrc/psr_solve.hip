@@ -4208,7 +4208,7 @@ __device__ __forceinline__ int neighbour_colour8(int g, int k) {
 // what was seen and the slots' sums, then the atomics and stores, each step's
 // loads issued together (a neighbour's colour follows from its slot, not from
 // its key).  22.6 us a launch slot by slot,
-// 4.9 us now (4,913 rows).
+// 9.0 us now (4,913 rows).
 template <class T>
 __global__ void __launch_bounds__(256) k_gs_reverse_colored_m(const int* __restrict__ order, const int* __restrict__ goff, int g,
                                                               int forward, const int* __restrict__ cols, const T* __restrict__ vals,
