@@ -6,6 +6,7 @@
 // serially" so sums keep the reference order.  Splat records are sorted as
 // (packed key, record id) pairs only; the reducing lane recomputes each
 // record's value from its id instead of storing and re-reading it.
+#include "psr_bitmap.h"
 #include "psr_splat.h"
 
 #include <cmath>
@@ -486,12 +487,418 @@ template <class T> T density_scale_host() {
   return total / T(1000);
 }
 
+// ------------------------------------------------------------ bitmap form
+// The aggregates' cells and the density nodes of every level as bitmaps
+// (psr_bitmap.h).  Parents are halved words, the nodes of a level its cells
+// dilated by one, and every sum is gathered by its receiver in the order the
+// sorts gave it: a parent adds its children by octant, a node the aggregates
+// around it in Morton order.  One host read sizes everything.  With a sort a
+// level (and one of 27 records an aggregate) the stage took 0.33 ms for 512
+// points at depth 4 and 1.95 ms for 800,000 at depth 9; 0.13 and 0.42 ms this
+// way.
+struct CellLattice {
+  uint32_t cells[BITMAP_MAX_LEVELS];  // first word of the aggregates' level
+  uint32_t nodes[BITMAP_MAX_LEVELS];  // first word of the density nodes' level
+};
+
+PSR_HD int cell_words(int d) { return d > 5 ? 1 << (d - 5) : 1; }  // words per (x, y) row of 2^d cells
+PSR_HD uint32_t cell_row(int d, int x, int y) { return (((uint32_t)x << d) | (uint32_t)y) * (uint32_t)cell_words(d); }
+
+// the leaf level's bits: the first key of each word gathers the word's run
+__global__ void k_cells_mark(const int64_t* __restrict__ keys, int64_t n, int d, uint32_t* __restrict__ bits) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t key = keys[i];
+  if (i > 0 && (keys[i - 1] >> 5) == (key >> 5)) return;  // z is the key's lowest field
+  uint32_t word = 0;
+  for (int64_t j = i; j < n && (keys[j] >> 5) == (key >> 5); ++j) word |= 1u << (int)(keys[j] & 31);
+  bits[cell_row(d, key_x(key), key_y(key)) + (uint32_t)(key_z(key) >> 5)] = word;
+}
+
+// word t of level d from level d + 1 (density.py:59-72, _parents)
+__device__ __forceinline__ uint32_t halved_word(const uint32_t* fine, int d, uint32_t t) {
+  const int wz = cell_words(d), fz = cell_words(d + 1);
+  const int w = (int)(t % (uint32_t)wz), y = (int)((t / (uint32_t)wz) & ((1u << d) - 1u)), x = (int)((t / (uint32_t)wz) >> d);
+  uint32_t c1 = 0, c2 = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t* row = fine + cell_row(d + 1, 2 * x + (k >> 1), 2 * y + (k & 1));
+    c1 |= row[2 * w];
+    if (2 * w + 1 < fz) c2 |= row[2 * w + 1];
+  }
+  uint64_t v = ((uint64_t)c2 << 32) | c1;
+  return even_bits(v | (v >> 1));
+}
+
+__global__ void k_cells_halve(CellLattice lat, int d, uint32_t words, uint32_t* __restrict__ bits) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < words) bits[lat.cells[d] + t] = halved_word(bits + lat.cells[d + 1], d, t);
+}
+
+// levels top..0 (at most 1,024 words each) one after another in one workgroup
+constexpr int COARSE_CELL_LEVEL = 5;
+__global__ void __launch_bounds__(1024) k_cells_coarse(CellLattice lat, int top, uint32_t* bits) {
+  for (int d = top; d >= 0; --d) {
+    const uint32_t words = (1u << (2 * d)) * (uint32_t)cell_words(d);
+    for (uint32_t t = threadIdx.x; t < words; t += 1024) bits[lat.cells[d] + t] = halved_word(bits + lat.cells[d + 1], d, t);
+    __syncthreads();
+  }
+}
+
+// Where a launch over all levels' words or keys finds its level: sets 0..depth
+// are the aggregates' levels, the rest the density levels.
+template <class T> struct CellArrays {
+  int sets;
+  int block0[2 * BITMAP_MAX_LEVELS];
+  int depth[2 * BITMAP_MAX_LEVELS];
+  uint32_t base[2 * BITMAP_MAX_LEVELS];
+  int64_t* keys[2 * BITMAP_MAX_LEVELS];
+};
+
+template <class A> __device__ __forceinline__ int set_of_block(const A& a, int block) {
+  int d = 0;
+  for (int k = 1; k < a.sets; ++k) d = block >= a.block0[k] ? k : d;
+  return d;
+}
+
+// every density level's nodes: the cells within one of an aggregate's
+// (density.py:74-106 skips targets outside the grid)
+template <class T>
+__global__ void __launch_bounds__(BITMAP_THREADS) k_cells_dilate(CellLattice lat, CellArrays<T> arr, int first_set,
+                                                                 uint32_t* __restrict__ bits) {
+  const int block = (int)blockIdx.x + arr.block0[first_set];
+  const int set = set_of_block(arr, block), d = arr.depth[set], n = 1 << d, wz = cell_words(d);
+  const uint32_t words = (1u << (2 * d)) * (uint32_t)wz;
+  const uint32_t* cells = bits + lat.cells[d];
+  for (int k = 0; k < BITMAP_ITEMS; ++k) {
+    const uint32_t t = (uint32_t)(block - arr.block0[set]) * BITMAP_BLOCK + k * BITMAP_THREADS + threadIdx.x;
+    if (t >= words) return;
+    const int w = (int)(t % (uint32_t)wz), y = (int)((t / (uint32_t)wz) & (uint32_t)(n - 1)), x = (int)((t / (uint32_t)wz) >> d);
+    uint32_t own = 0, below = 0, above = 0;
+    for (int a = imax(x - 1, 0); a <= imin(x + 1, n - 1); ++a)
+      for (int b = imax(y - 1, 0); b <= imin(y + 1, n - 1); ++b) {
+        const uint32_t* row = cells + cell_row(d, a, b) + w;
+        own |= row[0];
+        if (w > 0) below |= row[-1];
+        if (w + 1 < wz) above |= row[1];
+      }
+    bits[arr.base[set] + t] = (own | (own << 1) | (own >> 1) | (below >> 31) | (above << 31)) & word_range(w, 0, n);
+  }
+}
+
+// ranks at the sets' first words and the end, for the host
+template <class T>
+__global__ void k_cells_starts(CellArrays<T> arr, const int* __restrict__ pre, uint32_t words, int* __restrict__ out) {
+  const int k = threadIdx.x;
+  if (k <= arr.sets) out[k] = pre[k < arr.sets ? arr.base[k] : words];
+}
+
+// all sets' sorted keys
+template <class T>
+__global__ void __launch_bounds__(BITMAP_THREADS) k_cells_keys(CellArrays<T> arr, const uint32_t* __restrict__ bits,
+                                                               const int* __restrict__ pre) {
+  const int set = set_of_block(arr, (int)blockIdx.x), d = arr.depth[set], wz = cell_words(d);
+  const uint32_t words = (1u << (2 * d)) * (uint32_t)wz, base = arr.base[set];
+  for (int k = 0; k < BITMAP_ITEMS; ++k) {
+    const uint32_t t = (uint32_t)((int)blockIdx.x - arr.block0[set]) * BITMAP_BLOCK + k * BITMAP_THREADS + threadIdx.x;
+    if (t >= words) return;
+    uint32_t b = bits[base + t];
+    if (!b) continue;
+    const int w = (int)(t % (uint32_t)wz), y = (int)((t / (uint32_t)wz) & ((1u << d) - 1u)), x = (int)((t / (uint32_t)wz) >> d);
+    int64_t* out = arr.keys[set] + (pre[base + t] - pre[base]);
+    for (; b; b &= b - 1) *out++ = basis_key(d, x, y, 32 * w + __builtin_ctz(b));
+  }
+}
+
+// density.py:228-240: parent g of level d adds its children in octant order
+// (x lowest)
+template <class T>
+__device__ __forceinline__ void parent_sum(int g, int d, const int64_t* keys, const uint32_t* fine_bits, const int* fine_pre,
+                                           const T* fine_vals, T* vals) {
+  const int64_t key = keys[g];
+  const int z = 2 * key_z(key), base = fine_pre[0];
+  uint32_t two[4];
+  int rank[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {  // row (2x + (k & 1), 2y + (k >> 1)): its cells z, z + 1 lie in one word
+    const uint32_t t = cell_row(d + 1, 2 * key_x(key) + (k & 1), 2 * key_y(key) + (k >> 1)) + (uint32_t)(z >> 5);
+    const uint32_t b = fine_bits[t];
+    two[k] = (b >> (z & 31)) & 3u;
+    rank[k] = fine_pre[t] - base + __popc(b & ((1u << (z & 31)) - 1u));
+  }
+  T v[4] = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    const int k = o & 3, up = o >> 2;
+    if (!((two[k] >> up) & 1u)) continue;
+    const T* c = fine_vals + 4 * (int64_t)(rank[k] + (up && (two[k] & 1u) ? 1 : 0));
+#pragma unroll
+    for (int a = 0; a < 4; ++a) v[a] = v[a] + c[a];
+  }
+#pragma unroll
+  for (int a = 0; a < 4; ++a) vals[4 * (int64_t)g + a] = v[a];
+}
+
+template <class T>
+__global__ void k_parent_sums(int count, int d, const int64_t* __restrict__ keys, const uint32_t* __restrict__ fine_bits,
+                              const int* __restrict__ fine_pre, const T* __restrict__ fine_vals, T* __restrict__ vals) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < count) parent_sum(g, d, keys, fine_bits, fine_pre, fine_vals, vals);
+}
+
+template <class T> struct ParentChain {
+  int count[COARSE_CELL_LEVEL + 2];
+  const int64_t* keys[COARSE_CELL_LEVEL + 2];
+  T* vals[COARSE_CELL_LEVEL + 2];
+};
+
+template <class T>
+__global__ void __launch_bounds__(1024) k_parent_sums_coarse(CellLattice lat, ParentChain<T> c, int top, const uint32_t* bits,
+                                                             const int* pre) {
+  for (int d = top; d >= 0; --d) {
+    for (int g = threadIdx.x; g < c.count[d]; g += 1024)
+      parent_sum(g, d, c.keys[d], bits + lat.cells[d + 1], pre + lat.cells[d + 1], (const T*)c.vals[d + 1], c.vals[d]);
+    __syncthreads();
+  }
+}
+
+// Presence of cells z - 1, z, z + 1 of a row (bits 0..2) and the rank of the
+// first of them, relative to the level: (rank << 3) | presence.
+__device__ __forceinline__ int row_of_three(const uint32_t* bits, const int* pre, uint32_t row, int z, int d) {
+  const int z0 = imax(z - 1, 0), w = z0 >> 5, sh = z0 & 31;
+  const uint32_t b = bits[row + (uint32_t)w];
+  const uint32_t next = w + 1 < cell_words(d) ? bits[row + (uint32_t)w + 1] : 0u;
+  const uint32_t win = (uint32_t)((((uint64_t)next << 32) | b) >> sh);
+  const int m = z > 0 ? (int)(win & 7u) : (int)((win & 3u) << 1);
+  return ((pre[row + (uint32_t)w] - pre[0] + __popc(b & ((1u << sh) - 1u))) << 3) | m;
+}
+
+template <class T> struct DensityArrays {
+  int sets;  // density levels 0..kd
+  int block0[BITMAP_MAX_LEVELS];
+  int count[BITMAP_MAX_LEVELS];
+  const int64_t* keys[BITMAP_MAX_LEVELS];
+  const T* cell_vals[BITMAP_MAX_LEVELS];
+  T* vals[BITMAP_MAX_LEVELS];
+};
+
+// density.py:74-106, gathered: node t of level d adds the splats of the
+// aggregates in the 27 cells around it, in the aggregates' Morton order (the
+// stable sort of the splat records by node kept that order).  Three
+// neighbouring coordinates t - 1, t, t + 1 have one boundary at a high bit H
+// (the carry into t for even t, into t + 1 for odd t) and one at bit 0, so
+// two of the cells differ first at the most significant high boundary between
+// them, 3 H + axis over the axes, and else at bit 0: the order is the high
+// sides with the axes by 3 H + axis, then the low bits z, y, x.
+template <class T>
+__global__ void __launch_bounds__(256) k_density_gather(CellLattice lat, DensityArrays<T> arr, const uint32_t* __restrict__ bits,
+                                                        const int* __restrict__ pre, T scale) {
+  __shared__ int rows[9][256];  // row_of_three of the nine (x, y) rows; each thread its own column
+  const int d = set_of_block(arr, (int)blockIdx.x), n = 1 << d;
+  const int g = ((int)blockIdx.x - arr.block0[d]) * 256 + (int)threadIdx.x;
+  if (g >= arr.count[d]) return;
+  const int64_t key = arr.keys[d][g];
+  const int t[3] = {key_x(key), key_y(key), key_z(key)};
+  const uint32_t* cell_bits = bits + lat.cells[d];
+  const int* cell_pre = pre + lat.cells[d];
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {
+    const int x = t[0] + r / 3 - 1, y = t[1] + r % 3 - 1;
+    rows[r][threadIdx.x] = x >= 0 && y >= 0 && x < n && y < n ? row_of_three(cell_bits, cell_pre, cell_row(d, x, y), t[2], d) : 0;
+  }
+  int sig[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) sig[a] = 3 * (t[a] == 0 ? 30 : __builtin_ctz((t[a] & 1) ? t[a] + 1 : t[a])) + a;
+  // place[a]: the axis's bit in `hi`, 2 for the most significant
+  int place[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) place[a] = (sig[a] > sig[(a + 1) % 3] ? 1 : 0) + (sig[a] > sig[(a + 2) % 3] ? 1 : 0);
+  const T h = T(1) / T(n);
+  const T* vals = arr.cell_vals[d];
+  T acc = T(0);
+  for (int hi = 0; hi < 8; ++hi)
+    for (int low = 0; low < 8; ++low) {
+      int off[3];
+      bool there = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const int side = (hi >> place[a]) & 1, l = (low >> a) & 1;
+        // even t: {t - 1 (low bit 1)} | {t, t + 1}; odd t: {t - 1, t} | {t + 1 (low bit 0)}
+        const bool odd = t[a] & 1;
+        off[a] = odd ? (side ? 1 : l - 1) : (side ? l : -1);
+        there = there && (odd ? !(side && l) : (side || l));
+      }
+      if (!there) continue;
+      const int row = rows[(off[0] + 1) * 3 + off[1] + 1][threadIdx.x];
+      if (!((row >> (off[2] + 1)) & 1)) continue;
+      const T* v = vals + 4 * (int64_t)((row >> 3) + __popc((unsigned)(row & 7) & ((1u << (off[2] + 1)) - 1u)));
+      const T w = v[3];
+      const int sx = t[0] + off[0], sy = t[1] + off[1], sz = t[2] + off[2];
+      const Quad bx = quadratic(double((v[0] / w - T(sx) * h) / h));
+      const Quad by = quadratic(double((v[1] / w - T(sy) * h) / h));
+      const Quad bz = quadratic(double((v[2] / w - T(sz) * h) / h));
+      const T weight = w * scale;
+      acc = acc + T(double(weight) * quad_at(bx, 1 - off[0]) * quad_at(by, 1 - off[1]) * quad_at(bz, 1 - off[2]));
+    }
+  arr.vals[d][g] = acc;
+}
+
+// density.py:108-150 (density_value at each aggregate centroid), level
+// blockIdx.y, by the node bitmaps
+template <class T>
+__global__ void __launch_bounds__(256) k_density_at(CellLattice lat, DensityArrays<T> arr, const uint32_t* __restrict__ bits,
+                                                    const int* __restrict__ pre, const T* __restrict__ sums,
+                                                    const T* __restrict__ weights, int G, T* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, d = blockIdx.y;
+  if (i >= G) return;
+  const T w = weights[i];
+  const T p0 = sums[3 * i] / w, p1 = sums[3 * i + 1] / w, p2 = sums[3 * i + 2] / w;
+  const int n = 1 << d;
+  const int cx = cell_index(p0, n), cy = cell_index(p1, n), cz = cell_index(p2, n);
+  const T h = T(1) / T(n);
+  const Quad bx = quadratic(double((p0 - T(cx) * h) / h));
+  const Quad by = quadratic(double((p1 - T(cy) * h) / h));
+  const Quad bz = quadratic(double((p2 - T(cz) * h) / h));
+  const uint32_t* node_bits = bits + lat.nodes[d];
+  const int* node_pre = pre + lat.nodes[d];
+  const T* lvals = arr.vals[d];
+  int row[9];
+#pragma unroll
+  for (int r = 0; r < 9; ++r) {  // a centroid rounded past the cube's end has cell n: its row of three ends at n - 1
+    const int x = cx + r / 3 - 1, y = cy + r % 3 - 1;
+    row[r] = x >= 0 && y >= 0 && x < n && y < n && cz <= n ? row_of_three(node_bits, node_pre, cell_row(d, x, y), cz, d) : 0;
+  }
+  T v[27];
+#pragma unroll
+  for (int k = 0; k < 27; ++k) {
+    const int m = row[k / 3], z = k % 3;
+    v[k] = (m >> z) & 1 ? lvals[(m >> 3) + __popc((unsigned)(m & 7) & ((1u << z) - 1u))] : T(0);
+  }
+  T value = T(0);
+#pragma unroll
+  for (int k = 0; k < 27; ++k)  // k = 9x + 3y + z
+    if ((row[k / 3] >> (k % 3)) & 1)
+      value = value + T(quad_at(bx, k / 9) * quad_at(by, k / 3 % 3) * quad_at(bz, k % 3) * double(v[k]));
+  out[(int64_t)i * arr.sets + d] = value;
+}
+
+template <class T> void density_from_bitmaps(Result<T>& r) {
+  hipStream_t s = r.s;
+  const int depth = r.prm.depth, kd = r.prm.kernel_depth, G = r.G;
+  r.density_scale = density_scale_host<T>();
+  r.densities.reset((size_t)G * (kd + 1), s);
+  // lattices: the aggregates' levels, then the density levels
+  CellLattice lat{};
+  CellArrays<T> arr{};
+  size_t words = 0;
+  auto level_words = [](int d) { return ((size_t)1 << (2 * d)) * (size_t)cell_words(d); };
+  auto add_set = [&](int d) {
+    arr.base[arr.sets] = (uint32_t)words;
+    arr.depth[arr.sets] = d;
+    arr.block0[arr.sets++] = (int)(words / BITMAP_BLOCK);
+    words += (level_words(d) + BITMAP_BLOCK - 1) / BITMAP_BLOCK * BITMAP_BLOCK;
+    return arr.base[arr.sets - 1];
+  };
+  for (int d = 0; d <= depth; ++d) lat.cells[d] = add_set(d);
+  for (int d = 0; d <= kd; ++d) lat.nodes[d] = add_set(d);
+  const int blocks = (int)(words / BITMAP_BLOCK), node_set = depth + 1;
+  DArray<uint32_t> bits(words, s);
+  bits.zero();
+  hipLaunchKernelGGL(k_cells_mark, dim3(blocks_for(G, 256)), dim3(256), 0, s, (const int64_t*)r.sample_keys.data(), (int64_t)G, depth,
+                     bits.data() + lat.cells[depth]);
+  KERNEL_CHECK();
+  const int coarse = std::min(depth - 1, COARSE_CELL_LEVEL);
+  for (int d = depth - 1; d > coarse; --d) {
+    hipLaunchKernelGGL(k_cells_halve, dim3(blocks_for(level_words(d), 256)), dim3(256), 0, s, lat, d, (uint32_t)level_words(d),
+                       bits.data());
+    KERNEL_CHECK();
+  }
+  hipLaunchKernelGGL(k_cells_coarse, dim3(1), dim3(1024), 0, s, lat, coarse, bits.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_cells_dilate<T>, dim3(blocks - arr.block0[node_set]), dim3(BITMAP_THREADS), 0, s, lat, arr, node_set, bits.data());
+  KERNEL_CHECK();
+  DArray<int> sums(blocks, s), pre(words + 1, s), starts(arr.sets + 1, s);
+  hipLaunchKernelGGL(k_bits_count, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), sums.data());
+  KERNEL_CHECK();
+  scan_exclusive_i32(sums.data(), sums.data(), blocks, nullptr, s);
+  hipLaunchKernelGGL(k_bits_ranks, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), (const int*)sums.data(),
+                     pre.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_cells_starts<T>, dim3(1), dim3(64), 0, s, arr, (const int*)pre.data(), (uint32_t)words, starts.data());
+  KERNEL_CHECK();
+  std::vector<int> first(arr.sets + 1);
+  read_bytes(first.data(), starts.data(), sizeof(int) * first.size(), s);
+  auto count_of = [&](int set) { return first[set + 1] - first[set]; };
+  DensityArrays<T> den{};
+  den.sets = kd + 1;
+  int den_blocks = 0;
+  for (int d = 0; d <= depth; ++d) {
+    r.levels[d].agg_keys.reset(count_of(d), s);
+    r.levels[d].agg_vals.reset(4 * (size_t)count_of(d), s);
+    arr.keys[d] = r.levels[d].agg_keys.data();
+  }
+  for (int d = 0; d <= kd; ++d) {
+    LevelState<T>& L = r.levels[d];
+    const int count = count_of(node_set + d);
+    L.dens_keys.reset(count, s);
+    L.dens_vals.reset(count, s);
+    arr.keys[node_set + d] = L.dens_keys.data();
+    den.block0[d] = den_blocks;
+    den_blocks += (int)blocks_for(count, 256);
+    den.count[d] = count;
+    den.keys[d] = L.dens_keys.data();
+    den.cell_vals[d] = L.agg_vals.data();
+    den.vals[d] = L.dens_vals.data();
+  }
+  hipLaunchKernelGGL(k_cells_keys<T>, dim3(blocks), dim3(BITMAP_THREADS), 0, s, arr, (const uint32_t*)bits.data(),
+                     (const int*)pre.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_leaf_values<T>, dim3(blocks_for(G, 256)), dim3(256), 0, s, (const T*)r.position_sums.data(),
+                     (const T*)r.weights.data(), G, r.levels[depth].agg_vals.data());
+  KERNEL_CHECK();
+  for (int d = depth - 1; d > coarse; --d) {
+    const int count = count_of(d);
+    hipLaunchKernelGGL(k_parent_sums<T>, dim3(blocks_for(count, 256)), dim3(256), 0, s, count, d,
+                       (const int64_t*)r.levels[d].agg_keys.data(), (const uint32_t*)(bits.data() + lat.cells[d + 1]),
+                       (const int*)(pre.data() + lat.cells[d + 1]), (const T*)r.levels[d + 1].agg_vals.data(),
+                       r.levels[d].agg_vals.data());
+    KERNEL_CHECK();
+  }
+  ParentChain<T> chain{};
+  for (int d = 0; d <= coarse + 1; ++d) {
+    chain.count[d] = count_of(d);
+    chain.keys[d] = r.levels[d].agg_keys.data();
+    chain.vals[d] = r.levels[d].agg_vals.data();
+  }
+  hipLaunchKernelGGL(k_parent_sums_coarse<T>, dim3(1), dim3(1024), 0, s, lat, chain, coarse, (const uint32_t*)bits.data(),
+                     (const int*)pre.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_density_gather<T>, dim3(den_blocks), dim3(256), 0, s, lat, den, (const uint32_t*)bits.data(),
+                     (const int*)pre.data(), r.density_scale);
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_density_at<T>, dim3(blocks_for(G, 256), kd + 1), dim3(256), 0, s, lat, den, (const uint32_t*)bits.data(),
+                     (const int*)pre.data(), (const T*)r.position_sums.data(), (const T*)r.weights.data(), G, r.densities.data());
+  KERNEL_CHECK();
+}
+
+template <class T> void density_from_sorts(Result<T>& r);
+
 template <class T> void stage_density(Result<T>& r) {
+  hipStream_t s = r.s;
+  r.levels.resize(r.prm.depth + 1);
+  if (bitmap_fits((int64_t)1 << r.prm.depth)) density_from_bitmaps(r);
+  else density_from_sorts(r);
+  r.dw.reset(2 * (size_t)r.G, s);
+  hipLaunchKernelGGL(k_depths<T>, dim3(blocks_for(r.G, 256)), dim3(256), 0, s, (const T*)r.densities.data(), r.G,
+                     r.prm.kernel_depth, T(r.prm.samples_per_node), r.dw.data());
+  KERNEL_CHECK();
+}
+
+// The same by sorts (levels beyond the bitmap limit).
+template <class T> void density_from_sorts(Result<T>& r) {
   hipStream_t s = r.s;
   const int depth = r.prm.depth, kd = r.prm.kernel_depth;
   const int G = r.G;
-  r.levels.resize(depth + 1);
-  for (auto& L : r.levels) (void)L;
   LevelState<T>& leaf = r.levels[depth];
   leaf.agg_keys.reset(G, s);
   HIP_CHECK(hipMemcpyAsync(leaf.agg_keys.data(), r.sample_keys.data(), G * sizeof(int64_t), hipMemcpyDeviceToDevice, s));
@@ -581,10 +988,6 @@ template <class T> void stage_density(Result<T>& r) {
                        (const T*)r.weights.data(), G, d, kd + 1, r.densities.data());
     KERNEL_CHECK();
   }
-  r.dw.reset(2 * (size_t)G, s);
-  hipLaunchKernelGGL(k_depths<T>, dim3(blocks_for(G, 256)), dim3(256), 0, s, (const T*)r.densities.data(), G, kd,
-                     T(r.prm.samples_per_node), r.dw.data());
-  KERNEL_CHECK();
 }
 
 // ------------------------------------------------------------------ normals

@@ -6,9 +6,9 @@
 // Children of the sorted unique broods are placed at their lexicographic rank
 // directly (no second sort).
 //
-// Up to depth 11 (tree_bitmaps) the sets are bitmaps instead, and nothing is
+// Up to depth 11 (bitmap_fits) the sets are bitmaps instead, and nothing is
 // sorted: see TreeLattice.
-#include "psr_result.h"
+#include "psr_bitmap.h"
 
 namespace psr {
 
@@ -154,35 +154,13 @@ DArray<int64_t> unique_packed(DArray<uint64_t>& cand, int64_t total, BroodPack b
 // The whole tree is two host reads and about 20 launches; with a unique sort
 // a level it was some 25 launches and a host read a level (2.45 ms at depth 9
 // for 800,000 points, 0.56 ms at depth 4 for 512; 0.37 and 0.10 ms now).
-constexpr int TREE_MAX_LEVELS = 16;
-constexpr int TREE_THREADS = 256;
-constexpr int TREE_ITEMS = 8;
-constexpr int TREE_BLOCK = TREE_THREADS * TREE_ITEMS;  // words (or keys) of one workgroup, and the levels' alignment
-
 struct TreeLattice {
-  int side[TREE_MAX_LEVELS + 1];        // cells per axis
-  int wz[TREE_MAX_LEVELS + 1];          // words per (x, y) row
-  uint32_t base[TREE_MAX_LEVELS + 1];   // first word of the level
+  int side[BITMAP_MAX_LEVELS + 1];        // cells per axis
+  int wz[BITMAP_MAX_LEVELS + 1];          // words per (x, y) row
+  uint32_t base[BITMAP_MAX_LEVELS + 1];   // first word of the level
 };
 
 PSR_HD int lattice_side(int d) { return (d > 1 ? 1 << (d - 1) : 1) + 4; }
-
-// bits lo..hi-1 (of the row) that fall in word w
-__device__ __forceinline__ uint32_t word_range(int w, int lo, int hi) {
-  const int a = imax(lo - 32 * w, 0), b = imin(hi - 32 * w, 32);
-  if (a >= b) return 0u;
-  return (b == 32 ? ~0u : (1u << b) - 1u) & ~((1u << a) - 1u);
-}
-
-// even bits of v gathered into the low half
-__device__ __forceinline__ uint32_t even_bits(uint64_t v) {
-  v &= 0x5555555555555555ull;
-  v = (v | (v >> 1)) & 0x3333333333333333ull;
-  v = (v | (v >> 2)) & 0x0f0f0f0f0f0f0f0full;
-  v = (v | (v >> 4)) & 0x00ff00ff00ff00ffull;
-  v = (v | (v >> 8)) & 0x0000ffff0000ffffull;
-  return (uint32_t)(v | (v >> 16));
-}
 
 // Halved cells of the finer lattice's rows [x0, x1] x [y0, y1]: bit k of the
 // result is set if one of those rows has a cell whose parent is row position
@@ -234,11 +212,11 @@ __global__ void k_tree_seeds(const int64_t* __restrict__ nkeys, const T* __restr
 // to [-2^d, 2^d).  requests: the finer lattice's bits, null for none.  With
 // moved (requests_up from request_src, on this level's lattice) also the next
 // level's requests where they move up (tree.py:176-180): their parents.
-__global__ void __launch_bounds__(TREE_THREADS) k_tree_level(TreeLattice lat, int d, int coarse, const uint32_t* __restrict__ finer,
+__global__ void __launch_bounds__(BITMAP_THREADS) k_tree_level(TreeLattice lat, int d, int coarse, const uint32_t* __restrict__ finer,
                                                              const uint32_t* __restrict__ requests, uint32_t* __restrict__ bits,
                                                              const uint32_t* __restrict__ request_src,
                                                              uint32_t* __restrict__ requests_up, uint32_t words) {
-  const uint32_t t = blockIdx.x * TREE_THREADS + threadIdx.x;
+  const uint32_t t = blockIdx.x * BITMAP_THREADS + threadIdx.x;
   if (t >= words) return;
   const int side = lat.side[d], wz = lat.wz[d], fside = lat.side[d + 1], fwz = lat.wz[d + 1];
   const int w = (int)(t % (uint32_t)wz), y = (int)((t / (uint32_t)wz) % (uint32_t)side), x = (int)(t / (uint32_t)(wz * side));
@@ -260,66 +238,14 @@ __global__ void __launch_bounds__(TREE_THREADS) k_tree_level(TreeLattice lat, in
                                  : 0u;
 }
 
-// Sum over the workgroup's 256 threads and each thread's exclusive prefix.
-__device__ __forceinline__ int block_prefix(int v, int* total) {
-  __shared__ int wave_sum[TREE_THREADS / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += u;
-  }
-  if (lane == 63) wave_sum[wave] = inc;
-  __syncthreads();
-  int before = 0, all = 0;
-#pragma unroll
-  for (int k = 0; k < TREE_THREADS / 64; ++k) {
-    if (k < wave) before += wave_sum[k];
-    all += wave_sum[k];
-  }
-  *total = all;
-  return before + inc - v;
-}
-
-__global__ void __launch_bounds__(TREE_THREADS) k_tree_count(const uint32_t* __restrict__ bits, int* __restrict__ sums) {
-  const uint4* src = (const uint4*)(bits + (size_t)blockIdx.x * TREE_BLOCK) + threadIdx.x * (TREE_ITEMS / 4);
-  int n = 0;
-#pragma unroll
-  for (int k = 0; k < TREE_ITEMS / 4; ++k) {
-    const uint4 v = src[k];
-    n += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);
-  }
-  int total;
-  block_prefix(n, &total);
-  if (threadIdx.x == 0) sums[blockIdx.x] = total;
-}
-
-// pre[t] = set bits before word t (all levels), from the blocks' offsets
-__global__ void __launch_bounds__(TREE_THREADS) k_tree_ranks(const uint32_t* __restrict__ bits, const int* __restrict__ offsets,
-                                                             int* __restrict__ pre) {
-  const size_t first = (size_t)blockIdx.x * TREE_BLOCK + threadIdx.x * TREE_ITEMS;
-  int c[TREE_ITEMS], n = 0;
-#pragma unroll
-  for (int k = 0; k < TREE_ITEMS; ++k) {
-    c[k] = n;
-    n += __popc(bits[first + k]);
-  }
-  int total;
-  const int p = block_prefix(n, &total) + offsets[blockIdx.x];
-#pragma unroll
-  for (int k = 0; k < TREE_ITEMS; ++k) pre[first + k] = p + c[k];
-  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == TREE_THREADS - 1) pre[first + TREE_ITEMS] = p + n;
-}
-
 // Per level: first workgroup, and the arrays.  Keys of one level fill whole
 // workgroups, as words do.
 struct TreeArrays {
   int levels;
-  int block0[TREE_MAX_LEVELS + 1];
-  int64_t count[TREE_MAX_LEVELS];
-  int64_t* tree[TREE_MAX_LEVELS];
-  int64_t* basis[TREE_MAX_LEVELS];
+  int block0[BITMAP_MAX_LEVELS + 1];
+  int64_t count[BITMAP_MAX_LEVELS];
+  int64_t* tree[BITMAP_MAX_LEVELS];
+  int64_t* basis[BITMAP_MAX_LEVELS];
 };
 
 // ranks at the levels' first words and the end, for the host
@@ -343,15 +269,15 @@ __device__ __forceinline__ int level_of_block(const TreeArrays& a, int block) {
 // With ranks at the starts of x planes and (x, y) rows, the children before
 // one are: all of smaller planes, then this plane's x half, its smaller rows,
 // the row's y half, the row's earlier broods, the z half.
-__global__ void __launch_bounds__(TREE_THREADS) k_tree_children(TreeLattice lat, TreeArrays arr, const uint32_t* __restrict__ bits,
+__global__ void __launch_bounds__(BITMAP_THREADS) k_tree_children(TreeLattice lat, TreeArrays arr, const uint32_t* __restrict__ bits,
                                                                 const int* __restrict__ pre) {
   const int d = level_of_block(arr, (int)blockIdx.x);
   const int side = lat.side[d], wz = lat.wz[d];
   const uint32_t base = lat.base[d], words = (uint32_t)(side * side) * (uint32_t)wz;
   int64_t* tree = arr.tree[d];
   const int level0 = pre[base];
-  for (int k = 0; k < TREE_ITEMS; ++k) {
-    const uint32_t t = (blockIdx.x - (uint32_t)arr.block0[d]) * TREE_BLOCK + k * TREE_THREADS + threadIdx.x;
+  for (int k = 0; k < BITMAP_ITEMS; ++k) {
+    const uint32_t t = (blockIdx.x - (uint32_t)arr.block0[d]) * BITMAP_BLOCK + k * BITMAP_THREADS + threadIdx.x;
     if (t >= words) return;
     uint32_t b = bits[base + t];
     if (!b) continue;
@@ -380,13 +306,13 @@ __device__ __forceinline__ bool in_basis(int64_t key, int d) {
   return imin(imin(x, y), z) >= 0 && imax(imax(x, y), z) <= lim;
 }
 
-__global__ void __launch_bounds__(TREE_THREADS) k_basis_sums(TreeArrays arr, int* __restrict__ sums) {
+__global__ void __launch_bounds__(BITMAP_THREADS) k_basis_sums(TreeArrays arr, int* __restrict__ sums) {
   const int d = level_of_block(arr, (int)blockIdx.x);
-  const int64_t first = (int64_t)((int)blockIdx.x - arr.block0[d]) * TREE_BLOCK + threadIdx.x;
+  const int64_t first = (int64_t)((int)blockIdx.x - arr.block0[d]) * BITMAP_BLOCK + threadIdx.x;
   int n = 0;
 #pragma unroll
-  for (int k = 0; k < TREE_ITEMS; ++k) {
-    const int64_t i = first + k * TREE_THREADS;
+  for (int k = 0; k < BITMAP_ITEMS; ++k) {
+    const int64_t i = first + k * BITMAP_THREADS;
     if (i < arr.count[d] && in_basis(arr.tree[d][i], d)) ++n;
   }
   int total;
@@ -394,13 +320,13 @@ __global__ void __launch_bounds__(TREE_THREADS) k_basis_sums(TreeArrays arr, int
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ void __launch_bounds__(TREE_THREADS) k_basis_keys(TreeArrays arr, const int* __restrict__ offsets) {
+__global__ void __launch_bounds__(BITMAP_THREADS) k_basis_keys(TreeArrays arr, const int* __restrict__ offsets) {
   const int d = level_of_block(arr, (int)blockIdx.x);
-  const int64_t first = (int64_t)((int)blockIdx.x - arr.block0[d]) * TREE_BLOCK + threadIdx.x * TREE_ITEMS;
-  int64_t key[TREE_ITEMS];
+  const int64_t first = (int64_t)((int)blockIdx.x - arr.block0[d]) * BITMAP_BLOCK + threadIdx.x * BITMAP_ITEMS;
+  int64_t key[BITMAP_ITEMS];
   int n = 0;
 #pragma unroll
-  for (int k = 0; k < TREE_ITEMS; ++k) {
+  for (int k = 0; k < BITMAP_ITEMS; ++k) {
     key[k] = first + k < arr.count[d] ? arr.tree[d][first + k] : KMAX;
     if (key[k] != KMAX && !in_basis(key[k], d)) key[k] = KMAX;
     if (key[k] != KMAX) ++n;
@@ -408,15 +334,8 @@ __global__ void __launch_bounds__(TREE_THREADS) k_basis_keys(TreeArrays arr, con
   int total;
   int64_t at = (int64_t)block_prefix(n, &total) + offsets[blockIdx.x] - offsets[arr.block0[d]];
 #pragma unroll
-  for (int k = 0; k < TREE_ITEMS; ++k)
+  for (int k = 0; k < BITMAP_ITEMS; ++k)
     if (key[k] != KMAX) arr.basis[d][at++] = basis_key(d, tkey_x(key[k]), tkey_y(key[k]), tkey_z(key[k]));
-}
-
-// Whether every level's lattice fits: bits take 1/32 of an int index's
-// memory, so eight times its cells are allowed (depth 11 by default).
-bool tree_bitmaps(int depth) {
-  const int64_t side = lattice_side(depth);
-  return side * side * side <= 8 * dense_index_max_cells();
 }
 
 template <class T> void tree_from_bitmaps(Result<T>& r) {
@@ -424,16 +343,16 @@ template <class T> void tree_from_bitmaps(Result<T>& r) {
   const int depth = r.prm.depth, full = r.prm.full_depth, base = r.prm.base_depth;
   TreeLattice lat{};
   size_t words = 0;
-  for (int d = 0; d <= depth + 1 && d <= TREE_MAX_LEVELS; ++d) {
+  for (int d = 0; d <= depth + 1 && d <= BITMAP_MAX_LEVELS; ++d) {
     lat.side[d] = lattice_side(d);
     lat.wz[d] = (lat.side[d] + 31) / 32;
     lat.base[d] = (uint32_t)words;
     if (d > depth) break;  // the level past the finest has a shape, no words
     const size_t level = (size_t)lat.side[d] * lat.side[d] * lat.wz[d];
-    words += (level + TREE_BLOCK - 1) / TREE_BLOCK * TREE_BLOCK;
+    words += (level + BITMAP_BLOCK - 1) / BITMAP_BLOCK * BITMAP_BLOCK;
   }
   auto level_words = [&](int d) { return (uint32_t)(lat.side[d] * lat.side[d]) * (uint32_t)lat.wz[d]; };
-  const int blocks = (int)(words / TREE_BLOCK);
+  const int blocks = (int)(words / BITMAP_BLOCK);
   DArray<uint32_t> bits(words, s), moved(base < depth ? words : 0, s);
   bits.zero();
   const int64_t records = r.normal_offsets[depth + 1];
@@ -454,16 +373,16 @@ template <class T> void tree_from_bitmaps(Result<T>& r) {
     const bool up = d >= 1 && d - 1 <= base && !moved.empty();  // level d - 1's requests live on this lattice
     const int coarse = d <= full ? (d == 0 ? 2 : (1 << (d - 1)) + 2) : 0;
     const uint32_t n = level_words(d);
-    hipLaunchKernelGGL(k_tree_level, dim3(blocks_for(n, TREE_THREADS)), dim3(TREE_THREADS), 0, s, lat, d, coarse, finer, requests_of(d),
+    hipLaunchKernelGGL(k_tree_level, dim3(blocks_for(n, BITMAP_THREADS)), dim3(BITMAP_THREADS), 0, s, lat, d, coarse, finer, requests_of(d),
                        bits.data() + lat.base[d], requests_of(d), up ? moved.data() + lat.base[d] : (uint32_t*)nullptr, n);
     KERNEL_CHECK();
   }
   // ranks, then one read of the levels' brood counts
   DArray<int> sums(blocks, s), pre(words + 1, s);
-  hipLaunchKernelGGL(k_tree_count, dim3(blocks), dim3(TREE_THREADS), 0, s, (const uint32_t*)bits.data(), sums.data());
+  hipLaunchKernelGGL(k_bits_count, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), sums.data());
   KERNEL_CHECK();
   scan_exclusive_i32(sums.data(), sums.data(), blocks, nullptr, s);
-  hipLaunchKernelGGL(k_tree_ranks, dim3(blocks), dim3(TREE_THREADS), 0, s, (const uint32_t*)bits.data(), (const int*)sums.data(),
+  hipLaunchKernelGGL(k_bits_ranks, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), (const int*)sums.data(),
                      pre.data());
   KERNEL_CHECK();
   TreeArrays arr{};
@@ -477,30 +396,30 @@ template <class T> void tree_from_bitmaps(Result<T>& r) {
   }
   for (int d = 0; d <= depth; ++d) {
     LevelState<T>& L = r.levels[d];
-    arr.block0[d] = (int)(lat.base[d] / TREE_BLOCK);
+    arr.block0[d] = (int)(lat.base[d] / BITMAP_BLOCK);
     arr.count[d] = 8 * (int64_t)(first[d + 1] - first[d]);
     L.tree_keys.reset((size_t)arr.count[d], s);
     L.basis_keys.reset((size_t)arr.count[d], s);
     arr.tree[d] = L.tree_keys.data();
     arr.basis[d] = L.basis_keys.data();
   }
-  hipLaunchKernelGGL(k_tree_children, dim3(blocks), dim3(TREE_THREADS), 0, s, lat, arr, (const uint32_t*)bits.data(),
+  hipLaunchKernelGGL(k_tree_children, dim3(blocks), dim3(BITMAP_THREADS), 0, s, lat, arr, (const uint32_t*)bits.data(),
                      (const int*)pre.data());
   KERNEL_CHECK();
   // basis keys: the same order, filtered
   int key_blocks = 0;
   for (int d = 0; d <= depth; ++d) {
     arr.block0[d] = key_blocks;
-    key_blocks += (int)((arr.count[d] + TREE_BLOCK - 1) / TREE_BLOCK);
+    key_blocks += (int)((arr.count[d] + BITMAP_BLOCK - 1) / BITMAP_BLOCK);
   }
   arr.block0[depth + 1] = key_blocks;
   std::vector<int> ends(depth + 2, 0);
   if (key_blocks) {
     DArray<int> basis_sums(key_blocks + 1, s), starts(depth + 2, s);
-    hipLaunchKernelGGL(k_basis_sums, dim3(key_blocks), dim3(TREE_THREADS), 0, s, arr, basis_sums.data());
+    hipLaunchKernelGGL(k_basis_sums, dim3(key_blocks), dim3(BITMAP_THREADS), 0, s, arr, basis_sums.data());
     KERNEL_CHECK();
     scan_exclusive_i32(basis_sums.data(), basis_sums.data(), key_blocks, basis_sums.data() + key_blocks, s);
-    hipLaunchKernelGGL(k_basis_keys, dim3(key_blocks), dim3(TREE_THREADS), 0, s, arr, (const int*)basis_sums.data());
+    hipLaunchKernelGGL(k_basis_keys, dim3(key_blocks), dim3(BITMAP_THREADS), 0, s, arr, (const int*)basis_sums.data());
     KERNEL_CHECK();
     hipLaunchKernelGGL(k_basis_starts, dim3(1), dim3(64), 0, s, arr, (const int*)basis_sums.data(), starts.data());
     KERNEL_CHECK();
@@ -518,7 +437,7 @@ template <class T> void stage_tree(Result<T>& r) {
   hipStream_t s = r.s;
   const int depth = r.prm.depth, full = r.prm.full_depth, base = r.prm.base_depth;
   r.levels.resize(depth + 1);
-  if (tree_bitmaps(depth)) return tree_from_bitmaps(r);
+  if (bitmap_fits(lattice_side(depth))) return tree_from_bitmaps(r);
   DArray<int64_t> broods, requests;
   bool have_requests = false;
   // per-level basis counts stay on the device until the loop ends (one read):
