@@ -44,27 +44,34 @@ __global__ void k_cumulative(FieldIndex f, int d, const T* __restrict__ coef, T*
 template <class T> PSR_HD int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
 // Node words of levels 0..word_depth from the concatenated sorted keys: the
-// first key of each word (a key whose predecessor lies in another word)
-// collects the word's following keys, at most 32, so no two threads write one
-// word.  Words without keys keep the cleared value (no bits).
+// first key of each word (a key whose predecessor lies in another column or
+// below the word's first node) collects the word's keys, at most 32, so no two
+// threads write one word.  A shared node can be the first key of both its
+// words.  Words without keys keep the cleared value (no bits).
 __global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int word_depth, NodeWord* __restrict__ words) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int64_t key = keys[i];
   const int d = key_d(key);
   if (d > word_depth) return;
-  if (i > 0 && (keys[i - 1] >> 5) == (key >> 5)) return;  // z is the key's lowest field
-  uint32_t bits = 0;
-  for (int64_t j = i; j < n && (keys[j] >> 5) == (key >> 5); ++j) bits |= 1u << (int)(keys[j] & 31);
-  const int dim = (1 << d) + 1;
-  words[word_base(d) + (uint32_t)(key_x(key) * dim + key_y(key)) * (uint32_t)word_columns(d) + (uint32_t)(key_z(key) >> 5)] =
-      NodeWord{bits, (int32_t)i};
+  const int z = key_z(key), wc = word_columns(d), own = word_of(z);
+  const int64_t column = key >> 16;
+  const int before = i > 0 && (keys[i - 1] >> 16) == column ? key_z(keys[i - 1]) : -1;  // z of the column's key below
+  for (int w = z == 31 * own && own > 0 ? own - 1 : own; w <= own && w < wc; ++w) {
+    if (before >= 31 * w) continue;
+    uint32_t bits = 0;
+    for (int64_t j = i; j < n && (keys[j] >> 16) == column && key_z(keys[j]) <= 31 * w + 31; ++j) bits |= 1u << (key_z(keys[j]) - 31 * w);
+    words[word_at(d, key_x(key), key_y(key), w)] = NodeWord{bits, (int32_t)i};
+  }
 }
 
-// One level's eight trilinear corners of a cube point: cell, weights and
-// coefficient indices (-1 absent or left of the point's floor).
+// One level's eight trilinear corners of a cube point: weights and, for each
+// of the four z pairs, the index of the first node present (0 if none) and
+// which of the two count (bit 0 the lower, bit 1 the upper): present and not
+// left of the point's floor.  Present pairs are neighbours in memory.
 template <class T> struct Corners {
-  int idx[8];
+  int first[4];
+  unsigned present[4], counts[4];
   T fr[3];
   bool up[3];  // cell + 1 > floor: the upper corner has weight fr, else 1 - fr
 };
@@ -83,36 +90,49 @@ __device__ __forceinline__ void find_corners(const FieldIndex& f, const T* p, in
     c.up[a] = cell[a] + 1 > base[a];
   }
   if constexpr (WORDS) {
-    const int wc = word_columns(d);
-    const NodeWord* at = f.words + word_base(d) + (uint32_t)(cell[0] * (n + 1) + cell[1]) * (uint32_t)wc + (uint32_t)(cell[2] >> 5);
-    // the upper node's word: the same one, except at a word's end (then the
-    // next word of the column, which exists because cell + 1 <= 2^d)
-    const int next = ((cell[2] + 1) >> 5) - (cell[2] >> 5);
-    NodeWord lo[4], hi[4];
+    const int w = word_of(cell[2]), bit = cell[2] - 31 * w;
+    NodeWord word[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) word[k] = f.words[word_at(d, cell[0] + k / 2, cell[1] + k % 2, w)];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const NodeWord* w = at + (k / 2 * (n + 1) + k % 2) * wc;
-      lo[k] = w[0];
-      hi[k] = w[next];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      c.idx[2 * k] = node_in_word(lo[k], cell[2]);
-      c.idx[2 * k + 1] = node_in_word(hi[k], cell[2] + 1);
+      c.present[k] = (word[k].bits >> bit) & 3u;
+      c.first[k] = c.present[k] ? word[k].first + __popc(word[k].bits & ((1u << bit) - 1u)) : 0;
     }
   } else {
     for (int a = 0; a < 2; ++a)
       for (int b = 0; b < 2; ++b) {
         int64_t found[2];
         level_run<2>(f, d, cell[0] + a, cell[1] + b, cell[2], 2, found);
-        c.idx[4 * a + 2 * b] = (int)found[0];
-        c.idx[4 * a + 2 * b + 1] = (int)found[1];
+        c.present[2 * a + b] = (found[0] >= 0 ? 1u : 0u) | (found[1] >= 0 ? 2u : 0u);
+        c.first[2 * a + b] = (int)(found[0] >= 0 ? found[0] : found[1] >= 0 ? found[1] : 0);
       }
   }
   // a corner left of the point's floor (a knot owned by the left cell) does not count
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
-    if (imin(imin(cell[0] + k / 4 - base[0], cell[1] + k / 2 % 2 - base[1]), cell[2] + k % 2 - base[2]) < 0) c.idx[k] = -1;
+  for (int k = 0; k < 4; ++k)
+    c.counts[k] = imin(cell[0] + k / 2 - base[0], cell[1] + k % 2 - base[1]) < 0
+                      ? 0u
+                      : c.present[k] & ((cell[2] < base[2] ? 0u : 1u) | (cell[2] + 1 < base[2] ? 0u : 2u));
+}
+
+// The pair's two values of a field array (K + 1 values: the last pair's
+// second one is never counted), +0 where the node does not count.
+template <class T> struct ValuePair;
+template <> struct ValuePair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct ValuePair<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
+template <class T>
+__device__ __forceinline__ void corner_values(const Corners<T>& c, bool used, const T* __restrict__ src, T* v) {
+  using Pair = typename ValuePair<T>::type;
+  Pair p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) p[k] = *(const Pair*)(src + c.first[k]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const T a = p[k].x, b = p[k].y;
+    v[2 * k] = used && (c.counts[k] & 1u) ? a : T(0);
+    v[2 * k + 1] = used && (c.counts[k] & 2u) ? ((c.present[k] & 1u) ? b : a) : T(0);
+  }
 }
 
 // field.py:371-393 (add_level), sums only, corners in order.  An absent
@@ -142,9 +162,13 @@ __device__ __forceinline__ void blend_corners(const Corners<T>& c, const T* v, i
 // field.py:395-420 (reference evaluation kernel).  WORDS: every level has
 // node words, so the three dependent steps (leaf words, the three blended
 // levels' words, their coefficients) each issue all their loads at once; the
-// general form searches level by level.
+// general form searches level by level, a chain of some 40 dependent loads
+// (812,000 queries at depth 9 in float64: 561 us; 151 us with words, bound by
+// the lines they miss).  Four waves a SIMD: 127 registers, 136 without the
+// limit.
 template <class T, bool WORDS>
-__global__ void __launch_bounds__(256) k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth,
                                                   const T* __restrict__ queries, int64_t m, Affine<T> A, int point_div_mode,
                                                   const T* __restrict__ divisors, T* __restrict__ values, T* __restrict__ grads,
                                                   int* __restrict__ valid) {
@@ -181,12 +205,13 @@ __global__ void __launch_bounds__(256) k_evaluate(FieldIndex f, const T* __restr
       for (int k = 0; k < AHEAD; ++k) {
         const int d = imax(top - k, 0), up = depth - d;
         const int x = cf[0] >> up, y = cf[1] >> up, z = cf[2] >> up;
-        w[k] = f.words[word_base(d) + (uint32_t)(x * ((1 << d) + 1) + y) * (uint32_t)word_columns(d) + (uint32_t)(z >> 5)];
+        w[k] = f.words[word_at(d, x, y, word_of(z))];
       }
 #pragma unroll
       for (int k = 0; k < AHEAD; ++k) {
         const int d = imax(top - k, 0);
-        if (!found && ((w[k].bits >> ((cf[2] >> (depth - d)) & 31)) & 1u)) { leaf = d; found = true; }
+        const int z = cf[2] >> (depth - d);
+        if (!found && ((w[k].bits >> (z - 31 * word_of(z))) & 1u)) { leaf = d; found = true; }
       }
     }
   } else {
@@ -210,12 +235,9 @@ __global__ void __launch_bounds__(256) k_evaluate(FieldIndex f, const T* __restr
   find_corners<T, WORDS>(f, p, imax(leaf - 1, 0), c1);
   find_corners<T, WORDS>(f, p, imin(leaf + 1, depth), c2);
   T v0[8], v1[8], v2[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    v0[k] = c0.idx[k] >= 0 ? coef[c0.idx[k]] : T(0);
-    v1[k] = lower && c1.idx[k] >= 0 ? cum[c1.idx[k]] : T(0);
-    v2[k] = upper && c2.idx[k] >= 0 ? coef[c2.idx[k]] : T(0);
-  }
+  corner_values(c0, true, coef, v0);
+  corner_values(c1, lower, cum, v1);
+  corner_values(c2, upper, coef, v2);
   T res[4] = {T(0), T(0), T(0), T(0)};
   blend_corners(c0, v0, leaf, res);
   if (lower) {
@@ -432,7 +454,8 @@ template <class T> void stage_field(Result<T>& r) {
   for (int d = 0; d <= D; ++d) r.level_offsets[d + 1] = r.level_offsets[d] + r.levels[d].basis_count;
   const int64_t K = r.level_offsets[D + 1];
   r.keys.reset(K, s);
-  r.coefficients.reset(K, s);
+  r.coefficients.reset(K + 1, s);  // one value more: corner_values loads pairs
+  r.coefficients.shrink(K);
   for (int d = 0; d <= D; ++d) {
     const LevelState<T>& L = r.levels[d];
     const int64_t o = r.level_offsets[d];
@@ -450,8 +473,7 @@ template <class T> void stage_field(Result<T>& r) {
   const bool tables = D <= field_table_max_depth() && K;
   r.word_depth = tables ? field_word_depth(D) : -1;
   if (r.word_depth >= 0) {
-    r.node_words.reset(word_base(r.word_depth) + ((size_t)1 + ((size_t)1 << r.word_depth)) * ((1 << r.word_depth) + 1) *
-                                                     word_columns(r.word_depth), s);
+    r.node_words.reset(word_base(r.word_depth + 1), s);
     r.node_words.zero();
     hipLaunchKernelGGL(k_field_words, dim3(blocks_for(K, 256)), dim3(256), 0, s, (const int64_t*)r.keys.data(), K, r.word_depth,
                        r.node_words.data());
@@ -473,7 +495,8 @@ template <class T> void stage_field(Result<T>& r) {
     r.column_end.free();
   }
   const FieldIndex f = field_index(r);
-  r.cumulative.reset(K, s);
+  r.cumulative.reset(K + 1, s);
+  r.cumulative.shrink(K);
   if (K) HIP_CHECK(hipMemcpyAsync(r.cumulative.data(), r.coefficients.data(), sizeof(T) * K, hipMemcpyDeviceToDevice, s));
   for (int d = 1; d <= D; ++d) {
     const int cnt = r.levels[d].basis_count;

@@ -8,7 +8,8 @@ namespace psr {
 
 // Presence of 32 z-consecutive nodes of one (x, y) column of a level and the
 // concatenated index of the word's first present node: a lookup is one 8-byte
-// load and a population count, because keys are sorted with z fastest.
+// load and a population count, because keys are sorted with z fastest.  Words
+// overlap by a node (word_columns).
 struct NodeWord {
   uint32_t bits;
   int32_t first;
@@ -114,8 +115,8 @@ template <class T> struct Result {
   DArray<T> coefficients, cumulative, centroid_values;
   std::vector<int> level_offsets;  // concatenated key offsets per depth
   DArray<int> offsets_dev;         // the same on the device
-  // node words of levels 0..word_depth of keys, level after level, x-major
-  // (2^d + 1)^2 columns of ceil((2^d + 1) / 32) words each: 41 MB at depth 9,
+  // node words of levels 0..word_depth of keys, level after level (word_at),
+  // ceil(2^d / 31) for each of the (2^d + 1)^2 columns: 42 MB at depth 9;
   // deeper levels have none (see field_word_depth)
   DArray<NodeWord> node_words;
   int word_depth = -1;
