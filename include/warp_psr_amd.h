@@ -256,6 +256,19 @@ int psr_isovalue_noalloc(int dtype, const void* values, const void* weights, int
 int psr_field_evaluate(const PsrField* field, const void* queries, int64_t m, void* values, void* grads, int32_t* valid,
                        void* stream);
 
+/* Node words of a caller's field (a LevelField over its own keys): presence
+ * bits and ranks that answer a key lookup in one load.  With words NULL only
+ * *bytes is written: what they take, 0 for a field without words (depth
+ * beyond 9, or beyond PSR_DENSE_INDEX_MAX_CELLS).  Otherwise builds them in
+ * words (*bytes, device) and sets the device flag *sorted to 1, or to 0 where
+ * the keys do not ascend strictly on their levels' grids.
+ * psr_field_evaluate_words is psr_field_evaluate through them, with the same
+ * bits (also where *sorted is 0: it searches the keys then).  Words belong to
+ * the keys they were built from. */
+int psr_field_words(const int64_t* keys, int64_t count, int depth, void* words, int64_t* bytes, int32_t* sorted, void* stream);
+int psr_field_evaluate_words(const PsrField* field, const void* words, const int32_t* sorted, const void* queries, int64_t m,
+                             void* values, void* grads, int32_t* valid, void* stream);
+
 const char* psr_last_error(void);
 /* Frees the library's cached device blocks. */
 void psr_release_cache(void);

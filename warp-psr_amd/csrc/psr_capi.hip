@@ -5,6 +5,7 @@
 #include "../../include/warp_psr_amd.h"
 #include "../../include/warp_psr_amd_field.h"
 #include "psr_result.h"
+#include "psr_field_index.h"
 #include "psr_mesh.h"
 #include "psr_meta.h"
 
@@ -619,6 +620,52 @@ int psr_field_evaluate(const PsrField* field, const void* queries, int64_t m, vo
       hipLaunchKernelGGL(k_field_evaluate<double>, dim3(blocks_for(m, 256)), dim3(256), 0, s, *field,
                          (const double*)queries, m, (double*)values, (double*)grads, valid);
     KERNEL_CHECK();
+    return 0;
+  } catch (const PsrError& e) {
+    return fail(e);
+  } catch (const std::exception& e) {
+    g_error = e.what();
+    return 1;
+  }
+}
+
+int psr_field_words(const int64_t* keys, int64_t count, int depth, void* words, int64_t* bytes, int32_t* sorted, void* stream) {
+  try {
+    if (!bytes) throw PsrError(2, "bytes must be non-null");
+    if (depth < 0 || depth > 15) throw PsrError(2, "Keys support depths 0..15, including upper boundary nodes");
+    if (count < 0) throw PsrError(2, "key count must be nonnegative");
+    const int64_t need = level_field_words(count, depth) * (int64_t)sizeof(NodeWord);
+    if (!words) {
+      *bytes = need;
+      return 0;
+    }
+    if (*bytes < need || !need) throw PsrError(2, "words must hold the bytes psr_field_words asks for");
+    if (!sorted || (count && !keys)) throw PsrError(2, "keys and sorted must be non-null");
+    build_level_field_words(keys, count, depth, (NodeWord*)words, (int*)sorted, (hipStream_t)stream);
+    return 0;
+  } catch (const PsrError& e) {
+    return fail(e);
+  } catch (const std::exception& e) {
+    g_error = e.what();
+    return 1;
+  }
+}
+
+int psr_field_evaluate_words(const PsrField* field, const void* words, const int32_t* sorted, const void* queries, int64_t m,
+                             void* values, void* grads, int32_t* valid, void* stream) {
+  try {
+    if (!field || !field->keys || !field->level_offsets) throw PsrError(2, "field must be a psr_result_field view");
+    if (field->dtype != 0 && field->dtype != 1) throw PsrError(3, "field dtype must be 0 (float32) or 1 (float64)");
+    if (!words || !sorted || !level_field_words(field->count, field->depth)) throw PsrError(2, "the field has no node words");
+    if (m < 0) throw PsrError(2, "query count must be nonnegative");
+    if (m == 0) return 0;
+    if (!queries || !values) throw PsrError(2, "queries and values must be non-null");
+    if (field->dtype == 0)
+      evaluate_level_field(*field, (const NodeWord*)words, (const int*)sorted, (const float*)queries, m, (float*)values,
+                           (float*)grads, (int*)valid, (hipStream_t)stream);
+    else
+      evaluate_level_field(*field, (const NodeWord*)words, (const int*)sorted, (const double*)queries, m, (double*)values,
+                           (double*)grads, (int*)valid, (hipStream_t)stream);
     return 0;
   } catch (const PsrError& e) {
     return fail(e);

@@ -2,6 +2,7 @@
 // reference evaluation (field.py:364-421), the isovalue
 // (reconstruction.py:76-138) and the cube/model transforms (transforms.py).
 #include "psr_field_index.h"
+#include "../../include/warp_psr_amd_field.h"
 
 #include <cmath>
 
@@ -48,9 +49,8 @@ template <class T> PSR_HD int clampi(int v, int lo, int hi) { return v < lo ? lo
 // below the word's first node) collects the word's keys, at most 32, so no two
 // threads write one word.  A shared node can be the first key of both its
 // words.  Words without keys keep the cleared value (no bits).
-__global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int word_depth, NodeWord* __restrict__ words) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+__device__ __forceinline__ void field_word(const int64_t* __restrict__ keys, int64_t n, int word_depth,
+                                           NodeWord* __restrict__ words, int64_t i) {
   const int64_t key = keys[i];
   const int d = key_d(key);
   if (d > word_depth) return;
@@ -65,15 +65,23 @@ __global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int w
   }
 }
 
-// One level's eight trilinear corners of a cube point: weights and, for each
-// of the four z pairs, the index of the first node present (0 if none) and
-// which of the two count (bit 0 the lower, bit 1 the upper): present and not
-// left of the point's floor.  Present pairs are neighbours in memory.
+__global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int word_depth, NodeWord* __restrict__ words) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) field_word(keys, n, word_depth, words, i);
+}
+
+// One level's eight trilinear corners of a cube point: for each of the four z
+// pairs, the index of the first node present (0 if none), which
+// of the two are present (two bits each, the lower node's first) and which
+// count: present and not left of the point's floor.  A present pair's nodes
+// are neighbours in memory.  up: cell + 1 > floor, so the upper corner has
+// weight fr, else 1 - fr.  Flags are packed: registers bound the kernel.
 template <class T> struct Corners {
   int first[4];
-  unsigned present[4], counts[4];
-  T fr[3];
-  bool up[3];  // cell + 1 > floor: the upper corner has weight fr, else 1 - fr
+  unsigned flags;  // present: bits 0..7, counts: bits 8..15, up: bits 16..18
+  __device__ __forceinline__ unsigned present(int k) const { return (flags >> (2 * k)) & 3u; }
+  __device__ __forceinline__ unsigned counts(int k) const { return (flags >> (8 + 2 * k)) & 3u; }
+  __device__ __forceinline__ bool up(int a) const { return (flags >> (16 + a)) & 1u; }
 };
 
 // field.py:371-393 (add_level), lookups only
@@ -81,13 +89,13 @@ template <class T, bool WORDS>
 __device__ __forceinline__ void find_corners(const FieldIndex& f, const T* p, int d, Corners<T>& c) {
   const int n = 1 << d;
   int cell[3], base[3];
+  c.flags = 0;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const T t = p[a] * T(n);
     cell[a] = clampi<T>((int)ceil(t) - 1, 0, n - 1);
     base[a] = (int)floor(t);
-    c.fr[a] = t - T(base[a]);
-    c.up[a] = cell[a] + 1 > base[a];
+    c.flags |= cell[a] + 1 > base[a] ? 1u << (16 + a) : 0u;
   }
   if constexpr (WORDS) {
     const int w = word_of(cell[2]), bit = cell[2] - 31 * w;
@@ -96,42 +104,51 @@ __device__ __forceinline__ void find_corners(const FieldIndex& f, const T* p, in
     for (int k = 0; k < 4; ++k) word[k] = f.words[word_at(d, cell[0] + k / 2, cell[1] + k % 2, w)];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      c.present[k] = (word[k].bits >> bit) & 3u;
-      c.first[k] = c.present[k] ? word[k].first + __popc(word[k].bits & ((1u << bit) - 1u)) : 0;
+      const unsigned present = (word[k].bits >> bit) & 3u;
+      c.flags |= present << (2 * k);
+      c.first[k] = present ? word[k].first + __popc(word[k].bits & ((1u << bit) - 1u)) : 0;
     }
   } else {
     for (int a = 0; a < 2; ++a)
       for (int b = 0; b < 2; ++b) {
         int64_t found[2];
         level_run<2>(f, d, cell[0] + a, cell[1] + b, cell[2], 2, found);
-        c.present[2 * a + b] = (found[0] >= 0 ? 1u : 0u) | (found[1] >= 0 ? 2u : 0u);
+        c.flags |= ((found[0] >= 0 ? 1u : 0u) | (found[1] >= 0 ? 2u : 0u)) << (2 * (2 * a + b));
         c.first[2 * a + b] = (int)(found[0] >= 0 ? found[0] : found[1] >= 0 ? found[1] : 0);
       }
   }
   // a corner left of the point's floor (a knot owned by the left cell) does not count
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-    c.counts[k] = imin(cell[0] + k / 2 - base[0], cell[1] + k % 2 - base[1]) < 0
-                      ? 0u
-                      : c.present[k] & ((cell[2] < base[2] ? 0u : 1u) | (cell[2] + 1 < base[2] ? 0u : 2u));
+  for (int k = 0; k < 4; ++k) {
+    const unsigned right = (cell[2] < base[2] ? 0u : 1u) | (cell[2] + 1 < base[2] ? 0u : 2u);
+    if (imin(cell[0] + k / 2 - base[0], cell[1] + k % 2 - base[1]) >= 0) c.flags |= (c.present(k) & right) << (8 + 2 * k);
+  }
 }
 
-// The pair's two values of a field array (K + 1 values: the last pair's
-// second one is never counted), +0 where the node does not count.
+// The pair's two values of a field array, +0 where the node does not count.
+// PAIRS: one load of both, for arrays of K + 1 values (the last pair's second
+// one is never counted); else two, of present nodes.
 template <class T> struct ValuePair;
 template <> struct ValuePair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
 template <> struct ValuePair<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
-template <class T>
+template <bool PAIRS, class T>
 __device__ __forceinline__ void corner_values(const Corners<T>& c, bool used, const T* __restrict__ src, T* v) {
   using Pair = typename ValuePair<T>::type;
   Pair p[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) p[k] = *(const Pair*)(src + c.first[k]);
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (PAIRS) {
+      p[k] = *(const Pair*)(src + c.first[k]);
+    } else {
+      p[k].x = c.present(k) ? src[c.first[k]] : T(0);
+      p[k].y = c.present(k) == 3u ? src[c.first[k] + 1] : T(0);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const T a = p[k].x, b = p[k].y;
-    v[2 * k] = used && (c.counts[k] & 1u) ? a : T(0);
-    v[2 * k + 1] = used && (c.counts[k] & 2u) ? ((c.present[k] & 1u) ? b : a) : T(0);
+    v[2 * k] = used && (c.counts(k) & 1u) ? a : T(0);
+    v[2 * k + 1] = used && (c.counts(k) & 2u) ? ((c.present(k) & 1u) ? b : a) : T(0);
   }
 }
 
@@ -139,15 +156,16 @@ __device__ __forceinline__ void corner_values(const Corners<T>& c, bool used, co
 // corner enters as the coefficient +0: its products are zeros of either sign,
 // and a sum that starts at +0 is never -0, so adding them changes no bit.
 template <class T>
-__device__ __forceinline__ void blend_corners(const Corners<T>& c, const T* v, int d, T* res) {
+__device__ __forceinline__ void blend_corners(const Corners<T>& c, const T* v, const T* p, int d, T* res) {
   const T n = T(1 << d);
   T h[3][2], sg[3][2];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {  // lower corner: node <= floor, upper corner: by `up`
-    h[a][0] = T(1) - c.fr[a];
+    const T t = p[a] * n, fr = t - T((int)floor(t));
+    h[a][0] = T(1) - fr;
     sg[a][0] = T(-1);
-    h[a][1] = c.up[a] ? c.fr[a] : T(1) - c.fr[a];
-    sg[a][1] = c.up[a] ? T(1) : T(-1);
+    h[a][1] = c.up(a) ? fr : T(1) - fr;
+    sg[a][1] = c.up(a) ? T(1) : T(-1);
   }
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
@@ -159,36 +177,17 @@ __device__ __forceinline__ void blend_corners(const Corners<T>& c, const T* v, i
   }
 }
 
-// field.py:395-420 (reference evaluation kernel).  WORDS: every level has
+// field.py:395-420 (reference evaluation) at a cube point p, nudged off the
+// cube's faces here: value and cube-space gradient.  WORDS: every level has
 // node words, so the three dependent steps (leaf words, the three blended
 // levels' words, their coefficients) each issue all their loads at once; the
 // general form searches level by level, a chain of some 40 dependent loads
 // (812,000 queries at depth 9 in float64: 561 us; 151 us with words, bound by
-// the lines they miss).  Four waves a SIMD: 127 registers, 136 without the
-// limit.
-template <class T, bool WORDS>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth,
-                                                  const T* __restrict__ queries, int64_t m, Affine<T> A, int point_div_mode,
-                                                  const T* __restrict__ divisors, T* __restrict__ values, T* __restrict__ grads,
-                                                  int* __restrict__ valid) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  T q0 = queries[3 * i], q1 = queries[3 * i + 1], q2 = queries[3 * i + 2];
-  if (point_div_mode) {  // reconstruction.py:23-29 (_centroids)
-    const T w = divisors[i];
-    q0 = q0 / w; q1 = q1 / w; q2 = q2 / w;
-  }
-  T p[3];
-  for (int r = 0; r < 3; ++r) p[r] = A.L[3 * r] * q0 + A.L[3 * r + 1] * q1 + A.L[3 * r + 2] * q2 + A.t[r];
-  const bool ok = isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2]) && tmin(tmin(p[0], p[1]), p[2]) >= T(0) &&
-                  tmax(tmax(p[0], p[1]), p[2]) <= T(1);
-  if (valid) valid[i] = ok ? 1 : 0;
-  if (!ok) {
-    values[i] = T(NAN);
-    if (grads) { grads[3 * i] = T(NAN); grads[3 * i + 1] = T(NAN); grads[3 * i + 2] = T(NAN); }
-    return;
-  }
+// the lines they miss; 156 us where four waves a SIMD are asked for, which
+// spills).
+template <class T, bool WORDS, bool PAIRS>
+__device__ __forceinline__ void field_at(const FieldIndex& f, const T* __restrict__ coef, const T* __restrict__ cum, int depth, T (&p)[3],
+                                         T (&res)[4]) {
   int leaf = 0;
   if constexpr (WORDS) {
     // the cell at level d is the finest cell >> (depth - d): scaling by a
@@ -235,24 +234,162 @@ k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, 
   find_corners<T, WORDS>(f, p, imax(leaf - 1, 0), c1);
   find_corners<T, WORDS>(f, p, imin(leaf + 1, depth), c2);
   T v0[8], v1[8], v2[8];
-  corner_values(c0, true, coef, v0);
-  corner_values(c1, lower, cum, v1);
-  corner_values(c2, upper, coef, v2);
-  T res[4] = {T(0), T(0), T(0), T(0)};
-  blend_corners(c0, v0, leaf, res);
+  corner_values<PAIRS>(c0, true, coef, v0);
+  corner_values<PAIRS>(c1, lower, cum, v1);
+  corner_values<PAIRS>(c2, upper, coef, v2);
+  res[0] = res[1] = res[2] = res[3] = T(0);
+  blend_corners(c0, v0, p, leaf, res);
   if (lower) {
     T r2[4] = {T(0), T(0), T(0), T(0)};
-    blend_corners(c1, v1, leaf - 1, r2);
+    blend_corners(c1, v1, p, leaf - 1, r2);
     for (int a = 0; a < 4; ++a) res[a] = res[a] + r2[a];
   }
   if (upper) {
     T r2[4] = {T(0), T(0), T(0), T(0)};
-    blend_corners(c2, v2, leaf + 1, r2);
+    blend_corners(c2, v2, p, leaf + 1, r2);
     for (int a = 0; a < 4; ++a) res[a] = res[a] + r2[a];
   }
+}
+
+template <class T, bool WORDS>
+__global__ void __launch_bounds__(256)
+k_evaluate(FieldIndex f, const T* __restrict__ coef, const T* __restrict__ cum, int depth, const T* __restrict__ queries, int64_t m, Affine<T> A, int point_div_mode,
+                                                  const T* __restrict__ divisors, T* __restrict__ values, T* __restrict__ grads,
+                                                  int* __restrict__ valid) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  T q0 = queries[3 * i], q1 = queries[3 * i + 1], q2 = queries[3 * i + 2];
+  if (point_div_mode) {  // reconstruction.py:23-29 (_centroids)
+    const T w = divisors[i];
+    q0 = q0 / w; q1 = q1 / w; q2 = q2 / w;
+  }
+  T p[3];
+  for (int r = 0; r < 3; ++r) p[r] = A.L[3 * r] * q0 + A.L[3 * r + 1] * q1 + A.L[3 * r + 2] * q2 + A.t[r];
+  const bool ok = isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2]) && tmin(tmin(p[0], p[1]), p[2]) >= T(0) &&
+                  tmax(tmax(p[0], p[1]), p[2]) <= T(1);
+  if (valid) valid[i] = ok ? 1 : 0;
+  if (!ok) {
+    values[i] = T(NAN);
+    if (grads) { grads[3 * i] = T(NAN); grads[3 * i + 1] = T(NAN); grads[3 * i + 2] = T(NAN); }
+    return;
+  }
+  T res[4];
+  field_at<T, WORDS, true>(f, coef, cum, depth, p, res);
   values[i] = res[0];
   if (grads)
     for (int c = 0; c < 3; ++c) grads[3 * i + c] = A.L[c] * res[1] + A.L[3 + c] * res[2] + A.L[6 + c] * res[3];
+}
+
+// field.py:37-75 (evaluation_function): direct summation over all levels of a
+// field without cumulative coefficients, as psr_field_detail::direct_levels
+// with the cells' words.  Absent corners add +0 products, which change no bit.
+template <class T>
+__device__ __forceinline__ void direct_at(const FieldIndex& f, const T* __restrict__ coef, int depth, const T* p, T* res) {
+  for (int d = 0; d <= depth; ++d) {
+    const int n = 1 << d;
+    Corners<T> c;
+    c.flags = 0;
+    int cell[3];
+    T fr[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const T t = p[a] * T(n);
+      cell[a] = clampi<T>((int)ceil(t) - 1, 0, n - 1);
+      fr[a] = t - T(cell[a]);
+    }
+    const int w = word_of(cell[2]), bit = cell[2] - 31 * w;
+    NodeWord word[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) word[k] = f.words[word_at(d, cell[0] + k / 2, cell[1] + k % 2, w)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const unsigned present = (word[k].bits >> bit) & 3u;
+      c.flags |= present << (2 * k) | present << (8 + 2 * k);
+      c.first[k] = present ? word[k].first + __popc(word[k].bits & ((1u << bit) - 1u)) : 0;
+    }
+    T v[8];
+    corner_values<false>(c, true, coef, v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int o[3] = {k / 4, k / 2 % 2, k % 2};
+      T h[3], sg[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        h[a] = o[a] ? fr[a] : T(1) - fr[a];
+        sg[a] = o[a] ? T(1) : T(-1);
+      }
+      res[0] = res[0] + v[k] * h[0] * h[1] * h[2];
+      const T cn = v[k] * T(n);
+      res[1] = res[1] + cn * (sg[0] * h[1] * h[2]);
+      res[2] = res[2] + cn * (h[0] * sg[1] * h[2]);
+      res[3] = res[3] + cn * (h[0] * h[1] * sg[2]);
+    }
+  }
+}
+
+// A caller's field through its node words: the bits of psr_evaluate_field,
+// whose searches it takes itself where *sorted is 0 (keys that are not
+// strictly ascending, or off the grid, have no words).  100,003 queries at
+// depth 8 in float64: 130 us by searches, 18 us by words.
+template <class T>
+__global__ void __launch_bounds__(256) k_level_field(PsrField field, FieldIndex f, const int* __restrict__ sorted,
+                                                     const T* __restrict__ queries, int64_t m, T* __restrict__ values,
+                                                     T* __restrict__ grads, int* __restrict__ valid) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m) return;
+  const T q[3] = {queries[3 * i], queries[3 * i + 1], queries[3 * i + 2]};
+  if (!*sorted) {
+    T v, g[3];
+    const int ok = psr_evaluate_field<T>(field, q, &v, grads ? g : nullptr);
+    values[i] = v;
+    if (grads) { grads[3 * i] = g[0]; grads[3 * i + 1] = g[1]; grads[3 * i + 2] = g[2]; }
+    if (valid) valid[i] = ok;
+    return;
+  }
+  T L[9], t[3], p[3];
+  for (int k = 0; k < 9; ++k) L[k] = T(field.linear[k]);
+  for (int k = 0; k < 3; ++k) t[k] = T(field.translation[k]);
+  for (int r = 0; r < 3; ++r) p[r] = L[3 * r] * q[0] + L[3 * r + 1] * q[1] + L[3 * r + 2] * q[2] + t[r];
+  const bool ok = isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2]) && tmin(tmin(p[0], p[1]), p[2]) >= T(0) &&
+                  tmax(tmax(p[0], p[1]), p[2]) <= T(1);
+  if (valid) valid[i] = ok ? 1 : 0;
+  T res[4] = {T(0), T(0), T(0), T(0)};
+  if (!ok) {
+    values[i] = T(NAN);
+    if (grads) { grads[3 * i] = T(NAN); grads[3 * i + 1] = T(NAN); grads[3 * i + 2] = T(NAN); }
+    return;
+  }
+  const T* coef = (const T*)field.coefficients;
+  const T* cum = (const T*)field.cumulative;
+  if (cum)
+    field_at<T, true, false>(f, coef, cum, field.depth, p, res);
+  else
+    direct_at(f, coef, field.depth, p, res);
+  values[i] = res[0];
+  if (grads)
+    for (int c = 0; c < 3; ++c) grads[3 * i + c] = L[c] * res[1] + L[3 + c] * res[2] + L[6 + c] * res[3];
+}
+
+// *sorted stays 1 if the keys ascend strictly and lie on their levels' grids
+__global__ void k_keys_sorted(const int64_t* __restrict__ keys, int64_t n, int depth, int* __restrict__ sorted) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t k = keys[i];
+  const int d = key_d(k), top = imax(imax(key_x(k), key_y(k)), key_z(k));
+  if (k < 0 || d > depth || top > (1 << d) || (i > 0 && keys[i - 1] >= k)) *sorted = 0;
+}
+
+__global__ void k_clear_words(NodeWord* __restrict__ words, uint32_t n, int* __restrict__ sorted) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) words[i] = NodeWord{0u, 0};
+  if (i == 0) *sorted = 1;
+}
+
+// k_field_words over keys that may be off the grid (sorted 0): nothing then
+__global__ void k_level_field_words(const int64_t* __restrict__ keys, int64_t n, int depth, const int* __restrict__ sorted,
+                                    NodeWord* __restrict__ words) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && *sorted) field_word(keys, n, depth, words, i);
 }
 
 // Isovalue: <=1024 aggregates one serial double chain (reconstruction.py:66-83);
@@ -443,6 +580,38 @@ static int field_word_depth(int depth) {
   }
   return d;
 }
+
+int64_t level_field_words(int64_t count, int depth) {
+  return count <= INT32_MAX && depth >= 0 && field_word_depth(depth) == depth ? (int64_t)word_base(depth + 1) : 0;
+}
+
+void build_level_field_words(const int64_t* keys, int64_t count, int depth, NodeWord* words, int* sorted, hipStream_t s) {
+  const uint32_t n = word_base(depth + 1);
+  hipLaunchKernelGGL(k_clear_words, dim3(blocks_for(n, 256)), dim3(256), 0, s, words, n, sorted);
+  KERNEL_CHECK();
+  if (!count) return;
+  hipLaunchKernelGGL(k_keys_sorted, dim3(blocks_for(count, 256)), dim3(256), 0, s, keys, count, depth, sorted);
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_level_field_words, dim3(blocks_for(count, 256)), dim3(256), 0, s, keys, count, depth, (const int*)sorted,
+                     words);
+  KERNEL_CHECK();
+}
+
+template <class T>
+void evaluate_level_field(const PsrField& field, const NodeWord* words, const int* sorted, const T* queries, int64_t m, T* values,
+                          T* grads, int* valid, hipStream_t s) {
+  FieldIndex f{};
+  f.keys = field.keys;
+  f.off = field.level_offsets;
+  f.words = words;
+  f.word_depth = field.depth;
+  hipLaunchKernelGGL(k_level_field<T>, dim3(blocks_for(m, 256)), dim3(256), 0, s, field, f, sorted, queries, m, values, grads, valid);
+  KERNEL_CHECK();
+}
+template void evaluate_level_field<float>(const PsrField&, const NodeWord*, const int*, const float*, int64_t, float*, float*, int*,
+                                          hipStream_t);
+template void evaluate_level_field<double>(const PsrField&, const NodeWord*, const int*, const double*, int64_t, double*, double*,
+                                           int*, hipStream_t);
 
 template <class T> void stage_field(Result<T>& r) {
   hipStream_t s = r.s;

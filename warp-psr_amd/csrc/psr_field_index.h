@@ -3,6 +3,7 @@
 // tables), shared by the field stage and its adjoint.
 #pragma once
 #include "psr_result.h"
+#include "../../include/warp_psr_amd.h"
 
 namespace psr {
 
@@ -95,6 +96,15 @@ template <class T> inline FieldIndex field_index(const Result<T>& r) {
   f.end = r.column_start.empty() ? nullptr : r.column_end.data();
   return f;
 }
+
+// A caller's field (LevelField): the number of node words of its levels, 0 if
+// it takes none (levels beyond the dense limit), their construction
+// (*sorted = 0 for keys that have none) and the evaluation through them.
+int64_t level_field_words(int64_t count, int depth);
+void build_level_field_words(const int64_t* keys, int64_t count, int depth, NodeWord* words, int* sorted, hipStream_t s);
+template <class T>
+void evaluate_level_field(const PsrField& field, const NodeWord* words, const int* sorted, const T* queries, int64_t m, T* values,
+                          T* grads, int* valid, hipStream_t s);
 
 // model -> cube affine map of queries
 template <class T> struct Affine { T L[9]; T t[3]; };

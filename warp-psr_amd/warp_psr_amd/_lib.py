@@ -16,7 +16,7 @@ EXPORTED = (
     "psr_mesh_select", "psr_mesh_corner_points", "psr_mesh_triangulate", "psr_mesh_copy", "psr_mesh_vertex_vjp",
     "psr_mesh_case_table", "psr_mesh_free", "psr_tree_metadata", "psr_tree_metadata_levels", "psr_tree_metadata_level",
     "psr_tree_metadata_copy", "psr_tree_metadata_free", "psr_field_level_offsets", "psr_isovalue",
-    "psr_isovalue_noalloc",
+    "psr_isovalue_noalloc", "psr_field_words", "psr_field_evaluate_words",
 )
 
 
@@ -88,6 +88,10 @@ def load():
     lib.psr_field_evaluate.argtypes = [ctypes.POINTER(PsrField), vp, i64, vp, vp, vp, vp]
     lib.psr_field_level_offsets.restype = c_int
     lib.psr_field_level_offsets.argtypes = [vp, i64, c_int, vp, vp]
+    lib.psr_field_words.restype = c_int
+    lib.psr_field_words.argtypes = [vp, i64, c_int, vp, ctypes.POINTER(i64), vp, vp]
+    lib.psr_field_evaluate_words.restype = c_int
+    lib.psr_field_evaluate_words.argtypes = [ctypes.POINTER(PsrField), vp, vp, vp, i64, vp, vp, vp, vp]
     lib.psr_isovalue.restype = c_int
     lib.psr_isovalue.argtypes = [c_int, vp, vp, i64, vp, vp]
     lib.psr_isovalue_noalloc.restype = c_int

@@ -117,6 +117,7 @@ class LevelField:
         with torch.cuda.device(device):
             _lib.check(_lib.load().psr_field_level_offsets(self.keys.data_ptr(), self.keys.shape[0], depth,
                                                            self._offsets.data_ptr(), _stream_handle(device)))
+            self._words = self._words_of_keys(device)
         f = _lib.PsrField()
         f.keys, f.coefficients = self.keys.data_ptr(), self.coefficients.data_ptr()
         f.cumulative = None if self.cumulative is None else self.cumulative.data_ptr()
@@ -128,6 +129,20 @@ class LevelField:
             f.translation[i] = self.translation[i]
         f.iso_value = self.iso_value
         self._field = f
+
+    def _words_of_keys(self, device):
+        """The keys' node words and their device flag (psr_field_words), or None for a field without words."""
+        torch = _torch()
+        need = ctypes.c_int64()
+        args = (self.keys.data_ptr(), self.keys.shape[0], self.depth)
+        _lib.check(_lib.load().psr_field_words(*args, None, ctypes.byref(need), None, None))
+        if not need.value:
+            return None
+        words = torch.empty(need.value, dtype=torch.uint8, device=device)
+        flag = torch.empty(1, dtype=torch.int32, device=device)
+        _lib.check(_lib.load().psr_field_words(*args, words.data_ptr(), ctypes.byref(need), flag.data_ptr(),
+                                               _stream_handle(device)))
+        return words, flag
 
     @classmethod
     def _from_result(cls, result, dtype, device):
@@ -154,14 +169,19 @@ class LevelField:
         if (not isinstance(queries, torch.Tensor) or queries.dtype != self.dtype or queries.device != self.device
                 or queries.ndim != 2 or queries.shape[1] != 3):
             raise ValueError("Query precision/device must match coefficients")
-        if self._result is None:
+        if self._result is None and self._words is None:
             return self.device_field().evaluate(queries)
         q = queries.contiguous()
         m = q.shape[0]
         values = torch.empty(m, dtype=self.dtype, device=self.device)
         gradients = torch.empty((m, 3), dtype=self.dtype, device=self.device)
         valid = torch.empty(m, dtype=torch.int32, device=self.device)
-        if m:
+        if m and self._result is None:
+            words, flag = self._words
+            _lib.check(_lib.load().psr_field_evaluate_words(ctypes.byref(self._field), words.data_ptr(), flag.data_ptr(), q.data_ptr(),
+                                                            m, values.data_ptr(), gradients.data_ptr(), valid.data_ptr(),
+                                                            _stream_handle(self.device)))
+        elif m:
             _lib.check(_lib.load().psr_evaluate(self._result._handle, q.data_ptr(), m, values.data_ptr(),
                                                 gradients.data_ptr(), valid.data_ptr(), _stream_handle(self.device)))
         return values, gradients, valid
