@@ -195,6 +195,12 @@ int psr_mesh_begin(const int32_t shape[3], const float lower[3], const float upp
 int psr_mesh_slab_nodes(PsrMesh* mesh, int32_t start, int32_t width, int64_t* nodes);
 int psr_mesh_slab_points(PsrMesh* mesh, int32_t start, int32_t width, float* points);
 int psr_mesh_slab_values(PsrMesh* mesh, int32_t start, int32_t width, const float* values);
+/* psr_mesh_slab_points, the field less *iso (device) at them and
+ * psr_mesh_slab_values for every `slab` planes of cells, and the same at the
+ * selected cells' corners, for a float32 reconstruction: the numbers a callback
+ * over psr_evaluate gives. */
+int psr_mesh_field_values(PsrMesh* mesh, const PsrResult* result, const float* iso, int32_t slab);
+int psr_mesh_field_corners(PsrMesh* mesh, const PsrResult* result, const float* iso, float* values);
 int psr_mesh_select(PsrMesh* mesh, int64_t* retained, int32_t* invalid);
 int psr_mesh_corner_points(PsrMesh* mesh, float* points);
 int psr_mesh_triangulate(PsrMesh* mesh, const float* corner_values, int64_t* vertices, int64_t* triangles);

@@ -867,6 +867,34 @@ int psr_mesh_slab_values(PsrMesh* m, int32_t start, int32_t width, const float* 
   }
 }
 
+int psr_mesh_field_values(PsrMesh* m, const PsrResult* result, const float* iso, int32_t slab) {
+  try {
+    if (!m || !result || !iso) throw PsrError(2, "null argument");
+    if (result->dtype != 0) throw PsrError(2, "mesh extraction currently requires float32 fields");
+    mc_field_values(*m->state, *(const Result<float>*)result->impl, iso, slab);
+    return 0;
+  } catch (const PsrError& e) {
+    return fail(e);
+  } catch (const std::exception& e) {
+    g_error = e.what();
+    return 1;
+  }
+}
+
+int psr_mesh_field_corners(PsrMesh* m, const PsrResult* result, const float* iso, float* values) {
+  try {
+    if (!m || !result || !iso || !values) throw PsrError(2, "null argument");
+    if (result->dtype != 0) throw PsrError(2, "mesh extraction currently requires float32 fields");
+    mc_field_corners(*m->state, *(const Result<float>*)result->impl, iso, values);
+    return 0;
+  } catch (const PsrError& e) {
+    return fail(e);
+  } catch (const std::exception& e) {
+    g_error = e.what();
+    return 1;
+  }
+}
+
 int psr_mesh_select(PsrMesh* m, int64_t* retained, int32_t* invalid) {
   try {
     if (!m || !retained || !invalid) throw PsrError(2, "null argument");

@@ -14,6 +14,7 @@
 // increasing values) and is fanned into triangles from its first edge.
 #include "psr_runtime.h"
 #include "psr_mesh.h"
+#include "psr_bitmap.h"
 
 #include <algorithm>
 #include <cmath>
@@ -137,21 +138,7 @@ void upload_table() {
   done.push_back(dev);
 }
 
-struct Grid {
-  int nx, ny, nz;
-  float lo[3], hi[3], step[3];
-};
-
-// meshing.py:37-41 and :88-94 (lower + step * node, clamped to the box),
-// rounded after the product and after the sum
-__device__ __forceinline__ void node_point(const Grid& g, int x, int y, int z, float* out) {
-  const int c[3] = {x, y, z};
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float p = g.lo[a] + g.step[a] * float(c[a]);
-    out[a] = fminf(fmaxf(p, g.lo[a]), g.hi[a]);
-  }
-}
+using Grid = MeshGrid;
 
 __global__ void k_mc_slab_points(Grid g, int start, int64_t n, float* __restrict__ out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -201,13 +188,6 @@ __global__ void k_mc_emit(const uint32_t* __restrict__ mask, int64_t words, cons
     cells[out++] = (int)(w * 32 + b);
     bits &= bits - 1;
   }
-}
-
-__device__ __forceinline__ void cell_xyz(const Grid& g, int cell, int& x, int& y, int& z) {
-  const int cy = g.ny - 1, cz = g.nz - 1;
-  x = cell / (cy * cz);
-  y = (cell / cz) % cy;
-  z = cell % cz;
 }
 
 // meshing.py:88-94 (_cell_points): 8 corners per retained cell
@@ -265,6 +245,61 @@ __global__ void k_mc_edge_keys(Grid g, const int* __restrict__ cells, const floa
   }
 }
 
+// The crossing edges as a bitmap over edge keys (psr_bitmap.h): a vertex's
+// index is its edge's rank, in key order, and the cell that defines it is the
+// lowest cell and edge that has it, as the first of the stable sort's equal
+// keys is.
+__global__ void k_mc_mark_edges(Grid g, const int* __restrict__ cells, const float* __restrict__ values, int n,
+                                int* __restrict__ tris, uint32_t* __restrict__ bits) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int code = cell_code(values + 8 * (int64_t)i);
+  int x, y, z;
+  cell_xyz(g, cells[i], x, y, z);
+  for (int e = 0; e < 12; ++e) {
+    if (((code >> c_edge[e][0]) & 1) == ((code >> c_edge[e][1]) & 1)) continue;
+    const uint64_t key = edge_key(g, x, y, z, e);
+    atomicOr(&bits[key >> 5], 1u << (unsigned)(key & 31));
+  }
+  tris[i] = c_tri_count[code];
+}
+
+struct EdgeRanks {
+  const uint32_t* bits;
+  const int* pre;
+  __device__ __forceinline__ int of(uint64_t key) const {
+    return pre[key >> 5] + __popc(bits[key >> 5] & ((1u << (unsigned)(key & 31)) - 1u));
+  }
+};
+
+__global__ void k_mc_clear_refs(int* __restrict__ refs, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) refs[i] = INT32_MAX;
+}
+
+__global__ void k_mc_edge_refs(Grid g, const int* __restrict__ cells, const float* __restrict__ values, int n, EdgeRanks ranks,
+                               int* __restrict__ refs) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int code = cell_code(values + 8 * (int64_t)i);
+  int x, y, z;
+  cell_xyz(g, cells[i], x, y, z);
+  for (int e = 0; e < 12; ++e)
+    if (((code >> c_edge[e][0]) & 1) != ((code >> c_edge[e][1]) & 1)) atomicMin(&refs[ranks.of(edge_key(g, x, y, z, e))], 12 * i + e);
+}
+
+__global__ void k_mc_rank_triangles(Grid g, const int* __restrict__ cells, const float* __restrict__ values, int n,
+                                    const int* __restrict__ tri_offsets, EdgeRanks ranks, int* __restrict__ indices) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int code = cell_code(values + 8 * (int64_t)i);
+  const int nt = c_tri_count[code];
+  int x, y, z;
+  cell_xyz(g, cells[i], x, y, z);
+  const int64_t out = 3 * (int64_t)tri_offsets[i];
+  for (int k = 0; k < 3 * nt; ++k) indices[out + k] = ranks.of(edge_key(g, x, y, z, c_tri_edges[code][k]));
+}
+
 // one vertex per unique edge: t = v_lo / (v_lo - v_hi) along the edge's
 // axis, in grid units, then lower + step * coordinate
 __global__ void k_mc_vertices(Grid g, const int* __restrict__ cells, const float* __restrict__ values,
@@ -272,7 +307,7 @@ __global__ void k_mc_vertices(Grid g, const int* __restrict__ cells, const float
                               int* __restrict__ vref) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= V) return;
-  const int ref = refs[head_pos[v]];
+  const int ref = refs[head_pos ? head_pos[v] : v];
   const int cell = ref / 12, e = ref % 12;
   int x, y, z;
   cell_xyz(g, cells[cell], x, y, z);
@@ -414,6 +449,22 @@ void mc_slab_values(McState& m, int start, int width, const float* values) {
   KERNEL_CHECK();
 }
 
+void mc_field_values(McState& m, const Result<float>& r, const float* iso, int slab) {
+  if (slab < 1) throw PsrError(2, "slab_size must be a positive integer");
+  const int planes = m.g.nx - 1, most = std::min(slab, planes);
+  DArray<float> values((size_t)mc_slab_nodes(m, 0, most), m.s);
+  for (int start = 0; start < planes; start += slab) {
+    const int width = std::min(slab, planes - start);
+    mesh_values(r, m.g, start, nullptr, mc_slab_nodes(m, start, width), iso, values.data(), m.s);
+    mc_slab_values(m, start, width, values.data());
+  }
+}
+
+void mc_field_corners(McState& m, const Result<float>& r, const float* iso, float* values) {
+  if (m.retained < 0) throw PsrError(2, "select the cells first");
+  if (m.retained) mesh_values(r, m.g, 0, m.cells.data(), 8 * (int64_t)m.retained, iso, values, m.s);
+}
+
 int mc_select(McState& m, int* invalid) {
   DArray<int> counts(m.words, m.s), offsets(m.words, m.s), total(1, m.s);
   hipLaunchKernelGGL(k_mc_word_counts, dim3(blocks_for(m.words, 256)), dim3(256), 0, m.s, (const uint32_t*)m.mask.data(),
@@ -444,12 +495,61 @@ void mc_corner_points(McState& m, float* out) {
   KERNEL_CHECK();
 }
 
+// Vertices and triangles by edge ranks: no sort, no search.
+static void triangulate_ranks(McState& m, const float* values, int64_t edge_bits) {
+  const int n = m.retained;
+  hipStream_t s = m.s;
+  const int blocks = (int)((edge_bits + 32 * (int64_t)BITMAP_BLOCK - 1) / (32 * (int64_t)BITMAP_BLOCK));
+  const size_t words = (size_t)blocks * BITMAP_BLOCK;
+  DArray<uint32_t> bits(words, s);
+  bits.zero();
+  DArray<int> tcount(n, s), toff(n, s), sums(blocks, s), pre(words + 1, s), totals(2, s);
+  hipLaunchKernelGGL(k_mc_mark_edges, dim3(blocks_for(n, 256)), dim3(256), 0, s, m.g, (const int*)m.cells.data(), values, n,
+                     tcount.data(), bits.data());
+  KERNEL_CHECK();
+  scan_exclusive_i32(tcount.data(), toff.data(), n, totals.data(), s);
+  hipLaunchKernelGGL(k_bits_count, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), sums.data());
+  KERNEL_CHECK();
+  scan_exclusive_i32(sums.data(), sums.data(), blocks, totals.data() + 1, s);
+  hipLaunchKernelGGL(k_bits_ranks, dim3(blocks), dim3(BITMAP_THREADS), 0, s, (const uint32_t*)bits.data(), (const int*)sums.data(),
+                     pre.data());
+  KERNEL_CHECK();
+  int host[2];
+  read_bytes(host, totals.data(), sizeof(host), s);
+  const int Tn = host[0], Vn = host[1];
+  if (!Vn) return;
+  m.vertices.reset(3 * (size_t)Vn, s);
+  m.vref.reset(2 * (size_t)Vn, s);
+  m.indices.reset(3 * (size_t)Tn, s);
+  const EdgeRanks ranks{bits.data(), pre.data()};
+  DArray<int> refs(Vn, s);
+  hipLaunchKernelGGL(k_mc_clear_refs, dim3(blocks_for(Vn, 256)), dim3(256), 0, s, refs.data(), Vn);
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_mc_edge_refs, dim3(blocks_for(n, 256)), dim3(256), 0, s, m.g, (const int*)m.cells.data(), values, n, ranks,
+                     refs.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_mc_vertices, dim3(blocks_for(Vn, 256)), dim3(256), 0, s, m.g, (const int*)m.cells.data(), values,
+                     (const int*)refs.data(), (const int*)nullptr, Vn, m.vertices.data(), m.vref.data());
+  KERNEL_CHECK();
+  if (Tn) {
+    hipLaunchKernelGGL(k_mc_rank_triangles, dim3(blocks_for(n, 256)), dim3(256), 0, s, m.g, (const int*)m.cells.data(), values, n,
+                       (const int*)toff.data(), ranks, m.indices.data());
+    KERNEL_CHECK();
+  }
+  m.V = Vn;
+  m.T = Tn;
+}
+
 void mc_triangulate(McState& m, const float* values, int* V, int* T) {
   if (m.retained < 0) throw PsrError(2, "select the cells first");
   const int n = m.retained;
   hipStream_t s = m.s;
   m.V = m.T = 0;
-  if (n) {
+  // bits for three edges a node, under the bitmaps' limit (2^31 by default: 890^3 nodes)
+  const int64_t edge_bits = 3 * (int64_t)m.g.nx * m.g.ny * m.g.nz;
+  if (n && edge_bits <= 8 * dense_index_max_cells()) {
+    triangulate_ranks(m, values, edge_bits);
+  } else if (n) {
     DArray<int> ecount(n, s), eoff(n, s), tcount(n, s), toff(n, s), etotal(1, s), ttotal(1, s);
     hipLaunchKernelGGL(k_mc_cell_counts, dim3(blocks_for(n, 256)), dim3(256), 0, s, values, n, ecount.data(), tcount.data());
     KERNEL_CHECK();

@@ -17,6 +17,7 @@ EXPORTED = (
     "psr_mesh_case_table", "psr_mesh_free", "psr_tree_metadata", "psr_tree_metadata_levels", "psr_tree_metadata_level",
     "psr_tree_metadata_copy", "psr_tree_metadata_free", "psr_field_level_offsets", "psr_isovalue",
     "psr_isovalue_noalloc", "psr_field_words", "psr_field_evaluate_words",
+    "psr_mesh_field_values", "psr_mesh_field_corners",
 )
 
 
@@ -104,6 +105,8 @@ def load():
     lib.psr_mesh_slab_nodes.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, i64p]
     lib.psr_mesh_slab_points.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, vp]
     lib.psr_mesh_slab_values.argtypes = [vp, ctypes.c_int32, ctypes.c_int32, vp]
+    lib.psr_mesh_field_values.argtypes = [vp, vp, vp, ctypes.c_int32]
+    lib.psr_mesh_field_corners.argtypes = [vp, vp, vp, vp]
     lib.psr_mesh_select.argtypes = [vp, i64p, i32p]
     lib.psr_mesh_corner_points.argtypes = [vp, vp]
     lib.psr_mesh_triangulate.argtypes = [vp, vp, i64p, i64p]
@@ -112,7 +115,7 @@ def load():
     lib.psr_mesh_case_table.argtypes = [vp, vp]
     for name in ("psr_mesh_begin", "psr_mesh_slab_nodes", "psr_mesh_slab_points", "psr_mesh_slab_values", "psr_mesh_select",
                  "psr_mesh_corner_points", "psr_mesh_triangulate", "psr_mesh_copy", "psr_mesh_vertex_vjp",
-                 "psr_mesh_case_table"):
+                 "psr_mesh_case_table", "psr_mesh_field_values", "psr_mesh_field_corners"):
         getattr(lib, name).restype = c_int
     lib.psr_tree_metadata.argtypes = [vp, vp, ctypes.POINTER(vp)]
     lib.psr_tree_metadata_levels.argtypes = [vp, i32p]

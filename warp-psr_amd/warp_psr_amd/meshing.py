@@ -110,6 +110,24 @@ def _vertex_function():
     return MeshVertices
 
 
+class _FieldValues:
+    """``field(points) - iso`` of a LevelField, untracked.  Over a reconstruction's own field (``result`` set) the
+    extraction asks the library for the values at the grid nodes (psr_mesh_field_values, psr_mesh_field_corners: the same
+    numbers without points, gradients and validity in memory); over a caller's tensors it is called like any callback."""
+
+    def __init__(self, level_field, iso):
+        self.level_field, self.iso = level_field, iso
+        self.result = level_field._result
+
+    def __call__(self, points):
+        values, _, _ = self.level_field.evaluate(points)
+        return values - self.iso
+
+
+def _own_values(callback):
+    return isinstance(callback, _FieldValues) and callback.result is not None
+
+
 def _check_values(values, points, device):
     torch = _torch()
     if (not isinstance(values, torch.Tensor) or values.dtype != torch.float32 or values.ndim != 1
@@ -165,8 +183,15 @@ def extract_isosurface(field, *, resolution, bounds, backend="sparse", device=No
         slab = nx - 1 if backend != "sparse" else slab_size
         tracked = False
         peak = 0
+        classify = field if classification_field is None else classification_field
+        if _own_values(classify):
+            _lib.check(lib.psr_mesh_field_values(mesh._handle, classify.result._handle, classify.iso.data_ptr(), min(slab, nx - 1)))
         for start in range(0, nx - 1, slab):
             width = min(slab, nx - 1 - start)
+            if _own_values(classify):
+                samples += (width + 1) * shape[1] * shape[2]
+                peak = max(peak, (width + 1) * shape[1] * shape[2])
+                continue
             nodes = ctypes.c_int64()
             _lib.check(lib.psr_mesh_slab_nodes(mesh._handle, start, width, ctypes.byref(nodes)))
             points = torch.empty((nodes.value, 3), dtype=torch.float32, device=device)
@@ -184,9 +209,15 @@ def extract_isosurface(field, *, resolution, bounds, backend="sparse", device=No
         metadata.update(retained_cells=count, slab_size=slab, selection_bytes=((math.prod(n - 1 for n in shape) + 31) // 32) * 12,
                         peak_slab_nodes=peak)
         if count:
-            corners = torch.empty((8 * count, 3), dtype=torch.float32, device=device)
-            _lib.check(lib.psr_mesh_corner_points(mesh._handle, corners.data_ptr()))
-            corner_values = sample(corners)
+            if _own_values(field):
+                corner_values = torch.empty(8 * count, dtype=torch.float32, device=device)
+                _lib.check(lib.psr_mesh_field_corners(mesh._handle, field.result._handle, field.iso.data_ptr(),
+                                                      corner_values.data_ptr()))
+                samples += 8 * count
+            else:
+                corners = torch.empty((8 * count, 3), dtype=torch.float32, device=device)
+                _lib.check(lib.psr_mesh_corner_points(mesh._handle, corners.data_ptr()))
+                corner_values = sample(corners)
             V, T = ctypes.c_int64(), ctypes.c_int64()
             _lib.check(lib.psr_mesh_triangulate(mesh._handle, corner_values.detach().data_ptr(), ctypes.byref(V),
                                                 ctypes.byref(T)))
@@ -248,9 +279,7 @@ def extract_mesh(reconstruction, *, resolution, bounds, iso_value=None, differen
             raise ValueError("iso_value must be finite")
         iso = torch.full((1,), float(iso_value), dtype=torch.float32, device=device)
 
-    def untracked(points):
-        values, _, _ = level_field.evaluate(points)
-        return values - iso.detach()
+    untracked = _FieldValues(level_field, iso.detach())
 
     if full_backward:
         def sample(points):
