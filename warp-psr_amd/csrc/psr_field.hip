@@ -71,6 +71,25 @@ __global__ void k_field_words(const int64_t* __restrict__ keys, int64_t n, int w
   if (i < n) field_word(keys, n, word_depth, words, i);
 }
 
+template <class V> struct LevelArrays {
+  const V* a[MAX_LEVELS];
+};
+
+// The levels' keys one after another, and the levels' offsets in them.
+__global__ void __launch_bounds__(LEVEL_BLOCK) k_concat_keys(LevelBlocks lb, LevelArrays<int64_t> in, int64_t* __restrict__ keys,
+                                                             int* __restrict__ offsets) {
+  if (blockIdx.x == 0 && (int)threadIdx.x <= lb.levels) offsets[threadIdx.x] = lb.first[threadIdx.x];
+  const int d = lb.level_of((int)blockIdx.x), i = lb.row_of((int)blockIdx.x, d, (int)threadIdx.x);
+  if (i >= 0) keys[lb.first[d] + i] = in.a[d][i];
+}
+
+// The levels' values one after another; a level without an array holds zeros.
+template <class T>
+__global__ void __launch_bounds__(LEVEL_BLOCK) k_concat_values(LevelBlocks lb, LevelArrays<T> in, T* __restrict__ out) {
+  const int d = lb.level_of((int)blockIdx.x), i = lb.row_of((int)blockIdx.x, d, (int)threadIdx.x);
+  if (i >= 0) out[lb.first[d] + i] = in.a[d] ? in.a[d][i] : T(0);
+}
+
 // One level's eight trilinear corners of a cube point: for each of the four z
 // pairs, the index of the first node present (0 if none), which
 // of the two are present (two bits each, the lower node's first) and which
@@ -623,7 +642,7 @@ void evaluate_field(const Result<T>& r, const T* queries, int64_t m, const T* li
 
 // Deepest level with node words: the lookup-table limits' dense one (depth 9
 // by default; word_base is defined up to there), at most the field's depth.
-static int field_word_depth(int depth) {
+int node_word_depth(int depth) {
   const int64_t cells = dense_index_max_cells();
   int d = -1;
   for (int e = 0; e <= imin(depth, 9); ++e) {
@@ -635,7 +654,7 @@ static int field_word_depth(int depth) {
 }
 
 int64_t level_field_words(int64_t count, int depth) {
-  return count <= INT32_MAX && depth >= 0 && field_word_depth(depth) == depth ? (int64_t)word_base(depth + 1) : 0;
+  return count <= INT32_MAX && depth >= 0 && node_word_depth(depth) == depth ? (int64_t)word_base(depth + 1) : 0;
 }
 
 void build_level_field_words(const int64_t* keys, int64_t count, int depth, NodeWord* words, int* sorted, hipStream_t s) {
@@ -666,43 +685,51 @@ template void evaluate_level_field<float>(const PsrField&, const NodeWord*, cons
 template void evaluate_level_field<double>(const PsrField&, const NodeWord*, const int*, const double*, int64_t, double*, double*,
                                            int*, hipStream_t);
 
+void build_node_words(const int64_t* keys, int64_t n, int word_depth, DArray<NodeWord>& words, hipStream_t s) {
+  if (word_depth < 0) return words.free();
+  words.reset(word_base(word_depth + 1), s);
+  words.zero();
+  if (!n) return;
+  hipLaunchKernelGGL(k_field_words, dim3(blocks_for(n, 256)), dim3(256), 0, s, keys, n, word_depth, words.data());
+  KERNEL_CHECK();
+}
+
+template <class T> void index_field(Result<T>& r) {
+  hipStream_t s = r.s;
+  const int D = r.prm.depth;
+  const LevelBlocks lb = level_blocks(r);
+  r.level_offsets.assign(lb.first, lb.first + D + 2);
+  const int64_t K = r.level_offsets[D + 1];
+  r.keys.reset(K, s);
+  r.offsets_dev.reset(D + 2, s);
+  LevelArrays<int64_t> in;
+  for (int d = 0; d <= D; ++d) in.a[d] = r.levels[d].basis_keys.data();
+  hipLaunchKernelGGL(k_concat_keys, dim3((unsigned)imax(lb.blocks(), 1)), dim3(LEVEL_BLOCK), 0, s, lb, in, r.keys.data(),
+                     r.offsets_dev.data());
+  KERNEL_CHECK();
+  r.word_depth = K ? node_word_depth(D) : -1;
+  build_node_words(r.keys.data(), K, r.word_depth, r.node_words, s);
+}
+
 template <class T> void stage_field(Result<T>& r) {
   hipStream_t s = r.s;
   const int D = r.prm.depth;
   r.join_average();
   read_bytes(r.normal_average_host, r.normal_average.data(), sizeof(T) * 3, s);
   r.average_contrib.free();
-  r.level_offsets.assign(D + 2, 0);
-  for (int d = 0; d <= D; ++d) r.level_offsets[d + 1] = r.level_offsets[d] + r.levels[d].basis_count;
   const int64_t K = r.level_offsets[D + 1];
-  r.keys.reset(K, s);
   r.coefficients.reset(K + 1, s);  // one value more: corner_values loads pairs
   r.coefficients.shrink(K);
-  for (int d = 0; d <= D; ++d) {
-    const LevelState<T>& L = r.levels[d];
-    const int64_t o = r.level_offsets[d];
-    if (!L.basis_count) continue;
-    HIP_CHECK(hipMemcpyAsync(r.keys.data() + o, L.basis_keys.data(), sizeof(int64_t) * L.basis_count, hipMemcpyDeviceToDevice, s));
-    if (L.correction.size())
-      HIP_CHECK(hipMemcpyAsync(r.coefficients.data() + o, L.correction.data(), sizeof(T) * L.basis_count, hipMemcpyDeviceToDevice, s));
-    else
-      HIP_CHECK(hipMemsetAsync(r.coefficients.data() + o, 0, sizeof(T) * L.basis_count, s));
-  }
-  r.offsets_dev.reset(D + 2, s);
-  HIP_CHECK(hipMemcpyAsync(r.offsets_dev.data(), r.level_offsets.data(), sizeof(int) * (D + 2), hipMemcpyHostToDevice, s));
-  // lookup tables: node words for the levels within the dense limit, column
-  // tables where deeper levels remain, else searches of the keys
-  const bool tables = D <= field_table_max_depth() && K;
-  r.word_depth = tables ? field_word_depth(D) : -1;
-  if (r.word_depth >= 0) {
-    r.node_words.reset(word_base(r.word_depth + 1), s);
-    r.node_words.zero();
-    hipLaunchKernelGGL(k_field_words, dim3(blocks_for(K, 256)), dim3(256), 0, s, (const int64_t*)r.keys.data(), K, r.word_depth,
-                       r.node_words.data());
+  const LevelBlocks lb = level_blocks(r);
+  if (K) {
+    LevelArrays<T> in;
+    for (int d = 0; d <= D; ++d) in.a[d] = r.levels[d].correction.data();
+    hipLaunchKernelGGL(k_concat_values<T>, dim3((unsigned)lb.blocks()), dim3(LEVEL_BLOCK), 0, s, lb, in, r.coefficients.data());
     KERNEL_CHECK();
-  } else {
-    r.node_words.free();
   }
+  // node words are there for the levels within the dense limit (index_field):
+  // column tables where deeper levels remain, else searches of the keys
+  const bool tables = D <= field_table_max_depth() && K;
   if (tables && r.word_depth < D) {
     const size_t cells = (size_t)column_base(D + 1);
     r.column_start.reset(cells, s);
@@ -746,6 +773,8 @@ template <class T> void stage_field(Result<T>& r) {
   reference_inverse(r.cube_to_model, r.model_to_cube);
 }
 
+template void index_field<float>(Result<float>&);
+template void index_field<double>(Result<double>&);
 template void stage_field<float>(Result<float>&);
 template void stage_field<double>(Result<double>&);
 template void evaluate_field<float>(const Result<float>&, const float*, int64_t, const float*, const float*, float*, float*, int*,

@@ -86,6 +86,104 @@ __device__ __forceinline__ void level_run(const FieldIndex& f, int d, int x, int
     if (k < len && out[k] >= 0) out[k] += lo;
 }
 
+// Nodes z0 .. z0 + LEN - 1 (LEN <= 6) of one column: mask has bit k for a
+// present node z0 + k, base is the index of the lowest present one.  A column's
+// nodes are consecutive in the keys, so node z0 + k has index
+// base + popcount(mask below k).
+struct NodeSpan {
+  int base;
+  unsigned mask;
+  __device__ __forceinline__ int at(int k) const { return (mask >> k) & 1u ? base + __popc(mask & ((1u << k) - 1u)) : -1; }
+};
+
+// x, y and z0 in [0, 2^d]
+template <int LEN> __device__ __forceinline__ NodeSpan node_span(const NodeWord* __restrict__ words, int d, int x, int y, int z0) {
+  const int wc = word_columns(d), at = imin(word_of(z0), wc - 1), b = z0 - 31 * at;
+  const NodeWord w = words[word_at(d, x, y, at)];
+  unsigned bits = w.bits >> b;
+  int base = w.first + __popc(w.bits & ((1u << b) - 1u));
+  if (b + LEN > 32 && at + 1 < wc) {
+    const NodeWord v = words[word_at(d, x, y, at + 1)];
+    if (!bits) base = v.first;  // the shared node is absent, so v's first node is the next one
+    bits |= v.bits << (31 - b);
+  }
+  return NodeSpan{base, bits & ((1u << LEN) - 1u)};
+}
+
+// One level's sorted keys with their lookup: node words (whose indices count
+// from `first` keys earlier), else an (x, y) column table, else searches.
+struct NodeIndex {
+  const int64_t* keys = nullptr;
+  int64_t count = 0;
+  ColumnTable columns;
+  const NodeWord* words = nullptr;
+  int first = 0;
+};
+
+// Indices within the level of keys (d, x, y, z0 + k), k < LEN; x, y in any
+// range, z0 in [0, 2^d].
+template <int LEN> __device__ __forceinline__ NodeSpan find_span(const NodeIndex& f, int d, int x, int y, int z0) {
+  const int n = 1 << d;
+  const bool in = x >= 0 && y >= 0 && x <= n && y <= n;
+  if (f.words) {
+    // a load at a clamped address, so that several columns' loads go out together
+    NodeSpan s = node_span<LEN>(f.words, d, imin(imax(x, 0), n), imin(imax(y, 0), n), z0);
+    s.base -= f.first;
+    if (!in) s.mask = 0;
+    return s;
+  }
+  NodeSpan s{0, 0u};
+  if (!in) return s;
+  int64_t found[LEN];
+  find_run_table<LEN>(f.keys, f.count, f.columns, d, x, y, z0, LEN, found);
+#pragma unroll
+  for (int k = LEN - 1; k >= 0; --k)
+    if (found[k] >= 0) {
+      s.base = (int)found[k];
+      s.mask |= 1u << k;
+    }
+  return s;
+}
+
+// Deepest level with node words of keys up to `depth`: the lookup-table limits'
+// dense one (depth 9 by default), -1 for none.
+int node_word_depth(int depth);
+// Node words of levels 0..word_depth of n concatenated sorted keys.
+void build_node_words(const int64_t* keys, int64_t n, int word_depth, DArray<NodeWord>& words, hipStream_t s);
+
+// Block-aligned ranges of the levels' rows: every block of a launch over all
+// levels' rows belongs to one level, found from its index alone.
+constexpr int MAX_LEVELS = 16;  // keys hold 16 bits an axis
+constexpr int LEVEL_BLOCK = 256;
+struct LevelBlocks {
+  int levels = 0;
+  int block[MAX_LEVELS + 1];  // first block of each level
+  int rows[MAX_LEVELS], first[MAX_LEVELS + 1];
+  // level of a block, and its thread's row (-1 beyond the level's rows)
+  __device__ __forceinline__ int level_of(int b) const {
+    int d = 0;
+    while (d + 1 < levels && b >= block[d + 1]) ++d;
+    return d;
+  }
+  __device__ __forceinline__ int row_of(int b, int d, int tid) const {
+    const int i = (b - block[d]) * LEVEL_BLOCK + tid;
+    return i < rows[d] ? i : -1;
+  }
+  int blocks() const { return block[levels]; }
+};
+template <class T> inline LevelBlocks level_blocks(const Result<T>& r) {
+  LevelBlocks lb;
+  lb.levels = r.prm.depth + 1;
+  if (lb.levels > MAX_LEVELS) throw PsrError(1, "too many levels");
+  lb.block[0] = lb.first[0] = 0;
+  for (int d = 0; d < lb.levels; ++d) {
+    lb.rows[d] = r.levels[d].basis_count;
+    lb.block[d + 1] = lb.block[d] + (lb.rows[d] + LEVEL_BLOCK - 1) / LEVEL_BLOCK;
+    lb.first[d + 1] = lb.first[d] + lb.rows[d];
+  }
+  return lb;
+}
+
 template <class T> inline FieldIndex field_index(const Result<T>& r) {
   FieldIndex f;
   f.words = r.node_words.data();

@@ -37,9 +37,7 @@ template <class V> struct Stencil {
 template <class T> struct LevelState {
   DArray<int64_t> tree_keys, basis_keys;
   int basis_count = 0;
-  ColumnIndex columns;  // (x, y) runs of basis_keys
-  DArray<int> dense;    // z-major dense index of basis_keys during the solve stage
-  int dense_dim = 0;
+  ColumnIndex columns;  // (x, y) runs of basis_keys, for levels without node words
   // restriction gathers to this level from level d+1: 27 fine indices per row
   DArray<int> restriction;
   // aggregates (density.py:228-240): keys and (sum x, sum y, sum z, count)
@@ -117,7 +115,7 @@ template <class T> struct Result {
   DArray<int> offsets_dev;         // the same on the device
   // node words of levels 0..word_depth of keys, level after level (word_at),
   // ceil(2^d / 31) for each of the (2^d + 1)^2 columns: 42 MB at depth 9;
-  // deeper levels have none (see field_word_depth)
+  // deeper levels have none (see node_word_depth)
   DArray<NodeWord> node_words;
   int word_depth = -1;
   // (x, y) column runs of every level of keys (absolute indices), laid out
@@ -220,6 +218,9 @@ template <class T> void compute_isovalue(const T* v, const T* w, int64_t G, T* o
 constexpr int64_t ISOVALUE_NOALLOC_MAX = (int64_t)1 << 26;
 constexpr int64_t ISOVALUE_NOALLOC_PARTIALS = ISOVALUE_NOALLOC_MAX / 1024;
 template <class T> void isovalue_noalloc(const T* v, const T* w, int64_t G, T* out, hipStream_t s);
+// The levels' keys concatenated and their node words, once the tree is built:
+// the solve and the field look nodes up through them.
+template <class T> void index_field(Result<T>& r);
 template <class T> void stage_field(Result<T>& r);
 template <class T>
 void evaluate_field(const Result<T>& r, const T* queries, int64_t m, const T* linear, const T* translation, T* values,

@@ -9,6 +9,7 @@
 // Gauss-Seidel runs on a copy of the operator gathered into schedule order
 // (rows of one colour/slice group contiguous, slot-major), so the loads of one
 // phase are coalesced; x stays in canonical order for the neighbour gathers.
+#include "psr_field_index.h"
 #include "psr_result.h"
 
 #include <algorithm>
@@ -122,68 +123,54 @@ __global__ void k_normal_table(int test_depth, int normal_depth, int first, int 
 }
 
 // ---------------------------------------------------------------- stiffness (stiffness.py:38-109)
-// z-major dense index of one level's basis keys: dense[(z*dim + x)*dim + y] =
-// key index or -1.  Rows taken in sliced schedule order share a z slice, so
-// their neighbour reads fall in a few contiguous (x, y) lines.
-__global__ void k_dense_fill(const int64_t* __restrict__ keys, int n, int dim, int* __restrict__ dense) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t k = keys[i];
-  dense[((int64_t)key_z(k) * dim + key_x(k)) * dim + key_y(k)] = i;
-}
-
 // One row's 27 stiffness slots: slot k = kx*9 + ky*3 + kz holds the trial
 // function (p + (kx-1, ky-1, kz-1)), p the row's coordinates at trial_depth;
 // emit(k, index, value) receives the trial function's index (-1 if absent)
-// and the entry (0 if absent), slots in order.
+// and the entry (0 if absent), slots in order.  The nine columns' words are
+// loaded before any is used; a column's three nodes then cost one population
+// count, because they are consecutive in the keys.  (A dense index of 540 MB
+// at depth 9 took 27 loads: k_level_operator over all levels of 480,000
+// aggregates 3.6 -> 2.4 ms, and 0.3 ms to clear and fill it.)
 template <class Emit>
-__device__ __forceinline__ void stiffness_row(int64_t key, const int64_t* __restrict__ cols, int64_t C, ColumnTable ct,
-                                              const int* __restrict__ dense, int dense_dim, int depth, int trial_depth,
+__device__ __forceinline__ void stiffness_row(int64_t key, const NodeIndex& cols, int depth, int trial_depth,
                                               const D2* __restrict__ table, Emit&& emit) {
   const int cx = key_x(key), cy = key_y(key), cz = key_z(key);
   const int shift = depth - trial_depth;
   const int px = cx >> shift, py = cy >> shift, pz = cz >> shift;
-  const int lim = 1 << trial_depth;
-  const int zlo = imax(pz - 1, 0), zhi = imin(pz + 1, lim);
+  NodeSpan span[9];
 #pragma unroll
-  for (int kx = 0; kx < 3; ++kx) {
-    const int qx = px + kx - 1;
+  for (int c = 0; c < 9; ++c) {
+    span[c] = find_span<3>(cols, trial_depth, px + c / 3 - 1, py + c % 3 - 1, imax(pz - 1, 0));
+    if (pz == 0) span[c].mask = (span[c].mask << 1) & 7u;  // node z = -1 is absent
+  }
+  D2 hx[3], hy[3], hz[3];
 #pragma unroll
-    for (int ky = 0; ky < 3; ++ky) {
-      const int qy = py + ky - 1;
-      int64_t found[3] = {-1, -1, -1};
-      if (qx >= 0 && qx <= lim && qy >= 0 && qy <= lim && zlo <= zhi) {
-        if (dense) {
-          for (int z = zlo; z <= zhi; ++z) found[z - zlo] = dense[((int64_t)z * dense_dim + qx) * dense_dim + qy];
-        } else {
-          find_run_table<3>(cols, C, ct, trial_depth, qx, qy, zlo, zhi - zlo + 1, found);
-        }
-      }
+  for (int k = 0; k < 3; ++k) {
+    hx[k] = table[cx * 3 + k];
+    hy[k] = table[cy * 3 + k];
+    hz[k] = table[cz * 3 + k];
+  }
 #pragma unroll
-      for (int kz = 0; kz < 3; ++kz) {
-        const int qz = pz + kz - 1;
-        const int k = kx * 9 + ky * 3 + kz;
-        const int64_t index = (qz >= zlo && qz <= zhi) ? found[qz - zlo] : -1;
-        double v = 0.0;
-        if (index >= 0) {
-          const D2 x = table[cx * 3 + kx], y = table[cy * 3 + ky], z = table[cz * 3 + kz];
-          v = x.v1 * y.v0 * z.v0 + x.v0 * y.v1 * z.v0 + x.v0 * y.v0 * z.v1;
-        }
-        emit(k, index, v);
-      }
+  for (int c = 0; c < 9; ++c) {
+    const D2 x = hx[c / 3], y = hy[c % 3];
+#pragma unroll
+    for (int kz = 0; kz < 3; ++kz) {
+      const int index = span[c].at(kz);
+      const D2 z = hz[kz];
+      const double v = x.v1 * y.v0 * z.v0 + x.v0 * y.v1 * z.v0 + x.v0 * y.v0 * z.v1;
+      emit(c * 3 + kz, index, index >= 0 ? v : 0.0);
     }
   }
 }
 
-__global__ void k_stiffness(const int64_t* __restrict__ rows, int R, const int* __restrict__ row_order,
-                            const int64_t* __restrict__ cols, int64_t C, ColumnTable ct, const int* __restrict__ dense,
-                            int dense_dim, int depth, int trial_depth, const D2* __restrict__ table, int* __restrict__ out_cols,
+__global__ void k_stiffness(const int64_t* __restrict__ rows, int R, const int* __restrict__ row_order, NodeIndex cols, int depth,
+                            int trial_depth, const D2* __restrict__ table, int* __restrict__ out_cols,
                             double* __restrict__ out_vals) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x;  // output position
   if (j >= R) return;
   const int i = row_order ? row_order[j] : j;
-  stiffness_row(rows[i], cols, C, ct, dense, dense_dim, depth, trial_depth, table, [&](int k, int64_t index, double v) {
-    out_cols[(int64_t)k * R + j] = (int)index;
+  stiffness_row(rows[i], cols, depth, trial_depth, table, [&](int k, int index, double v) {
+    out_cols[(int64_t)k * R + j] = index;
     out_vals[(int64_t)k * R + j] = v;
   });
 }
@@ -404,8 +391,7 @@ template <class T, class V> union RowRecordWords {
 // records (the tiled relaxation's input) each row's record.
 template <class T, class V, bool SCREEN>
 __global__ void __launch_bounds__(256) k_level_operator(const int64_t* __restrict__ rows, int R, const int* __restrict__ row_order,
-                                                        const int64_t* __restrict__ cols, int64_t C, ColumnTable ct,
-                                                        const int* __restrict__ dense, int dense_dim, int depth, int trial_depth,
+                                                        NodeIndex cols, int depth, int trial_depth,
                                                         const D2* __restrict__ table, PointBins<T> pb, double* __restrict__ load,
                                                         int* __restrict__ out_cols, V* __restrict__ out_vals,
                                                         const int* __restrict__ inv, int* __restrict__ sched_cols,
@@ -424,10 +410,10 @@ __global__ void __launch_bounds__(256) k_level_operator(const int64_t* __restric
     }
     T diagonal = T(0);
     RowRecordWords<T, V> rec;
-    stiffness_row(key, cols, C, ct, dense, dense_dim, depth, trial_depth, table, [&](int k, int64_t index, double v) {
+    stiffness_row(key, cols, depth, trial_depth, table, [&](int k, int index, double v) {
       const bool found = index >= 0;
       const V stored = V(found && SCREEN ? v + acc[k] : v);
-      out_cols[(int64_t)k * R + j] = (int)index;
+      out_cols[(int64_t)k * R + j] = index;
       out_vals[(int64_t)k * R + j] = stored;
       rec.r.v[k] = stored;
       if (inv_diag) {
@@ -472,53 +458,61 @@ __global__ void k_rhs(const double* __restrict__ load, const double* __restrict_
 }
 
 // ---------------------------------------------------------------- prolongation (transfer_stencils.py:15-66)
-template <class T>
-__global__ void k_prolongation(const int64_t* __restrict__ fine, int R, const int64_t* __restrict__ coarse, int64_t C, ColumnTable ct, int depth,
-                               int* __restrict__ cols, T* __restrict__ vals) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= R) return;
-  const int64_t key = fine[i];
-  const int f[3] = {key_x(key), key_y(key), key_z(key)};
-  T h[3][2];
-  for (int a = 0; a < 3; ++a)
-    for (int o = 0; o < 2; ++o) h[a][o] = T(1) - fabs(T(f[a]) * T(0.5) - T(f[a] / 2 + o));
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) {
-      const T wz0 = h[0][a] * h[1][b] * h[2][0], wz1 = h[0][a] * h[1][b] * h[2][1];
-      int64_t found[2] = {-1, -1};
-      if (wz0 > T(0) || wz1 > T(0)) find_run_table<2>(coarse, C, ct, depth - 1, f[0] / 2 + a, f[1] / 2 + b, f[2] / 2, 2, found);
-      for (int c = 0; c < 2; ++c) {
-        const int k = a * 4 + b * 2 + c;
-        const T weight = c ? wz1 : wz0;
-        const int64_t column = weight > T(0) ? found[c] : -1;
-        cols[(int64_t)k * R + i] = (int)column;
-        vals[(int64_t)k * R + i] = column >= 0 ? weight : T(0);
-      }
-    }
-}
-
+// Every level's prolongation rows and restriction gathers in one launch over
+// all levels' rows.
+//
+// Row i of P_d: the eight coarse corners with their trilinear weights.
+//
 // Restriction P^T as a gather: coarse row r takes the fine nodes 2r+o,
 // o in {-1,0,1}^3 (ascending fine index = lexicographic o), weight 1/2 per
 // nonzero axis offset; exactly the rows of the transposed prolongation.
-__global__ void k_restriction(const int64_t* __restrict__ coarse, int C, const int64_t* __restrict__ fine, int64_t F,
-                              ColumnTable ct, int fine_depth, int* __restrict__ cols) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= C) return;
-  const int64_t key = coarse[r];
-  const int x = 2 * key_x(key), y = 2 * key_y(key), z = 2 * key_z(key);
-  const int lim = 1 << fine_depth;
-  const int zlo = imax(z - 1, 0), zhi = imin(z + 1, lim);
-  for (int kx = 0; kx < 3; ++kx)
-    for (int ky = 0; ky < 3; ++ky) {
-      const int fx = x + kx - 1, fy = y + ky - 1;
-      int64_t found[3] = {-1, -1, -1};
-      if (fx >= 0 && fx <= lim && fy >= 0 && fy <= lim && zlo <= zhi)
-        find_run_table<3>(fine, F, ct, fine_depth, fx, fy, zlo, zhi - zlo + 1, found);
-      for (int kz = 0; kz < 3; ++kz) {
-        const int fz = z + kz - 1;
-        cols[(int64_t)(kx * 9 + ky * 3 + kz) * C + r] = (fz >= zlo && fz <= zhi) ? (int)found[fz - zlo] : -1;
-      }
+//
+// What it writes bounds it (64 or 96 bytes of P and 108 of restriction a row).
+// Two launches a level through column tables and a search of each column's
+// keys took 843 us at 480,000 aggregates and depth 9 in float64, and 178 us
+// for the tables; this one 676 us, the base loads running beside it.
+template <class T> struct TransferLevels {
+  NodeIndex nodes[MAX_LEVELS];
+  int* pcols[MAX_LEVELS];
+  T* pvals[MAX_LEVELS];
+  int* restr[MAX_LEVELS];  // of the level's rows from the next level
+};
+
+template <class T> __global__ void __launch_bounds__(LEVEL_BLOCK) k_transfers(LevelBlocks lb, TransferLevels<T> tl) {
+  const int d = lb.level_of((int)blockIdx.x), i = lb.row_of((int)blockIdx.x, d, (int)threadIdx.x);
+  if (i < 0) return;
+  const int64_t R = lb.rows[d];
+  const int64_t key = tl.nodes[d].keys[i];
+  const int f[3] = {key_x(key), key_y(key), key_z(key)};
+  if (d > 0) {
+    int* cols = tl.pcols[d];
+    T* vals = tl.pvals[d];
+    NodeSpan span[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) span[k] = find_span<2>(tl.nodes[d - 1], d - 1, f[0] / 2 + k / 2, f[1] / 2 + k % 2, f[2] / 2);
+    T h[3][2];
+    for (int a = 0; a < 3; ++a)
+      for (int o = 0; o < 2; ++o) h[a][o] = T(1) - fabs(T(f[a]) * T(0.5) - T(f[a] / 2 + o));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const T weight = h[0][k / 4] * h[1][k / 2 % 2] * h[2][k % 2];
+      const int column = weight > T(0) ? span[k / 2].at(k % 2) : -1;
+      cols[k * R + i] = column;
+      vals[k * R + i] = column >= 0 ? weight : T(0);
     }
+  }
+  if (d + 1 < lb.levels) {
+    int* cols = tl.restr[d];
+    const int z0 = imax(2 * f[2] - 1, 0);
+    NodeSpan span[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) {
+      span[c] = find_span<3>(tl.nodes[d + 1], d + 1, 2 * f[0] + c / 3 - 1, 2 * f[1] + c % 3 - 1, z0);
+      if (f[2] == 0) span[c].mask = (span[c].mask << 1) & 7u;
+    }
+#pragma unroll
+    for (int k = 0; k < 27; ++k) cols[k * R + i] = span[k / 3].at(k % 3);
+  }
 }
 
 PSR_HD double restriction_weight(int k) {
@@ -605,112 +599,56 @@ __global__ void k_spmv(const int* __restrict__ cols, const V* __restrict__ vals,
 }
 
 // ---------------------------------------------------------------- normal loads (normal_stencils.py, normal_loads.py)
-// Dense index of a key set: zmajor ? (z*dim + x)*dim + y : (x*dim + y)*dim + z
-struct DenseIndex {
-  const int* idx = nullptr;
-  int dim = 0;
-  int zmajor = 0;
-};
-
-__global__ void k_dense_fill_xyz(const int64_t* __restrict__ keys, int64_t n, int dim, int* __restrict__ dense) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const int64_t k = keys[i];
-  dense[((int64_t)key_x(k) * dim + key_y(k)) * dim + key_z(k)] = (int)i;
-}
-
-template <class V>
-__global__ void k_normal_load(const int64_t* __restrict__ keys, int R, const int64_t* __restrict__ nkeys, int64_t ncount, ColumnTable ct,
-                              DenseIndex dn, const V* __restrict__ nvals, int nstride, int test_depth, int normal_depth, int first,
-                              int width, const D2* __restrict__ table, double* __restrict__ out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= R) return;
-  const int64_t key = keys[i];
-  const int c0 = key_x(key), c1 = key_y(key), c2 = key_z(key);
-  const int e0 = normal_center(c0, test_depth, normal_depth), e1 = normal_center(c1, test_depth, normal_depth),
-            e2 = normal_center(c2, test_depth, normal_depth);
-  const int lim = 1 << normal_depth;
-  const int zlo = imax(e2 + first, 0), zhi = imin(e2 + first + width - 1, lim - 1);
-  double value = 0.0;
-  for (int x = 0; x < width; ++x) {
-    const int nx = e0 + x + first;
-    if (nx < 0 || nx >= lim) continue;
-    for (int y = 0; y < width; ++y) {
-      const int ny = e1 + y + first;
-      if (ny < 0 || ny >= lim || zlo > zhi) continue;
-      int64_t found[6];
-      if (dn.idx) {
-        for (int z = zlo; z <= zhi; ++z)
-          found[z - zlo] = dn.zmajor ? dn.idx[((int64_t)z * dn.dim + nx) * dn.dim + ny] : dn.idx[((int64_t)nx * dn.dim + ny) * dn.dim + z];
-      } else {
-        find_run_table<6>(nkeys, ncount, ct, normal_depth, nx, ny, zlo, zhi - zlo + 1, found);
-      }
-      for (int z = 0; z < width; ++z) {
-        const int nz = e2 + z + first;
-        if (nz < zlo || nz > zhi) continue;
-        const int64_t jn = found[nz - zlo];
-        if (jn < 0) continue;
-        const D2 ix = table[c0 * width + x], iy = table[c1 * width + y], iz = table[c2 * width + z];
-        const V* nv = nvals + (int64_t)nstride * jn;
-        value += double(nv[0]) * ix.v1 * iy.v0 * iz.v0;
-        value += double(nv[1]) * ix.v0 * iy.v1 * iz.v0;
-        value += double(nv[2]) * ix.v0 * iy.v0 * iz.v1;
-      }
-    }
-  }
-  out[i] = value;
-}
-
-// k_normal_load over a dense record index with each (x, y) column's loads
-// batched: the column's W dense entries, then all W records' values, then the
-// terms in the same (x, y, z, component) order as k_normal_load, so the sum is
-// identical.  Unconditional, clamped addresses keep the loads independent of
-// the presence tests (k_normal_load issues them one record at a time).
+// One row's load from the records of a level: the W^3 records around it, in
+// (x, y, z, component) order.  The words of an x plane's W columns go out
+// together and a column's records are consecutive, so a row waits twice a
+// plane or column; the dense index this replaces (one int a node, 540 MB at
+// depth 9, cleared for each of the two key sets) waited as often on loads that
+// missed every cache.
 template <class V, int W>
-__global__ void __launch_bounds__(128) k_normal_load_dense(const int64_t* __restrict__ keys, int R, DenseIndex dn,
-                                                           const V* __restrict__ nvals, int nstride, int test_depth,
-                                                           int normal_depth, int first, const D2* __restrict__ table,
-                                                           double* __restrict__ out) {
+__global__ void __launch_bounds__(128) k_normal_load(const int64_t* __restrict__ keys, int R, NodeIndex nodes,
+                                                     const V* __restrict__ nvals, int test_depth, int normal_depth, int first,
+                                                     const D2* __restrict__ table, double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= R) return;
   const int64_t key = keys[i];
   const int c0 = key_x(key), c1 = key_y(key), c2 = key_z(key);
   const int e0 = normal_center(c0, test_depth, normal_depth), e1 = normal_center(c1, test_depth, normal_depth),
             e2 = normal_center(c2, test_depth, normal_depth);
+  // records lie in cells 0 .. lim - 1 of an axis; the first found is offset
+  // `shift` of the row's W
   const int lim = 1 << normal_depth;
-  const int zlo = imax(e2 + first, 0), zhi = imin(e2 + first + W - 1, lim - 1);
+  const int zlo = imax(e2 + first, 0), shift = zlo - (e2 + first);
+  const int len = imax(imin(e2 + first + W - 1, lim - 1) - zlo + 1, 0);
   D2 iz[W];
 #pragma unroll
   for (int k = 0; k < W; ++k) iz[k] = table[c2 * W + k];
-  const int64_t dim = dn.dim;
   double value = 0.0;
   for (int x = 0; x < W; ++x) {
     const int nx = e0 + x + first;
     if (nx < 0 || nx >= lim) continue;
     const D2 ix = table[c0 * W + x];
+    NodeSpan span[W];
+#pragma unroll
     for (int y = 0; y < W; ++y) {
       const int ny = e1 + y + first;
-      if (ny < 0 || ny >= lim) continue;
-      const D2 iy = table[c1 * W + y];
-      int jn[W];
+      span[y] = find_span<W>(nodes, normal_depth, nx, ny, imin(zlo, lim));
+      span[y].mask = ny < 0 || ny >= lim ? 0u : (span[y].mask & ((1u << len) - 1u)) << shift;
+    }
 #pragma unroll
-      for (int z = 0; z < W; ++z) {
-        const int nz = e2 + z + first;
-        const bool in = nz >= zlo && nz <= zhi;
-        int64_t cell = dn.zmajor ? ((int64_t)nz * dim + nx) * dim + ny : ((int64_t)nx * dim + ny) * dim + nz;
-        cell = in ? cell : 0;
-        jn[z] = in ? dn.idx[cell] : -1;
-      }
+    for (int y = 0; y < W; ++y) {
+      if (!span[y].mask) continue;
+      const D2 iy = table[c1 * W + y];
       V v[W][3];
 #pragma unroll
       for (int z = 0; z < W; ++z) {
-        const int64_t j = jn[z] >= 0 ? jn[z] : 0;
+        const int64_t j = span[y].at(z);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) v[z][c] = jn[z] >= 0 ? nvals[(int64_t)nstride * j + c] : V(0);
+        for (int c = 0; c < 3; ++c) v[z][c] = j >= 0 ? nvals[3 * j + c] : V(0);
       }
 #pragma unroll
       for (int z = 0; z < W; ++z) {
-        if (jn[z] < 0) continue;
+        if (!((span[y].mask >> z) & 1u)) continue;
         value += double(v[z][0]) * ix.v1 * iy.v0 * iz[z].v0;
         value += double(v[z][1]) * ix.v0 * iy.v1 * iz[z].v0;
         value += double(v[z][2]) * ix.v0 * iy.v0 * iz[z].v1;
@@ -722,21 +660,20 @@ __global__ void __launch_bounds__(128) k_normal_load_dense(const int64_t* __rest
 
 // normal_loads.py:27-63 (prolong degree-2 coefficients with degree-1 weights, issue #35)
 template <class T>
-__global__ void k_normal_prolong(const int64_t* __restrict__ keys, int R, const int64_t* __restrict__ own_keys, int64_t own_count,
-                                 ColumnTable own_ct, const T* __restrict__ own_vals, const int64_t* __restrict__ prev_keys, int64_t prev_count, ColumnTable ct,
-                                 const T* __restrict__ prev_vals, int depth, T* __restrict__ out) {
+__global__ void k_normal_prolong(const int64_t* __restrict__ keys, int R, NodeIndex records, const T* __restrict__ own_vals,
+                                 NodeIndex prev, const T* __restrict__ prev_vals, int depth, T* __restrict__ out) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= R) return;
   const int64_t key = keys[i];
   const int c[3] = {key_x(key), key_y(key), key_z(key)};
   T v0 = T(0), v1 = T(0), v2 = T(0);
-  int64_t own;
-  find_run_table<1>(own_keys, own_count, own_ct, depth, c[0], c[1], c[2], 1, &own);
+  const int64_t own = find_span<1>(records, depth, c[0], c[1], c[2]).at(0);
   if (own >= 0) { v0 = own_vals[3 * own]; v1 = own_vals[3 * own + 1]; v2 = own_vals[3 * own + 2]; }
   if (depth > 0) {
-    int64_t idx[2][2][2];  // [x bit][y bit][z bit]
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b) find_run_table<2>(prev_keys, prev_count, ct, depth - 1, c[0] / 2 + a, c[1] / 2 + b, c[2] / 2, 2, idx[a][b]);
+    NodeSpan span[2][2];  // [x bit][y bit]
+#pragma unroll
+    for (int k = 0; k < 4; ++k) span[k / 2][k % 2] = find_span<2>(prev, depth - 1, c[0] / 2 + k / 2, c[1] / 2 + k % 2, c[2] / 2);
+#pragma unroll
     for (int corner = 0; corner < 8; ++corner) {  // x is bit 0 here (normal_loads.py:285-297)
       int p[3] = {c[0] / 2, c[1] / 2, c[2] / 2};
       T weight = T(1);
@@ -745,7 +682,7 @@ __global__ void k_normal_prolong(const int64_t* __restrict__ keys, int R, const 
         weight = weight * (T(1) - fabs(T(c[axis]) * T(0.5) - T(p[axis])));
       }
       if (weight > T(0)) {
-        const int64_t j = idx[corner & 1][(corner >> 1) & 1][(corner >> 2) & 1];
+        const int64_t j = span[corner & 1][(corner >> 1) & 1].at((corner >> 2) & 1);
         if (j >= 0) {
           v0 = v0 + prev_vals[3 * j] * weight;
           v1 = v1 + prev_vals[3 * j + 1] * weight;
@@ -1545,7 +1482,7 @@ __global__ void k_tile_entries(const uint32_t* __restrict__ skeys, const int* __
   entries[e] = make_int2(j, lx | (ly << 8) | (interior << 16));
 }
 
-// Tile tables from a level's dense z-major index, tile by tile: the
+// Tile tables from a level's node words, tile by tile: the
 // workgroup of tile t scans its (ts + 8)^2 window of its slice in window
 // order (lx-major) and files each row it finds under its categories -- the
 // computed colour (ring <= 3 - colour) and the staged values (every row of
@@ -1561,14 +1498,13 @@ struct TileCell {
 };
 
 template <bool EMIT>
-__device__ __forceinline__ TileCell tile_cell(const int* __restrict__ dense, int dim, int n, int z, int ox, int oy, int ts,
+__device__ __forceinline__ TileCell tile_cell(const NodeIndex& nodes, int depth, int z, int ox, int oy, int ts,
                                               int g, int w, int flip, const int* __restrict__ inv) {
   TileCell c{0, 0, -1, false};
   if (w >= g * g) return c;
   const int lx = w / g, ly = w - (w / g) * g;
   const int x = ox + lx, y = oy + ly;
-  if (x < 0 || y < 0 || x > n || y > n) return c;
-  const int i = dense[((int64_t)z * dim + x) * dim + y];
+  const int i = find_span<1>(nodes, depth, x, y, z).at(0);
   if (i < 0) return c;
   c.present = true;
   const int r = max(ring_of(x, ox + 4, ts), ring_of(y, oy + 4, ts));
@@ -1581,7 +1517,7 @@ __device__ __forceinline__ TileCell tile_cell(const int* __restrict__ dense, int
   return c;
 }
 
-__global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int* __restrict__ dense, int dim, int n,
+__global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(NodeIndex nodes, int depth,
                                                                         const int* __restrict__ dense_of, int nt, int ts,
                                                                         int flip, int* __restrict__ counts) {
   __shared__ int total[5];
@@ -1593,7 +1529,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int
   const int ox = tx * ts - 4, oy = ty * ts - 4, g = ts + 8;
   int cnt[5] = {0, 0, 0, 0, 0};
   for (int w = tid; w < g * g; w += TILE_SCAN_THREADS) {
-    const TileCell c = tile_cell<false>(dense, dim, n, z, ox, oy, ts, g, w, flip, nullptr);
+    const TileCell c = tile_cell<false>(nodes, depth, z, ox, oy, ts, g, w, flip, nullptr);
     if (!c.present) continue;
     if (c.cat >= 0) ++cnt[c.cat];
     ++cnt[4];
@@ -1605,7 +1541,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_count(const int
   if (tid < 5) counts[5 * (int64_t)t + tid] = total[tid];
 }
 
-__global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_emit(const int* __restrict__ dense, int dim, int n,
+__global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_emit(NodeIndex nodes, int depth,
                                                                        const int* __restrict__ dense_of, int nt, int ts,
                                                                        int flip, const int* __restrict__ inv, const int* __restrict__ offs,
                                                                        int2* __restrict__ entries) {
@@ -1620,7 +1556,7 @@ __global__ void __launch_bounds__(TILE_SCAN_THREADS) k_tile_scan_emit(const int*
   const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
   __syncthreads();
   for (int w0 = 0; w0 < g * g; w0 += TILE_SCAN_THREADS) {
-    const TileCell c = tile_cell<true>(dense, dim, n, z, ox, oy, ts, g, w0 + tid, flip, inv);
+    const TileCell c = tile_cell<true>(nodes, depth, z, ox, oy, ts, g, w0 + tid, flip, inv);
     int pre[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
@@ -2179,6 +2115,47 @@ int relax_sliced_any(const GsOperator<T, V>& op, const Schedule<T>& sc, T* x, in
   }
 }
 
+// ---------------------------------------------------------------- node lookups
+// Level d's nodes: by the run's node words, or by the level's column table.
+template <class T> static NodeIndex level_nodes(const Result<T>& r, int d) {
+  const LevelState<T>& L = r.levels[d];
+  NodeIndex f;
+  f.keys = L.basis_keys.data();
+  f.count = L.basis_count;
+  f.columns = L.columns.view();
+  f.words = d <= r.word_depth ? (const NodeWord*)r.node_words.data() : (const NodeWord*)nullptr;
+  f.first = r.level_offsets[d];
+  return f;
+}
+
+// The levels' normal records: one set of node words over all levels, column
+// tables for the levels beyond them.
+template <class T> struct RecordIndex {
+  DArray<NodeWord> words;
+  int word_depth = -1;
+  std::vector<ColumnIndex> columns;
+
+  void build(const Result<T>& r, hipStream_t s) {
+    const int D = r.prm.depth;
+    const int64_t n = r.normal_offsets[D + 1];
+    word_depth = n ? node_word_depth(D) : -1;
+    build_node_words(r.normal_keys.data(), n, word_depth, words, s);
+    columns.resize(D + 1);
+    for (int d = word_depth + 1; d <= D; ++d)
+      build_column_index(r.normal_keys.data() + r.normal_offsets[d], r.normal_offsets[d + 1] - r.normal_offsets[d], (1 << d) + 1,
+                         columns[d], s);
+  }
+  NodeIndex at(const Result<T>& r, int d) const {
+    NodeIndex f;
+    f.keys = r.normal_keys.data() + r.normal_offsets[d];
+    f.count = r.normal_offsets[d + 1] - r.normal_offsets[d];
+    f.columns = columns[d].view();
+    f.words = d <= word_depth ? (const NodeWord*)words.data() : (const NodeWord*)nullptr;
+    f.first = (int)r.normal_offsets[d];
+    return f;
+  }
+};
+
 // ---------------------------------------------------------------- tiled sliced relaxation (host)
 // The tile tables of one level (see k_relax_tiled).
 struct TileTable {
@@ -2206,12 +2183,13 @@ static int relax_tile_size(int requested, int depth) {
   return depth <= 6 ? 12 : depth <= 8 ? 16 : 18;
 }
 
-// With the level's dense z-major index (level_dense, side dim) the entries
-// come tile by tile from the index (k_tile_scan_*); without it, row by row
-// and a sort of the (tile, category) keys.  flip: see k_tile_members.
-static void build_tile_table(const int64_t* keys, const int* order, int R, int depth, int ts, const int* level_dense,
-                             int dim, TileTable& tt, hipStream_t s, int flip = 0) {
+// With the level's node words the entries come tile by tile from them
+// (k_tile_scan_*); without, row by row and a sort of the (tile, category) keys.
+// flip: see k_tile_members.
+static void build_tile_table(const NodeIndex& nodes, const int* order, int R, int depth, int ts, TileTable& tt, hipStream_t s,
+                             int flip = 0) {
   const int n = 1 << depth;
+  const int64_t* keys = nodes.keys;
   tt.ts = ts;
   tt.nt = (n + 1 + ts - 1) / ts;
   const int64_t per_slice = (int64_t)tt.nt * tt.nt;
@@ -2223,7 +2201,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
                      (const int*)nullptr, (int*)nullptr, (uint32_t*)nullptr, (int*)nullptr);
   KERNEL_CHECK();
   scan_exclusive_i32(flags.data(), compact.data(), ndense + 1, total.data(), s);
-  if (level_dense && dim == n + 1) {
+  if (nodes.words) {
     tt.tiles = read_int(total.data(), s);
     const int tiles = tt.tiles;
     DArray<int> dense_of(std::max(tiles, 1), s);
@@ -2235,7 +2213,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
     KERNEL_CHECK();
     HIP_CHECK(hipMemsetAsync(offs.data() + 5 * (size_t)tiles, 0, sizeof(int), s));
     if (tiles) {
-      hipLaunchKernelGGL(k_tile_scan_count, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, level_dense, dim, n,
+      hipLaunchKernelGGL(k_tile_scan_count, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, nodes, depth,
                          (const int*)dense_of.data(), tt.nt, ts, flip, offs.data());
       KERNEL_CHECK();
     }
@@ -2247,7 +2225,7 @@ static void build_tile_table(const int64_t* keys, const int* order, int R, int d
     HIP_CHECK(hipMemsetAsync(small.data() + n + 2, 0, 2 * sizeof(int), s));
     tt.desc.reset(TILE_DESC_INTS * (size_t)std::max(tiles, 1), s);
     if (tiles) {
-      hipLaunchKernelGGL(k_tile_scan_emit, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, level_dense, dim, n,
+      hipLaunchKernelGGL(k_tile_scan_emit, dim3(tiles), dim3(TILE_SCAN_THREADS), 0, s, nodes, depth,
                          (const int*)dense_of.data(), tt.nt, ts, flip, (const int*)inv.data(), (const int*)offs.data(),
                          tt.entries.data());
       KERNEL_CHECK();
@@ -2796,8 +2774,9 @@ void relax_colored(const GsOperator<T>& op, const Schedule<T>& sc, T* x, int ite
 }
 
 // row_order (optional, device): output position j holds row row_order[j]
-template <class T> static Stencil<double> assemble_stiffness(const LevelState<T>& rowsL, const LevelState<T>& colsL, int depth,
-                                                             int trial_depth, hipStream_t s, const int* row_order = nullptr) {
+template <class T> static Stencil<double> assemble_stiffness(const Result<T>& r, int depth, int trial_depth, hipStream_t s,
+                                                             const int* row_order = nullptr) {
+  const LevelState<T>&rowsL = r.levels[depth], &colsL = r.levels[trial_depth];
   Stencil<double> m;
   const int R = rowsL.basis_count;
   m.rows = R;
@@ -2810,9 +2789,7 @@ template <class T> static Stencil<double> assemble_stiffness(const LevelState<T>
   KERNEL_CHECK();
   if (R) {
     hipLaunchKernelGGL(k_stiffness, dim3(blocks_for(R, 256)), dim3(256), 0, s, (const int64_t*)rowsL.basis_keys.data(), R,
-                       row_order, (const int64_t*)colsL.basis_keys.data(), (int64_t)colsL.basis_count, colsL.columns.view(),
-                       colsL.dense_dim ? (const int*)colsL.dense.data() : (const int*)nullptr, colsL.dense_dim, depth, trial_depth,
-                       (const D2*)table.data(), m.cols.data(), m.vals.data());
+                       row_order, level_nodes(r, trial_depth), depth, trial_depth, (const D2*)table.data(), m.cols.data(), m.vals.data());
     KERNEL_CHECK();
   }
   return m;
@@ -2899,14 +2876,15 @@ template <class T> static Stencil<T> cast_stencil(Stencil<double>&& m, hipStream
   return out;
 }
 
-// A sliced finer level's operator (colsL = rowsL, trial_depth = depth; op and
-// present given) or cross operator (colsL one level coarser) in one pass of
+// A sliced finer level's operator (trial_depth = depth; op and present given)
+// or cross operator (trial_depth one level coarser) in one pass of
 // k_level_operator, rows in schedule order ord (inv = its inverse) or, with ord
 // null, in canonical order.
 template <class T, class V>
-static void level_operator(const LevelState<T>& rowsL, const LevelState<T>& colsL, int depth, int trial_depth,
+static void level_operator(const Result<T>& r, int depth, int trial_depth,
                            const PointSet<T>* pts, double* load, const int* ord, const int* inv, Stencil<V>& out,
                            GsOperator<T, V>* op, RowRecord<T, V>* records, unsigned long long* present, hipStream_t s) {
+  const LevelState<T>&rowsL = r.levels[depth], &colsL = r.levels[trial_depth];
   const int R = rowsL.basis_count;
   out.rows = R;
   out.cols_count = colsL.basis_count;
@@ -2923,31 +2901,29 @@ static void level_operator(const LevelState<T>& rowsL, const LevelState<T>& cols
   hipLaunchKernelGGL(k_hat_table, dim3(blocks_for((res + 1) * 3, 256)), dim3(256), 0, s, depth, trial_depth, table.data());
   KERNEL_CHECK();
   const PointBins<T> pb = pts ? point_bins(*pts) : PointBins<T>{};
-  const int* dense = colsL.dense_dim ? (const int*)colsL.dense.data() : (const int*)nullptr;
+  const NodeIndex nodes = level_nodes(r, trial_depth);
   int* sched = op && inv ? op->cols.data() : nullptr;
   T* inv_diag = op ? op->inv_diag.data() : nullptr;
   unsigned char* has_diag = op ? op->has_diag.data() : nullptr;
   if (pts)
     hipLaunchKernelGGL((k_level_operator<T, V, true>), dim3(blocks_for(R, 256)), dim3(256), 0, s,
-                       (const int64_t*)rowsL.basis_keys.data(), R, ord, (const int64_t*)colsL.basis_keys.data(),
-                       (int64_t)colsL.basis_count, colsL.columns.view(), dense, colsL.dense_dim, depth, trial_depth,
+                       (const int64_t*)rowsL.basis_keys.data(), R, ord, nodes, depth, trial_depth,
                        (const D2*)table.data(), pb, load, out.cols.data(), out.vals.data(), inv, sched, inv_diag, has_diag,
                        records, present);
   else
     hipLaunchKernelGGL((k_level_operator<T, V, false>), dim3(blocks_for(R, 256)), dim3(256), 0, s,
-                       (const int64_t*)rowsL.basis_keys.data(), R, ord, (const int64_t*)colsL.basis_keys.data(),
-                       (int64_t)colsL.basis_count, colsL.columns.view(), dense, colsL.dense_dim, depth, trial_depth,
+                       (const int64_t*)rowsL.basis_keys.data(), R, ord, nodes, depth, trial_depth,
                        (const D2*)table.data(), pb, load, out.cols.data(), out.vals.data(), inv, sched, inv_diag, has_diag,
                        records, present);
   KERNEL_CHECK();
 }
 
 template <class T>
-static void normal_stencil_load(const LevelState<T>& testL, int test_depth, const int64_t* nkeys, int64_t ncount, ColumnTable ct,
-                                DenseIndex dn, const T* nvals, int normal_depth, double* out, hipStream_t s) {
+static void normal_stencil_load(const LevelState<T>& testL, int test_depth, const NodeIndex& nodes, const T* nvals, int normal_depth,
+                                double* out, hipStream_t s) {
   const int R = testL.basis_count;
   if (!R) return;
-  if (!ncount) {
+  if (!nodes.count) {
     HIP_CHECK(hipMemsetAsync(out, 0, sizeof(double) * R, s));
     return;
   }
@@ -2958,17 +2934,9 @@ static void normal_stencil_load(const LevelState<T>& testL, int test_depth, cons
   hipLaunchKernelGGL(k_normal_table, dim3(blocks_for(rows * width, 256)), dim3(256), 0, s, test_depth, normal_depth, first, width,
                      table.data());
   KERNEL_CHECK();
-  if (dn.idx && width == 4)
-    hipLaunchKernelGGL((k_normal_load_dense<T, 4>), dim3(blocks_for(R, 128)), dim3(128), 0, s,
-                       (const int64_t*)testL.basis_keys.data(), R, dn, nvals, 3, test_depth, normal_depth, first,
-                       (const D2*)table.data(), out);
-  else if (dn.idx && width == 6)
-    hipLaunchKernelGGL((k_normal_load_dense<T, 6>), dim3(blocks_for(R, 128)), dim3(128), 0, s,
-                       (const int64_t*)testL.basis_keys.data(), R, dn, nvals, 3, test_depth, normal_depth, first,
-                       (const D2*)table.data(), out);
-  else
-    hipLaunchKernelGGL(k_normal_load<T>, dim3(blocks_for(R, 128)), dim3(128), 0, s, (const int64_t*)testL.basis_keys.data(), R,
-                       nkeys, ncount, ct, dn, nvals, 3, test_depth, normal_depth, first, width, (const D2*)table.data(), out);
+  auto kernel = width == 4 ? k_normal_load<T, 4> : k_normal_load<T, 6>;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(R, 128)), dim3(128), 0, s, (const int64_t*)testL.basis_keys.data(), R, nodes, nvals,
+                     test_depth, normal_depth, first, (const D2*)table.data(), out);
   KERNEL_CHECK();
 }
 
@@ -3214,9 +3182,7 @@ template <class T> static void ordered_normal_loads(Result<T>& r, hipStream_t s)
 template <class T> struct NormalLoadPlan {
   bool active = false;  // false: every level's load is already set
   int base = 0, depth = 0;
-  std::vector<ColumnIndex> records;         // per level, the normal records' column index
-  std::vector<DArray<int>> rdense;          // and their dense (x, y, z)-major index
-  std::vector<DenseIndex> rdn;
+  RecordIndex<T> records;
   std::vector<DArray<double>> finer;        // loads restricted to level d from the finer levels
   std::vector<DArray<double>> from_parent;  // from-parent loads, filled by the chain
   DArray<T> previous;                       // the chain's last cumulative coefficients
@@ -3245,37 +3211,19 @@ template <class T> static void normal_loads_base_levels(Result<T>& r, NormalLoad
   plan.depth = D;
   if (std::is_same<T, float>::value && base == 0) return;  // the ordered loads (normal_loads_base)
   plan.active = true;
-  plan.records.resize(D + 1);
-  plan.rdense.resize(D + 1);
-  plan.rdn.assign(D + 1, DenseIndex{});
   plan.finer.resize(D + 1);
   plan.from_parent.resize(D + 1);
   plan.from_child.resize(D + 1);
-  for (int d = 0; d <= D; ++d) {
-    const int64_t r0 = r.normal_offsets[d], r1 = r.normal_offsets[d + 1];
-    const int64_t* nk = r.normal_keys.data() + r0;
-    const T* nv = r.normal_vals.data() + 3 * r0;
-    build_column_index(nk, r1 - r0, (1 << d) + 1, plan.records[d], s);
-    // dense (x, y, z)-major index of the level's records for the tests taken
-    // in canonical order (consecutive z)
-    const int64_t rdim = (1 << d) + 1;
-    if (r1 > r0 && d >= 5 && rdim * rdim * rdim <= dense_index_max_cells()) {
-      plan.rdense[d].reset((size_t)(rdim * rdim * rdim), s);
-      HIP_CHECK(hipMemsetAsync(plan.rdense[d].data(), 0xff, sizeof(int) * (size_t)(rdim * rdim * rdim), s));
-      hipLaunchKernelGGL(k_dense_fill_xyz, dim3(blocks_for(r1 - r0, 256)), dim3(256), 0, s, nk, r1 - r0, (int)rdim,
-                         plan.rdense[d].data());
-      KERNEL_CHECK();
-      plan.rdn[d].idx = plan.rdense[d].data();
-      plan.rdn[d].dim = (int)rdim;
-    }
+  plan.records.build(r, s);
+  for (int d = base; d <= D; ++d) {
+    const NodeIndex nodes = plan.records.at(r, d);
+    const T* nv = r.normal_vals.data() + 3 * r.normal_offsets[d];
     if (d == base) {
       plan.same_base.reset(r.levels[d].basis_count, s);
-      normal_stencil_load(r.levels[d], d, nk, r1 - r0, plan.records[d].view(), plan.rdn[d], nv, d, plan.same_base.data(), s);
-    }
-    if (d > base) {
+      normal_stencil_load(r.levels[d], d, nodes, nv, d, plan.same_base.data(), s);
+    } else {
       plan.from_child[d - 1].reset(r.levels[d - 1].basis_count, s);
-      normal_stencil_load(r.levels[d - 1], d - 1, nk, r1 - r0, plan.records[d].view(), plan.rdn[d], nv, d,
-                          plan.from_child[d - 1].data(), s);
+      normal_stencil_load(r.levels[d - 1], d - 1, nodes, nv, d, plan.from_child[d - 1].data(), s);
     }
   }
   plan.levels_done = true;
@@ -3330,39 +3278,28 @@ template <class T> static void normal_loads_level(Result<T>& r, NormalLoadPlan<T
   while (plan.chain <= d - 1) {
     const int c = plan.chain;
     const int64_t r0 = r.normal_offsets[c], r1 = r.normal_offsets[c + 1];
-    const int64_t* nk = r.normal_keys.data() + r0;
     const T* nv = r.normal_vals.data() + 3 * r0;
     plan.has_cumulative = plan.has_cumulative || (r1 > r0);
     LevelState<T>& L = r.levels[c];
     DArray<T> cumulative(3 * (size_t)L.basis_count, s);
     if (L.basis_count) {
-      const LevelState<T>* P = c > 0 ? &r.levels[c - 1] : nullptr;
       hipLaunchKernelGGL(k_normal_prolong<T>, dim3(blocks_for(L.basis_count, 256)), dim3(256), 0, s,
-                         (const int64_t*)L.basis_keys.data(), L.basis_count, nk, r1 - r0, plan.records[c].view(), nv,
-                         P ? (const int64_t*)P->basis_keys.data() : (const int64_t*)nullptr, (int64_t)(P ? P->basis_count : 0),
-                         P ? P->columns.view() : ColumnTable{}, (const T*)plan.previous.data(), c, cumulative.data());
+                         (const int64_t*)L.basis_keys.data(), L.basis_count, plan.records.at(r, c), nv,
+                         c > 0 ? level_nodes(r, c - 1) : NodeIndex{}, (const T*)plan.previous.data(), c, cumulative.data());
       KERNEL_CHECK();
     }
     if (c >= plan.base && plan.has_cumulative) {
       plan.from_parent[c + 1].reset(r.levels[c + 1].basis_count, s);
-      DenseIndex bdn;
-      if (L.dense_dim) {
-        bdn.idx = L.dense.data();
-        bdn.dim = L.dense_dim;
-        bdn.zmajor = 1;
-      }
-      normal_stencil_load(r.levels[c + 1], c + 1, (const int64_t*)L.basis_keys.data(), (int64_t)L.basis_count,
-                          L.columns.view(), bdn, (const T*)cumulative.data(), c, plan.from_parent[c + 1].data(), s);
+      normal_stencil_load(r.levels[c + 1], c + 1, level_nodes(r, c), (const T*)cumulative.data(), c,
+                          plan.from_parent[c + 1].data(), s);
     }
     plan.previous = std::move(cumulative);
     ++plan.chain;
   }
-  const int64_t r0 = r.normal_offsets[d], r1 = r.normal_offsets[d + 1];
   LevelState<T>& L = r.levels[d];
   const int R = L.basis_count;
   DArray<double> load(R, s);
-  normal_stencil_load(L, d, r.normal_keys.data() + r0, r1 - r0, plan.records[d].view(), plan.rdn[d],
-                      r.normal_vals.data() + 3 * r0, d, load.data(), s);
+  normal_stencil_load(L, d, plan.records.at(r, d), r.normal_vals.data() + 3 * r.normal_offsets[d], d, load.data(), s);
   if (R) {
     hipLaunchKernelGGL(k_add_f64, dim3(blocks_for(R, 256)), dim3(256), 0, s, load.data(), (const double*)plan.finer[d].data(), R);
     KERNEL_CHECK();
@@ -3498,8 +3435,7 @@ static void prepare_finer(Result<T>& r, int d, Stencil<V>& Aop, Stencil<V>& Cop,
   const int* ord = f.sc.order.data();
   const int ts = relax_tile_size(r.prm.relax_tile, d);
   if (ts && R && r.prm.iters <= RELAX_MAX_SLICES)
-    build_tile_table(L.basis_keys.data(), ord, R, d, ts, L.dense_dim ? (const int*)L.dense.data() : (const int*)nullptr,
-                     L.dense_dim, f.tiles, s);
+    build_tile_table(level_nodes(r, d), ord, R, d, ts, f.tiles, s);
   L.point_load.reset(R, s);
   if (!screened) L.point_load.zero();
   PointSet<T> pts;
@@ -3518,12 +3454,12 @@ static void prepare_finer(Result<T>& r, int d, Stencil<V>& Aop, Stencil<V>& Cop,
   GsOperator<T, V>& op = f.op;
   op.R = R;
   if (f.tiles.tiles > 0) f.records.reset(R, s);
-  level_operator<T, V>(L, L, d, d, screened ? &pts : nullptr, L.point_load.data(), ord, inv.data(), Aop, &op,
+  level_operator<T, V>(r, d, d, screened ? &pts : nullptr, L.point_load.data(), ord, inv.data(), Aop, &op,
                        f.records.data(), f.nnz.data(), s);
   op.vals = std::move(Aop.vals);
   // the cross operator keeps canonical rows: its product with the coarser
   // cumulative solution gathers from neighbouring parents in key order
-  level_operator<T, V>(L, r.levels[d - 1], d, d - 1, screened ? &pts : nullptr, (double*)nullptr, (const int*)nullptr,
+  level_operator<T, V>(r, d, d - 1, screened ? &pts : nullptr, (double*)nullptr, (const int*)nullptr,
                        (const int*)nullptr, Cop, (GsOperator<T, V>*)nullptr, (RowRecord<T, V>*)nullptr,
                        (unsigned long long*)nullptr, s);
 }
@@ -3624,6 +3560,7 @@ static void solve_finer(Result<T>& r, int d, Stencil<V>& Aop, Stencil<V>& Cop, F
     st.launches = relax_sliced_any(op, f.sc, xs.data(), d, r.prm.iters, s);
   HIP_CHECK(hipEventRecord(st.end, s));
   r.relax_stats.push_back(st);
+  L.correction.reset(R, s);
   hipLaunchKernelGGL(k_scatter_rows<T>, dim3(blocks_for(R, 256)), dim3(256), 0, s, ord, R, (const T*)xs.data(),
                      L.correction.data());
   KERNEL_CHECK();
@@ -3807,7 +3744,7 @@ static void solve_cascade(Result<T>& r, std::vector<DArray<int>>& restr, bool sc
       L.point_load.reset(R, s);
       L.point_load.zero();
       L.rhs.reset(R, s);
-      Stencil<double> A = assemble_stiffness(L, L, d, d, s);
+      Stencil<double> A = assemble_stiffness(r, d, d, s);
       if (screened) {
         PointSet<T> pts = point_constraints(r, d, s);
         add_screening(A, L.basis_keys, pts, d, d, L.point_load.data(), s);
@@ -3887,46 +3824,30 @@ template <class T> void stage_solve(Result<T>& r) {
     (void)hipEventDestroy(tree_done);
     normal_loads_base_levels(r, plan, h);
   }
-  for (int d = 0; d <= D; ++d) {
-    LevelState<T>& L = r.levels[d];
-    build_column_index((const int64_t*)L.basis_keys.data(), L.basis_count, (1 << d) + 1, L.columns, s);
-    const int64_t dim = (1 << d) + 1;
-    if (L.basis_count && d >= 5 && dim * dim * dim <= dense_index_max_cells()) {
-      L.dense.reset((size_t)(dim * dim * dim), s);
-      HIP_CHECK(hipMemsetAsync(L.dense.data(), 0xff, sizeof(int) * (size_t)(dim * dim * dim), s));  // -1
-      hipLaunchKernelGGL(k_dense_fill, dim3(blocks_for(L.basis_count, 256)), dim3(256), 0, s, (const int64_t*)L.basis_keys.data(),
-                         L.basis_count, (int)dim, L.dense.data());
-      KERNEL_CHECK();
-      L.dense_dim = (int)dim;
-    }
-  }
+  index_field(r);
+  for (int d = r.word_depth + 1; d <= D; ++d)
+    build_column_index((const int64_t*)r.levels[d].basis_keys.data(), r.levels[d].basis_count, (1 << d) + 1, r.levels[d].columns, s);
   // prolongation P_d and restriction gathers (solver.py:340-342)
+  const LevelBlocks lb = level_blocks(r);
   std::vector<DArray<int>> restr(D + 1);
-  for (int d = 1; d <= D; ++d) {
-    LevelState<T>& F = r.levels[d];
-    LevelState<T>& C = r.levels[d - 1];
-    F.P.rows = F.basis_count;
-    F.P.cols_count = C.basis_count;
-    F.P.cols.reset(8 * (size_t)F.basis_count, s);
-    F.P.vals.reset(8 * (size_t)F.basis_count, s);
-    if (F.basis_count) {
-      hipLaunchKernelGGL(k_prolongation<T>, dim3(blocks_for(F.basis_count, 256)), dim3(256), 0, s,
-                         (const int64_t*)F.basis_keys.data(), F.basis_count, (const int64_t*)C.basis_keys.data(),
-                         (int64_t)C.basis_count, C.columns.view(), d, F.P.cols.data(), F.P.vals.data());
-      KERNEL_CHECK();
-    }
-    restr[d - 1].reset(27 * (size_t)C.basis_count, s);
-    if (C.basis_count) {
-      hipLaunchKernelGGL(k_restriction, dim3(blocks_for(C.basis_count, 256)), dim3(256), 0, s,
-                         (const int64_t*)C.basis_keys.data(), C.basis_count, (const int64_t*)F.basis_keys.data(),
-                         (int64_t)F.basis_count, F.columns.view(), d, restr[d - 1].data());
-      KERNEL_CHECK();
-    }
-  }
+  TransferLevels<T> tl;
   for (int d = 0; d <= D; ++d) {
     LevelState<T>& L = r.levels[d];
-    L.correction.reset(L.basis_count, s);
-    L.correction.zero();
+    tl.nodes[d] = level_nodes(r, d);
+    if (d < D) restr[d].reset(27 * (size_t)L.basis_count, s);
+    tl.restr[d] = restr[d].data();
+    if (d > 0) {
+      L.P.rows = L.basis_count;
+      L.P.cols_count = r.levels[d - 1].basis_count;
+      L.P.cols.reset(8 * (size_t)L.basis_count, s);
+      L.P.vals.reset(8 * (size_t)L.basis_count, s);
+    }
+    tl.pcols[d] = L.P.cols.data();
+    tl.pvals[d] = L.P.vals.data();
+  }
+  if (lb.blocks()) {
+    hipLaunchKernelGGL(k_transfers<T>, dim3((unsigned)lb.blocks()), dim3(LEVEL_BLOCK), 0, s, lb, tl);
+    KERNEL_CHECK();
   }
   const bool screened = r.prm.point_weight > 0 && !r.prm.exact_interpolation;
   if (r.prm.float_operators)
@@ -3935,8 +3856,10 @@ template <class T> void stage_solve(Result<T>& r) {
     solve_levels<T, T>(r, restr, screened, plan, s);
   for (int d = 0; d < D; ++d) r.levels[d].restriction = std::move(restr[d]);
   for (int d = 0; d <= D; ++d) {
-    r.levels[d].dense.free();
-    r.levels[d].dense_dim = 0;
+    LevelState<T>& L = r.levels[d];
+    if (L.solved) continue;
+    L.correction.reset(L.basis_count, s);
+    L.correction.zero();
   }
 }
 
@@ -4574,9 +4497,8 @@ __global__ void k_axpy_d(double* __restrict__ y, const double* __restrict__ x, d
 }
 
 // transpose of k_normal_load: record gradients from the load gradient
-__global__ void k_normal_load_vjp(const int64_t* __restrict__ keys, int R, const int64_t* __restrict__ nkeys, int64_t ncount,
-                                  ColumnTable ct, int test_depth, int normal_depth, int first, int width,
-                                  const D2* __restrict__ table, const double* __restrict__ gout, double* __restrict__ gvals) {
+__global__ void k_normal_load_vjp(const int64_t* __restrict__ keys, int R, NodeIndex nodes, int test_depth, int normal_depth,
+                                  int first, int width, const D2* __restrict__ table, const double* __restrict__ gout, double* __restrict__ gvals) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= R) return;
   const double g = gout[i];
@@ -4593,12 +4515,11 @@ __global__ void k_normal_load_vjp(const int64_t* __restrict__ keys, int R, const
     for (int y = 0; y < width; ++y) {
       const int ny = e1 + y + first;
       if (ny < 0 || ny >= lim || zlo > zhi) continue;
-      int64_t found[6];
-      find_run_table<6>(nkeys, ncount, ct, normal_depth, nx, ny, zlo, zhi - zlo + 1, found);
+      const NodeSpan span = find_span<6>(nodes, normal_depth, nx, ny, zlo);
       for (int z = 0; z < width; ++z) {
         const int nz = e2 + z + first;
         if (nz < zlo || nz > zhi) continue;
-        const int64_t jn = found[nz - zlo];
+        const int64_t jn = span.at(nz - zlo);
         if (jn < 0) continue;
         const D2 ix = table[c0 * width + x], iy = table[c1 * width + y], iz = table[c2 * width + z];
         atomicAdd(&gvals[3 * jn], g * ix.v1 * iy.v0 * iz.v0);
@@ -4612,25 +4533,23 @@ __global__ void k_normal_load_vjp(const int64_t* __restrict__ keys, int R, const
 // transpose of k_normal_prolong: own records and the previous level's
 // cumulative normal coefficients from this level's
 template <class T>
-__global__ void k_normal_prolong_vjp(const int64_t* __restrict__ keys, int R, const int64_t* __restrict__ own_keys,
-                                     int64_t own_count, ColumnTable own_ct, const int64_t* __restrict__ prev_keys,
-                                     int64_t prev_count, ColumnTable ct, int depth, const double* __restrict__ gcum,
-                                     double* __restrict__ gown, double* __restrict__ gprev) {
+__global__ void k_normal_prolong_vjp(const int64_t* __restrict__ keys, int R, NodeIndex records, NodeIndex prev, int depth,
+                                     const double* __restrict__ gcum, double* __restrict__ gown, double* __restrict__ gprev) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= R) return;
   const double g0 = gcum[3 * i], g1 = gcum[3 * i + 1], g2 = gcum[3 * i + 2];
   if (g0 == 0.0 && g1 == 0.0 && g2 == 0.0) return;
   const int64_t key = keys[i];
   const int c[3] = {key_x(key), key_y(key), key_z(key)};
-  int64_t own;
-  find_run_table<1>(own_keys, own_count, own_ct, depth, c[0], c[1], c[2], 1, &own);
+  const int64_t own = find_span<1>(records, depth, c[0], c[1], c[2]).at(0);
   if (own >= 0) {  // one row per record key: no other writer in this launch
     gown[3 * own] += g0; gown[3 * own + 1] += g1; gown[3 * own + 2] += g2;
   }
   if (depth == 0) return;
-  int64_t idx[2][2][2];
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) find_run_table<2>(prev_keys, prev_count, ct, depth - 1, c[0] / 2 + a, c[1] / 2 + b, c[2] / 2, 2, idx[a][b]);
+  NodeSpan span[2][2];  // [x bit][y bit]
+#pragma unroll
+  for (int k = 0; k < 4; ++k) span[k / 2][k % 2] = find_span<2>(prev, depth - 1, c[0] / 2 + k / 2, c[1] / 2 + k % 2, c[2] / 2);
+#pragma unroll
   for (int corner = 0; corner < 8; ++corner) {
     int p[3] = {c[0] / 2, c[1] / 2, c[2] / 2};
     T weight = T(1);
@@ -4639,7 +4558,7 @@ __global__ void k_normal_prolong_vjp(const int64_t* __restrict__ keys, int R, co
       weight = weight * (T(1) - fabs(T(c[axis]) * T(0.5) - T(p[axis])));
     }
     if (weight > T(0)) {
-      const int64_t j = idx[corner & 1][(corner >> 1) & 1][(corner >> 2) & 1];
+      const int64_t j = span[corner & 1][(corner >> 1) & 1].at((corner >> 2) & 1);
       if (j >= 0) {
         const double w = double(weight);
         atomicAdd(&gprev[3 * j], w * g0);
@@ -4739,22 +4658,14 @@ void tiled_backward(Result<T>& r, int d, int ts, const Stencil<V>& Aop, const do
   const int* cols = Aop.cols.data();
   const V* vals = Aop.vals.data();
   const unsigned blocks = blocks_for(R, 256);
-  DArray<int> dense, inv(R, s);
-  const int64_t dim = (1 << d) + 1;
-  const bool dense_ok = dim * dim * dim <= dense_index_max_cells();
-  if (dense_ok) {
-    dense.reset((size_t)(dim * dim * dim), s);
-    HIP_CHECK(hipMemsetAsync(dense.data(), 0xff, sizeof(int) * dense.size(), s));  // -1
-    hipLaunchKernelGGL(k_dense_fill, dim3(blocks), dim3(256), 0, s, (const int64_t*)L.basis_keys.data(), R, (int)dim, dense.data());
-    KERNEL_CHECK();
-  }
-  const int* level_dense = dense_ok ? (const int*)dense.data() : (const int*)nullptr;
+  const NodeIndex nodes = level_nodes(r, d);
+  DArray<int> inv(R, s);
   hipLaunchKernelGGL(k_inverse_permutation, dim3(blocks), dim3(256), 0, s, ord, R, inv.data());
   KERNEL_CHECK();
   DArray<T> xsnap;
   if (gA) {
     TileTable tt;
-    build_tile_table(L.basis_keys.data(), ord, R, d, ts, level_dense, (int)dim, tt, s);
+    build_tile_table(nodes, ord, R, d, ts, tt, s);
     DArray<RowRecord<T, V>> records(R, s);
     hipLaunchKernelGGL((k_row_records<T, T, V>), dim3(blocks), dim3(256), 0, s, ord, (const int*)inv.data(), 0, R, cols, vals,
                        records.data());
@@ -4772,7 +4683,7 @@ void tiled_backward(Result<T>& r, int d, int ts, const Stencil<V>& Aop, const do
     tiled_sweeps<T, V, TILED_SNAP>(tt, a, d, iters, s);
   }
   TileTable tt;
-  build_tile_table(L.basis_keys.data(), ord, R, d, ts, level_dense, (int)dim, tt, s, 3);
+  build_tile_table(nodes, ord, R, d, ts, tt, s, 3);
   DArray<RowRecord<double, V>> records(R, s);
   hipLaunchKernelGGL((k_row_records<double, T, V>), dim3(blocks), dim3(256), 0, s, ord, (const int*)inv.data(), 1, R, cols, vals,
                      records.data());
@@ -4929,10 +4840,10 @@ void gs_colored_reverse(const GsOperator<T>& op, const DArray<T>& tvals, const S
 
 // transpose of normal_stencil_load
 template <class T>
-void normal_load_vjp(const LevelState<T>& testL, int test_depth, const int64_t* nkeys, int64_t ncount, ColumnTable ct,
-                     int normal_depth, const double* gout, double* gvals, hipStream_t s) {
+void normal_load_vjp(const LevelState<T>& testL, int test_depth, const NodeIndex& nodes, int normal_depth, const double* gout,
+                     double* gvals, hipStream_t s) {
   const int R = testL.basis_count;
-  if (!R || !ncount) return;
+  if (!R || !nodes.count) return;
   const int width = test_depth < normal_depth ? 6 : 4;
   const int first = test_depth < normal_depth ? -3 : -2;
   const int rows = (1 << test_depth) + 1;
@@ -4941,7 +4852,7 @@ void normal_load_vjp(const LevelState<T>& testL, int test_depth, const int64_t* 
                      table.data());
   KERNEL_CHECK();
   hipLaunchKernelGGL(k_normal_load_vjp, dim3(blocks_for(R, 128)), dim3(128), 0, s, (const int64_t*)testL.basis_keys.data(), R,
-                     nkeys, ncount, ct, test_depth, normal_depth, first, width, (const D2*)table.data(), gout, gvals);
+                     nodes, test_depth, normal_depth, first, width, (const D2*)table.data(), gout, gvals);
   KERNEL_CHECK();
 }
 
@@ -4969,39 +4880,34 @@ void normal_loads_backward(Result<T>& r, std::vector<DArray<double>>& gload, int
       KERNEL_CHECK();
     }
   }
+  RecordIndex<T> records;
+  records.build(r, s);
   std::vector<DArray<double>> gcumn(D + 1);
   bool has_cumulative = false;
   for (int d = 0; d <= D; ++d) {
     const int64_t r0 = r.normal_offsets[d], r1 = r.normal_offsets[d + 1];
-    const int64_t* nk = r.normal_keys.data() + r0;
     double* gv = grecords + 3 * r0;
     has_cumulative = has_cumulative || (r1 > r0);
     LevelState<T>& L = r.levels[d];
-    ColumnIndex records;
-    build_column_index(nk, r1 - r0, (1 << d) + 1, records, s);
     if (d >= base) {
-      if (has(d)) normal_load_vjp(L, d, nk, r1 - r0, records.view(), d, (const double*)gload[d].data(), gv, s);
-      if (d > base) normal_load_vjp(r.levels[d - 1], d - 1, nk, r1 - r0, records.view(), d, (const double*)G[d - 1].data(), gv, s);
+      const NodeIndex nodes = records.at(r, d);
+      if (has(d)) normal_load_vjp(L, d, nodes, d, (const double*)gload[d].data(), gv, s);
+      if (d > base) normal_load_vjp(r.levels[d - 1], d - 1, nodes, d, (const double*)G[d - 1].data(), gv, s);
     }
     if (d < D) {
       gcumn[d] = zeros_d(3 * (size_t)L.basis_count, s);
       if (d >= base && has_cumulative && has(d + 1))
-        normal_load_vjp(r.levels[d + 1], d + 1, (const int64_t*)L.basis_keys.data(), (int64_t)L.basis_count, L.columns.view(), d,
-                        (const double*)gload[d + 1].data(), gcumn[d].data(), s);
+        normal_load_vjp(r.levels[d + 1], d + 1, level_nodes(r, d), d, (const double*)gload[d + 1].data(), gcumn[d].data(), s);
     }
   }
   // cumulative normal coefficients, finest first (normal_loads.py:27-63)
   for (int d = D - 1; d >= 0; --d) {
     LevelState<T>& L = r.levels[d];
     if (!L.basis_count) continue;
-    const int64_t r0 = r.normal_offsets[d], r1 = r.normal_offsets[d + 1];
-    ColumnIndex records;
-    build_column_index(r.normal_keys.data() + r0, r1 - r0, (1 << d) + 1, records, s);
-    const LevelState<T>* P = d > 0 ? &r.levels[d - 1] : nullptr;
+    const int64_t r0 = r.normal_offsets[d];
     hipLaunchKernelGGL(k_normal_prolong_vjp<T>, dim3(blocks_for(L.basis_count, 256)), dim3(256), 0, s,
-                       (const int64_t*)L.basis_keys.data(), L.basis_count, (const int64_t*)(r.normal_keys.data() + r0), r1 - r0,
-                       records.view(), P ? (const int64_t*)P->basis_keys.data() : (const int64_t*)nullptr,
-                       (int64_t)(P ? P->basis_count : 0), P ? P->columns.view() : ColumnTable{}, d,
+                       (const int64_t*)L.basis_keys.data(), L.basis_count, records.at(r, d),
+                       d > 0 ? level_nodes(r, d - 1) : NodeIndex{}, d,
                        (const double*)gcumn[d].data(), grecords + 3 * r0, d > 0 ? gcumn[d - 1].data() : (double*)nullptr);
     KERNEL_CHECK();
   }
