@@ -87,7 +87,7 @@ template <class T> struct Result {
   hipStream_t side = nullptr;  // a companion stream kept for the process (not owned)
   hipEvent_t average_done = nullptr;
   bool average_pending = false;
-  DArray<T> average_contrib;
+  DArray<T> average_contrib, average_totals;
   // HIP-event span of the main stream's wait for the side stream (metadata)
   hipEvent_t join_begin = nullptr, join_end = nullptr;
   void join_average() {

@@ -1093,70 +1093,147 @@ __global__ void k_average_contributions(const int* __restrict__ order, int G, co
   out[i] = v0; out[G + i] = v1; out[2 * (int64_t)G + i] = v2;
 }
 
-// One component chain per wave (three waves on three SIMDs), in element
-// order.  A skipped contribution is exactly (0,0,0); the running sums start at
-// +0 and never become -0, so adding it (or the +0 padding of the last chunk)
-// is the identity and the reference's `> 0` test (normals.py:160-163) needs no
-// branch.  Each wave stages AVG_CHUNK values of its component in LDS and reads
-// them back with one broadcast LDS load per value, so a step of the chain is
-// that load and one add; the next chunk's global loads are in flight
-// meanwhile.
-constexpr int AVG_PER_LANE = 16;
-constexpr int AVG_CHUNK = 64 * AVG_PER_LANE;
+// The three serial chains, each acc = fl(acc + v) in element order, without
+// their latency: one add after another takes 7 ns a value (480,000 float64
+// aggregates: 3.4 ms, which the operators' assembly and the base solve waited
+// for; this form 0.55 ms).
+//
+// While acc stays in one binade [2^e, 2^(e+1)) it is a whole number S of units
+// u = 2^(e-p), and adding v >= 0 is a whole-number addition: v / u rounded to
+// the nearest, and halfway cases to the side that leaves S even.  So a value
+// is a function of S's parity alone, "add a if S is even, b if odd", and such
+// functions compose associatively: a workgroup scans them over a chunk of
+// values and every thread knows its S exactly.  The thread in whose values S
+// reaches the binade's end adds them to acc one by one in T, and the threads
+// after it scan again in the new binade (a chain of n equal values crosses
+// log2 n of them).  acc starts at +0, where the first thread with a value
+// other than zero adds its own one by one.  Values that are negative or NaN, and
+// sums near underflow or not finite, take the whole chunk one by one.
+// A skipped contribution is exactly (0,0,0), the identity, as the reference's
+// `> 0` test (normals.py:160-163) makes it.
+constexpr int AVG_THREADS = 512;
+constexpr int AVG_EACH = 8;
+constexpr int AVG_CHUNK = AVG_THREADS * AVG_EACH;
+constexpr long long AVG_CAP = 1ll << 54;  // sums are only used below 2^53
+
+struct ParityAdd {
+  long long even, odd;
+};
+__device__ __forceinline__ ParityAdd then(ParityAdd l, ParityAdd r) {
+  const long long even = l.even + ((l.even & 1) ? r.odd : r.even), odd = l.odd + ((l.odd & 1) ? r.even : r.odd);
+  return ParityAdd{even < AVG_CAP ? even : AVG_CAP, odd < AVG_CAP ? odd : AVG_CAP};
+}
 
 template <class T>
-__global__ void __launch_bounds__(192) k_average_serial(const T* __restrict__ contrib, int G, T* __restrict__ out) {
-  __shared__ T stage[2][3][AVG_CHUNK];
-  __shared__ T totals[3];
-  const int comp = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (G <= 0) {
-    if (threadIdx.x == 0) out[0] = out[1] = out[2] = T(0);
-    return;
-  }
-  const T* __restrict__ src = contrib + (int64_t)comp * G;
-  T pre[AVG_PER_LANE];
-  auto load = [&](int first) {  // clamped addresses (G >= 1)
+__global__ void __launch_bounds__(AVG_THREADS) k_average_chains(const T* __restrict__ contrib, int G, T* __restrict__ totals) {
+  constexpr int P = sizeof(T) == 8 ? 52 : 23;  // fraction bits
+  constexpr int WAVES = AVG_THREADS / 64;
+  __shared__ T stage[AVG_CHUNK + AVG_CHUNK / AVG_EACH];  // a value of padding a thread: no bank conflicts
+  __shared__ ParityAdd wave_total[WAVES];
+  __shared__ int first_cross[WAVES];
+  __shared__ T acc;
+  __shared__ int bad;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const T* __restrict__ src = contrib + (int64_t)blockIdx.x * G;
+  T pre[AVG_EACH];
+  auto load = [&](int64_t first) {
 #pragma unroll
-    for (int k = 0; k < AVG_PER_LANE; ++k) {
-      const int e = first + k * 64 + lane;
-      pre[k] = src[e < G ? e : G - 1];
+    for (int k = 0; k < AVG_EACH; ++k) {
+      const int64_t i = first + k * AVG_THREADS + tid;
+      pre[k] = i < G ? src[i] : T(0);
     }
   };
-  auto keep = [&](int b, int first) {  // +0 past the end
-#pragma unroll
-    for (int k = 0; k < AVG_PER_LANE; ++k) stage[b][comp][k * 64 + lane] = first + k * 64 + lane < G ? pre[k] : T(0);
-  };
-  T acc = T(0);
+  if (tid == 0) acc = T(0);
   load(0);
-  keep(0, 0);
-  __syncthreads();
-  int b = 0;
-  for (int first = 0; first < G; first += AVG_CHUNK) {
-    const bool more = first + AVG_CHUNK < G;
-    if (more) load(first + AVG_CHUNK);
-    const T* chunk = stage[b][comp];
-    // the next 16 values are read while the current 16 are added
-    T cur[16], nxt[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) cur[u] = chunk[u];
-    for (int k = 0; k < AVG_CHUNK; k += 16) {
-      if (k + 16 < AVG_CHUNK) {
-#pragma unroll
-        for (int u = 0; u < 16; ++u) nxt[u] = chunk[k + 16 + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 16; ++u) acc = acc + cur[u];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) cur[u] = nxt[u];
-    }
-    // the staging stores wait for the next chunk's loads: keep them after the chain
-    __asm__ __volatile__("" ::: "memory");
-    if (more) keep(b ^ 1, first + AVG_CHUNK);
+  for (int64_t first = 0; first < G; first += AVG_CHUNK) {
     __syncthreads();
-    b ^= 1;
+    if (tid == 0) bad = 0;
+#pragma unroll
+    for (int k = 0; k < AVG_EACH; ++k) {
+      const int i = k * AVG_THREADS + tid;
+      stage[i + i / AVG_EACH] = pre[k];
+    }
+    __syncthreads();
+    if (first + AVG_CHUNK < G) load(first + AVG_CHUNK);
+    T v[AVG_EACH];
+    bool any = false, wrong = false;
+#pragma unroll
+    for (int k = 0; k < AVG_EACH; ++k) {
+      v[k] = stage[tid * (AVG_EACH + 1) + k];
+      any = any || v[k] != T(0);
+      wrong = wrong || !(v[k] >= T(0));
+    }
+    if (wrong) bad = 1;
+    __syncthreads();
+    for (int from = 0; from < AVG_THREADS;) {  // uniform over the workgroup
+      const T a0 = acc;
+      if (bad || !(a0 == T(0) || (a0 >= T(1e-30) && a0 <= T(1e30)))) {
+        __syncthreads();  // acc is read
+        if (tid == 0) {
+          T t = a0;
+          for (int i = from * AVG_EACH; i < AVG_CHUNK; ++i) t = t + stage[i + i / AVG_EACH];
+          acc = t;
+        }
+        __syncthreads();
+        break;
+      }
+      int e = 0;
+      if (a0 != T(0)) e = ilogb(double(a0));
+      const double scale = ldexp(1.0, P - e), unit = ldexp(1.0, e - P);
+      const long long limit = 1ll << (P + 1), S0 = (long long)(double(a0) * scale);
+      ParityAdd own{0, 0};
+      if (tid >= from) {
+#pragma unroll
+        for (int k = 0; k < AVG_EACH; ++k) {
+          const double x = fmin(double(v[k]) * scale, double(AVG_CAP)), m = floor(x), f = x - m;
+          const long long lo = (long long)m, hi = lo + 1;
+          // halfway: to the neighbour that leaves S even
+          const ParityAdd one = f == 0.5 ? ParityAdd{(lo & 1) ? hi : lo, (lo & 1) ? lo : hi}
+                                         : ParityAdd{f > 0.5 ? hi : lo, f > 0.5 ? hi : lo};
+          own = then(own, one);
+        }
+      }
+      ParityAdd scan = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const ParityAdd l{__shfl_up(scan.even, o), __shfl_up(scan.odd, o)};
+        if (lane >= o) scan = then(l, scan);
+      }
+      if (lane == 63) wave_total[wave] = scan;
+      ParityAdd before{__shfl_up(scan.even, 1), __shfl_up(scan.odd, 1)};
+      if (lane == 0) before = ParityAdd{0, 0};
+      __syncthreads();
+      ParityAdd base{0, 0}, all{0, 0};
+      for (int w = 0; w < WAVES; ++w) {
+        if (w == wave) base = all;
+        all = then(all, wave_total[w]);
+      }
+      before = then(base, before);
+      const long long start = S0 + ((S0 & 1) ? before.odd : before.even);
+      const long long end = start + ((start & 1) ? own.odd : own.even);
+      const bool cross = tid >= from && (a0 == T(0) ? any : end >= limit);
+      const unsigned long long m = __ballot(cross);
+      if (lane == 0) first_cross[wave] = m ? wave * 64 + __ffsll(m) - 1 : AVG_THREADS;
+      __syncthreads();
+      int at = AVG_THREADS;
+      for (int w = 0; w < WAVES; ++w) at = min(at, first_cross[w]);
+      if (at == AVG_THREADS) {
+        if (tid == 0) acc = T(double(S0 + ((S0 & 1) ? all.odd : all.even)) * unit);
+      } else if (tid == at) {
+        T t = a0 == T(0) ? T(0) : T(double(start) * unit);
+#pragma unroll
+        for (int k = 0; k < AVG_EACH; ++k) t = t + v[k];
+        acc = t;
+      }
+      from = at + 1;
+      __syncthreads();
+    }
   }
-  if (lane == 0) totals[comp] = acc;
   __syncthreads();
+  if (tid == 0) totals[blockIdx.x] = acc;
+}
+
+template <class T> __global__ void k_average_finish(const T* __restrict__ totals, T* __restrict__ out) {
   if (threadIdx.x == 0) {
     const T t0 = totals[0], t1 = totals[1], t2 = totals[2];
     out[0] = out[1] = out[2] = T(0);
@@ -1234,6 +1311,7 @@ template <class T> void stage_normals(Result<T>& r) {
   // side stream (joined before the first use of the average)
   r.average_contrib.reset(3 * (size_t)G, s);
   r.normal_average.reset(3, s);
+  r.average_totals.reset(3, s);
   hipLaunchKernelGGL(k_average_contributions<T>, dim3(blocks_for(G, 256)), dim3(256), 0, s,
                      (const int*)r.normal_order.data(), G, (const T*)r.normal_sums.data(), (const T*)r.weights.data(),
                      (const T*)r.dw.data(), r.average_contrib.data());
@@ -1251,8 +1329,10 @@ template <class T> void stage_normals(Result<T>& r) {
     HIP_CHECK(hipStreamWaitEvent(r.side, ready, 0));
     HIP_CHECK(hipEventDestroy(ready));
   }
-  hipLaunchKernelGGL(k_average_serial<T>, dim3(1), dim3(192), 0, r.side, (const T*)r.average_contrib.data(), G,
-                     r.normal_average.data());
+  hipLaunchKernelGGL(k_average_chains<T>, dim3(3), dim3(AVG_THREADS), 0, r.side, (const T*)r.average_contrib.data(), G,
+                     r.average_totals.data());
+  KERNEL_CHECK();
+  hipLaunchKernelGGL(k_average_finish<T>, dim3(1), dim3(64), 0, r.side, (const T*)r.average_totals.data(), r.normal_average.data());
   KERNEL_CHECK();
   HIP_CHECK(hipEventRecord(r.average_done, r.side));
   r.average_pending = true;
