@@ -606,7 +606,7 @@ __global__ void k_spmv(const int* __restrict__ cols, const V* __restrict__ vals,
 // depth 9, cleared for each of the two key sets) waited as often on loads that
 // missed every cache.
 template <class V, int W>
-__global__ void __launch_bounds__(128) k_normal_load(const int64_t* __restrict__ keys, int R, NodeIndex nodes,
+__global__ void __launch_bounds__(256) k_normal_load(const int64_t* __restrict__ keys, int R, NodeIndex nodes,
                                                      const V* __restrict__ nvals, int test_depth, int normal_depth, int first,
                                                      const D2* __restrict__ table, double* __restrict__ out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2876,6 +2876,18 @@ template <class T> static Stencil<T> cast_stencil(Stencil<double>&& m, hipStream
   return out;
 }
 
+// LDS that a launch of the large assembly kernels (k_level_operator,
+// k_normal_load; they use none) asks for: two of their 256-thread workgroups
+// then fill a compute unit and 32 KB of it stay free for a workgroup of the
+// relaxation, which runs beside them on the solve stream.  Without, they take
+// every slot as it comes free and a wave of the relaxation waits for the end of
+// their grid: 45 us a step in place of 10, two steps 430 us, while level 9 of
+// 480,000 aggregates is assembled.  Fewer workgroups cost the assembly
+// little (it waits on memory).  800,000 points at depth 9 in mixed precision
+// 21.0 -> 20.3 ms, 250,000 at depth 8 in float32 7.2 -> 7.0 (with 44 KB for
+// k_normal_load and none for k_level_operator 20.5 and 7.15).
+constexpr size_t ASSEMBLY_LDS = 64 * 1024;
+
 // A sliced finer level's operator (trial_depth = depth; op and present given)
 // or cross operator (trial_depth one level coarser) in one pass of
 // k_level_operator, rows in schedule order ord (inv = its inverse) or, with ord
@@ -2906,12 +2918,12 @@ static void level_operator(const Result<T>& r, int depth, int trial_depth,
   T* inv_diag = op ? op->inv_diag.data() : nullptr;
   unsigned char* has_diag = op ? op->has_diag.data() : nullptr;
   if (pts)
-    hipLaunchKernelGGL((k_level_operator<T, V, true>), dim3(blocks_for(R, 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL((k_level_operator<T, V, true>), dim3(blocks_for(R, 256)), dim3(256), ASSEMBLY_LDS, s,
                        (const int64_t*)rowsL.basis_keys.data(), R, ord, nodes, depth, trial_depth,
                        (const D2*)table.data(), pb, load, out.cols.data(), out.vals.data(), inv, sched, inv_diag, has_diag,
                        records, present);
   else
-    hipLaunchKernelGGL((k_level_operator<T, V, false>), dim3(blocks_for(R, 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL((k_level_operator<T, V, false>), dim3(blocks_for(R, 256)), dim3(256), ASSEMBLY_LDS, s,
                        (const int64_t*)rowsL.basis_keys.data(), R, ord, nodes, depth, trial_depth,
                        (const D2*)table.data(), pb, load, out.cols.data(), out.vals.data(), inv, sched, inv_diag, has_diag,
                        records, present);
@@ -2935,7 +2947,7 @@ static void normal_stencil_load(const LevelState<T>& testL, int test_depth, cons
                      table.data());
   KERNEL_CHECK();
   auto kernel = width == 4 ? k_normal_load<T, 4> : k_normal_load<T, 6>;
-  hipLaunchKernelGGL(kernel, dim3(blocks_for(R, 128)), dim3(128), 0, s, (const int64_t*)testL.basis_keys.data(), R, nodes, nvals,
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(R, 256)), dim3(256), ASSEMBLY_LDS, s, (const int64_t*)testL.basis_keys.data(), R, nodes, nvals,
                      test_depth, normal_depth, first, (const D2*)table.data(), out);
   KERNEL_CHECK();
 }
@@ -3613,7 +3625,6 @@ template <class T, class V> class FinerAssembly {
     HIP_CHECK(hipEventDestroy(fork));
     // the point constraints' weights use the serial normal average
     if (r.average_pending) HIP_CHECK(hipStreamWaitEvent(as_, r.average_done, 0));
-    HIP_CHECK(hipEventCreateWithFlags(&gate_, hipEventDisableTiming));
     thread_ = std::thread([this, dev, screened] { run(dev, screened); });
   }
   FinerAssembly(const FinerAssembly&) = delete;
@@ -3633,17 +3644,6 @@ template <class T, class V> class FinerAssembly {
       (void)hipEventDestroy(end);
     }
     for (auto& e : events_) (void)hipEventDestroy(e);
-    (void)hipEventDestroy(gate_);
-  }
-  // Levels after the first two are assembled only once the solve stream has
-  // passed this point (the base solve's single-workgroup kernels slow down
-  // several times when they share compute units with the assembly).
-  void open_gate() {
-    if (!thread_.joinable()) return;
-    HIP_CHECK(hipEventRecord(gate_, s_));
-    std::lock_guard<std::mutex> g(mu_);
-    gate_open_ = true;
-    cv_.notify_all();
   }
   // The finer levels' loads: each is set on the assembly stream before its
   // level's event, after the solve stream's plan.ready.
@@ -3675,13 +3675,6 @@ template <class T, class V> class FinerAssembly {
         {
           std::lock_guard<std::mutex> g(mu_);
           if (cancel_) break;
-        }
-        if (d == first_ + 2) {
-          std::unique_lock<std::mutex> g(mu_);
-          cv_.wait(g, [&] { return gate_open_ || cancel_; });
-          if (cancel_) break;
-          g.unlock();
-          HIP_CHECK(hipStreamWaitEvent(as_, gate_, 0));
         }
         LevelState<T>& L = r_.levels[d];
         if (!L.basis_count) break;
@@ -3716,14 +3709,13 @@ template <class T, class V> class FinerAssembly {
   Result<T>& r_;
   int first_, last_;
   hipStream_t s_, as_ = nullptr;
-  hipEvent_t gate_ = nullptr;
   std::vector<FinerLevel<T, V>> levels_;
   std::vector<hipEvent_t> events_;
   std::thread thread_;
   std::mutex mu_;
   std::condition_variable cv_;
   int ready_ = 0;
-  bool cancel_ = false, done_ = false, gate_open_ = false;
+  bool cancel_ = false, done_ = false;
   NormalLoadPlan<T>* loads_ = nullptr;
   bool loads_waited_ = false;  // assembly thread only
   std::exception_ptr error_;
@@ -3760,7 +3752,6 @@ static void solve_cascade(Result<T>& r, std::vector<DArray<int>>& restr, bool sc
       });
       cumulative.reset(R, s);
       HIP_CHECK(hipMemcpyAsync(cumulative.data(), L.correction.data(), sizeof(T) * R, hipMemcpyDeviceToDevice, s));
-      finer.open_gate();
     } else {
       FinerLevel<T, V>& f = finer.wait(d);
       PreparedLevel<T> cur = next.ready ? std::move(next) : finer_prepare<T, V>(r, d, f, s);
