@@ -163,18 +163,6 @@ __device__ __forceinline__ void stiffness_row(int64_t key, const NodeIndex& cols
   }
 }
 
-__global__ void k_stiffness(const int64_t* __restrict__ rows, int R, const int* __restrict__ row_order, NodeIndex cols, int depth,
-                            int trial_depth, const D2* __restrict__ table, int* __restrict__ out_cols,
-                            double* __restrict__ out_vals) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;  // output position
-  if (j >= R) return;
-  const int i = row_order ? row_order[j] : j;
-  stiffness_row(rows[i], cols, depth, trial_depth, table, [&](int k, int index, double v) {
-    out_cols[(int64_t)k * R + j] = index;
-    out_vals[(int64_t)k * R + j] = v;
-  });
-}
-
 // ---------------------------------------------------------------- constraints (constraints.py:20-84)
 template <class T>
 __global__ void k_points(const int64_t* __restrict__ akeys, const T* __restrict__ avals, int P, const int64_t* __restrict__ active,
@@ -346,24 +334,6 @@ __device__ __forceinline__ void screening_row(int64_t key, int depth, int trial_
     }
 }
 
-// screening_stencils.py:34-70 (add): per row, the screening sums added to
-// the present slots of an assembled stencil, and the point load.
-template <class T>
-__global__ void __launch_bounds__(128) k_screening(const int64_t* __restrict__ rows, int R, const int* __restrict__ row_order,
-                                                   int depth, int trial_depth, PointBins<T> pb,
-                                                   const int* __restrict__ scols, double* __restrict__ svals,
-                                                   double* __restrict__ load) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;  // output position
-  if (j >= R) return;
-  const int i = row_order ? row_order[j] : j;
-  double acc[27], rhs;
-  screening_row(rows[i], depth, trial_depth, pb, acc, rhs);
-  if (load) load[j] = rhs;
-#pragma unroll
-  for (int k = 0; k < 27; ++k)
-    if (scols[(int64_t)k * R + j] >= 0) svals[(int64_t)k * R + j] += acc[k];
-}
-
 // One row of a finer level's operator for the tiled relaxation: its 27 slot
 // values, diagonal flag and 1/A_ii, at schedule position j, so a row's
 // operator is a few consecutive 16-byte words.
@@ -442,12 +412,6 @@ __global__ void __launch_bounds__(256) k_level_operator(const int64_t* __restric
     __syncthreads();
     if (threadIdx.x == 0 && block_count) atomicAdd(present, block_count);
   }
-}
-
-template <class T>
-__global__ void k_cast(const double* __restrict__ in, T* __restrict__ out, int64_t n) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = T(in[i]);
 }
 
 // solver.py:119-126 (_rhs)
@@ -711,17 +675,20 @@ __global__ void __launch_bounds__(128) k_galerkin(const int* __restrict__ rcols,
   // thread t sums its contributions in ascending R-row order (one A slot per
   // R entry reaches t), then thread s sums row s of (R A) P over t ascending
   // and P slot ascending -- the sequential order of both products.
-  __shared__ T ra[125];
-  __shared__ int rak[125];
-  __shared__ int cs[125][8];
-  __shared__ int cn[125][8];  // the coarse column a contribution lands in
-  __shared__ T cv[125][8];
-  __shared__ int landed[128];  // contributions per fine offset
+  // Slot o of the result (coarse offset o per axis) receives from the fine
+  // offsets 2o-1..2o+1 per axis only (trilinear P: fine f feeds coarse f/2 when
+  // f is even, (f-1)/2 and (f+1)/2 when odd), from each at most once: term
+  // [slot][candidate], candidates ascending, which is the sequential order.
+  // Dependent loads bound it: 14 us a level.  One thread a slot scanning its
+  // candidates' eight P slots took as long again (27 us).
+  __shared__ T term[27][27];
+  __shared__ int term_col[27][27];  // the coarse column a term lands in, -1 for none
   const int r = blockIdx.x;
   const int t = threadIdx.x;
   const int64_t rkey = ckeys[r];
   const int rx = key_x(rkey), ry = key_y(rkey), rz = key_z(rkey);
-  int n = 0;
+  for (int e = t; e < 27 * 27; e += 128) term_col[e / 27][e % 27] = -1;
+  __syncthreads();
   if (t < 125) {
     // Each dependent step (R columns, A columns, A values; P columns, coarse
     // keys, P values) is issued for every slot before any is used, then the
@@ -749,89 +716,39 @@ __global__ void __launch_bounds__(128) k_galerkin(const int* __restrict__ rcols,
       acc = acc + T(restriction_weight(kr)) * av[kr];
       col = ac[kr];
     }
-    ra[t] = acc;
-    rak[t] = col;
     int pc[8];
 #pragma unroll
     for (int kp = 0; kp < 8; ++kp) pc[kp] = col >= 0 ? pcols[(int64_t)kp * F + col] : -1;
     int64_t pkey[8];
 #pragma unroll
     for (int kp = 0; kp < 8; ++kp) pkey[kp] = pc[kp] >= 0 ? ckeys[pc[kp]] : int64_t(0);
+    T pv[8];
+#pragma unroll
+    for (int kp = 0; kp < 8; ++kp) pv[kp] = pc[kp] >= 0 ? pvals[(int64_t)kp * F + col] : T(0);
 #pragma unroll
     for (int kp = 0; kp < 8; ++kp) {
-      int sidx = -1;
-      T pv = T(0);
-      if (pc[kp] >= 0) {
-        const int ox = key_x(pkey[kp]) - rx + 1, oy = key_y(pkey[kp]) - ry + 1, oz = key_z(pkey[kp]) - rz + 1;
-        if ((unsigned)ox <= 2u && (unsigned)oy <= 2u && (unsigned)oz <= 2u) {  // always for trilinear P
-          sidx = ox * 9 + oy * 3 + oz;
-          pv = pvals[(int64_t)kp * F + col];
-        }
-      }
-      cs[t][kp] = sidx;
-      cn[t][kp] = pc[kp];
-      cv[t][kp] = pv;
-      n += sidx >= 0 ? 1 : 0;
+      if (pc[kp] < 0) continue;
+      const int ox = key_x(pkey[kp]) - rx + 1, oy = key_y(pkey[kp]) - ry + 1, oz = key_z(pkey[kp]) - rz + 1;
+      if ((unsigned)ox > 2u || (unsigned)oy > 2u || (unsigned)oz > 2u) continue;  // never for trilinear P
+      const int slot = ox * 9 + oy * 3 + oz;
+      const int candidate = (tx - 2 * ox + 1) * 9 + (ty - 2 * oy + 1) * 3 + (tz - 2 * oz + 1);
+      term[slot][candidate] = acc * pv[kp];
+      term_col[slot][candidate] = pc[kp];
     }
   }
-  if (t < 128) landed[t] = n;
   __syncthreads();
-  if (t < 64) {
-    // Slot t (coarse offset o per axis) is reached only from fine offsets
-    // 2o-1..2o+1 per axis (trilinear P: fine f feeds coarse f/2 when f is
-    // even, (f-1)/2 and (f+1)/2 when odd), so each slot scans those 27 in
-    // ascending order -- the order of the full scan.  Every contribution is
-    // counted once: if the candidates miss any, the full scan runs instead.
-    // The column of slot t is the coarse index of any contribution landing
-    // there (keys are unique).
-    int total = landed[t] + landed[t + 64];
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m);
+  if (t < 27) {
     T out = T(0);
-    int col = -1, found = 0;
-    if (t < 27) {
-      const int ox = t / 9, oy = (t / 3) % 3, oz = t % 3;
-      for (int a = 0; a < 3; ++a) {
-        const int ux = 2 * ox - 1 + a;
-        if (ux < 0 || ux > 4) continue;
-        for (int b = 0; b < 3; ++b) {
-          const int uy = 2 * oy - 1 + b;
-          if (uy < 0 || uy > 4) continue;
-          for (int c = 0; c < 3; ++c) {
-            const int uz = 2 * oz - 1 + c;
-            if (uz < 0 || uz > 4) continue;
-            const int u = ux * 25 + uy * 5 + uz;
-            if (rak[u] < 0) continue;
+    int col = -1;
 #pragma unroll
-            for (int kp = 0; kp < 8; ++kp)
-              if (cs[u][kp] == t) {
-                out = out + ra[u] * cv[u][kp];
-                col = cn[u][kp];
-                ++found;
-              }
-          }
-        }
-      }
+    for (int e = 0; e < 27; ++e) {
+      const int c = term_col[t][e];
+      const T sum = out + term[t][e];
+      out = c >= 0 ? sum : out;
+      col = c >= 0 ? c : col;
     }
-    int all = found;
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) all += __shfl_xor(all, m);
-    if (all != total && t < 27) {
-      out = T(0);
-      col = -1;
-      for (int u = 0; u < 125; ++u) {
-        if (rak[u] < 0) continue;
-        for (int kp = 0; kp < 8; ++kp)
-          if (cs[u][kp] == t) {
-            out = out + ra[u] * cv[u][kp];
-            col = cn[u][kp];
-          }
-      }
-    }
-    if (t < 27) {
-      out_cols[(int64_t)t * C + r] = col;
-      out_vals[(int64_t)t * C + r] = out;
-    }
+    out_cols[(int64_t)t * C + r] = col;
+    out_vals[(int64_t)t * C + r] = out;
   }
 }
 
@@ -1038,7 +955,7 @@ __global__ void k_gather_operator(const int* __restrict__ order, int R, const in
     svals[(int64_t)k * R + j] = v;
     if (c == i) diagonal = v;
   }
-  sb[j] = b[i];
+  if (b) sb[j] = b[i];
   has_diag[j] = diagonal != T(0);
   inv_diag[j] = diagonal != T(0) ? T(1) / diagonal : T(0);
 }
@@ -1052,7 +969,7 @@ __device__ __forceinline__ int root_row(const int64_t* __restrict__ keys, int i)
 }
 
 template <class T>
-__device__ void root_apply(const int* __restrict__ cols, const T* __restrict__ vals, int R, const int64_t* __restrict__ keys, int dc,
+__device__ __forceinline__ void root_apply(const int* __restrict__ cols, const T* __restrict__ vals, int R, const int64_t* __restrict__ keys, int dc,
                            const T* v, T* out) {
   if (!dc) {
     for (int i = 0; i < R; ++i) {
@@ -1093,10 +1010,9 @@ __device__ void root_apply(const int* __restrict__ cols, const T* __restrict__ v
 // Root solve on one lane: skip when |r|^2 <= eps^2, else unpreconditioned CG
 // (solver.py:276-297; Warp's cg restated, bitwise parity unpinned).
 template <class T>
-__global__ void k_root_solve(const int* __restrict__ cols, const T* __restrict__ vals, int R, const int64_t* __restrict__ keys,
-                             const T* __restrict__ rhs, T* __restrict__ x, T* __restrict__ pad_x, T* __restrict__ work,
-                             int dc, int base, int cycle, double acc, int maxiter, int* __restrict__ ran) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ __forceinline__ void root_solve(const int* __restrict__ cols, const T* __restrict__ vals, int R,
+                                           const int64_t* __restrict__ keys, const T* rhs, T* x, T* pad_x, T* work, int dc,
+                                           int base, int cycle, double acc, int maxiter, int* __restrict__ ran) {
   const int m = dc ? 64 : R;
   T* b = work;
   T* r = work + 64;
@@ -1140,6 +1056,14 @@ __global__ void k_root_solve(const int* __restrict__ cols, const T* __restrict__
     rz = rz_new;
     for (int i = 0; i < m; ++i) p[i] = r[i] + beta * p[i];
   }
+}
+
+template <class T>
+__global__ void k_root_solve(const int* __restrict__ cols, const T* __restrict__ vals, int R, const int64_t* __restrict__ keys,
+                             const T* __restrict__ rhs, T* __restrict__ x, T* __restrict__ pad_x, T* __restrict__ work,
+                             int dc, int base, int cycle, double acc, int maxiter, int* __restrict__ ran) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  root_solve(cols, vals, R, keys, rhs, x, pad_x, work, dc, base, cycle, acc, maxiter, ran);
 }
 
 // Reverse of k_root_solve when its conjugate gradient ran (solver_adjoint.py
@@ -1926,8 +1850,7 @@ template <class T, class V = T> struct GsOperator {
 };
 
 template <class T>
-static GsOperator<T> gather_operator(const Schedule<T>& sc, const DArray<int>& cols, const DArray<T>& vals, const T* b, int R,
-                                     hipStream_t s) {
+static GsOperator<T> gather_operator(const Schedule<T>& sc, const int* cols, const T* vals, const T* b, int R, hipStream_t s) {
   GsOperator<T> op;
   op.R = R;
   op.update_order = sc.order.data();
@@ -1938,8 +1861,7 @@ static GsOperator<T> gather_operator(const Schedule<T>& sc, const DArray<int>& c
   op.has_diag.reset(R, s);
   if (R) {
     hipLaunchKernelGGL(k_gather_operator<T>, dim3(blocks_for(R, 256)), dim3(256), 0, s, (const int*)sc.order.data(), R,
-                       (const int*)cols.data(), (const T*)vals.data(), b, op.cols.data(), op.vals.data(), op.b.data(),
-                       op.inv_diag.data(), op.has_diag.data());
+                       cols, vals, b, op.cols.data(), op.vals.data(), op.b.data(), op.inv_diag.data(), op.has_diag.data());
     KERNEL_CHECK();
   }
   return op;
@@ -2739,6 +2661,174 @@ __global__ void __launch_bounds__(RELAX_BLOCK_REGS_ROWS) k_relax_block_regs(cons
 constexpr size_t RELAX_BLOCK_LDS_BYTES = 65536;
 
 // snap (optional): x before the call, then after every sweep, R values each.
+// One V-cycle over the base levels of at most RELAX_BLOCK_REGS_ROWS rows
+// (solver.py:241-317): relaxation, residual and restriction down to the root,
+// the root solve, prolongation and relaxation back up, all in one workgroup.
+// Launches bound the base solve, not its work: at base depth 3 it was 27 small
+// launches a cycle (and 24 to set schedules and gathered operators up, which a
+// workgroup does without: a thread takes the row whose place in the colour
+// order is its own, so one or two waves work in a phase).  Every sum keeps its
+// order.  Base depth 3 in float32: 171 us (280 with a select for absent
+// neighbours); reconstructions of 20,000 points at depth 6 2.62 -> 2.47 ms, of
+// 60,001 at depth 7 in float64 (base depth 4, the same below it) 4.34 -> 4.05.
+template <class T> struct BaseLevel {
+  const int64_t* keys;
+  const int* cols;  // 27 slots, canonical rows
+  const T* vals;
+  const int* pcols;  // prolongation from the level below
+  const T* pvals;
+  const int* restr;  // this level's gathers from the level above
+  T* rhs;
+  T* x;
+  int R;
+};
+template <class T> struct BaseCycle {
+  BaseLevel<T> level[MAX_LEVELS];
+  int top, base, cycle, iters;
+  int zero_top;  // the top level starts from zero, not from its x
+  double acc;
+  int* ran;
+  T* root_b;  // the root solve's inputs, for the reverse pass
+  T* root_x;
+};
+
+template <class T> __global__ void __launch_bounds__(RELAX_BLOCK_REGS_ROWS) k_base_cycle(BaseCycle<T> a) {
+  constexpr int WAVES = RELAX_BLOCK_REGS_ROWS / 64;
+  // an absent neighbour is the slot past the rows, +0 times +0: r - (+0) is r,
+  // and a sum that started at +0 is never -0, so it needs no select
+  constexpr int ABSENT = RELAX_BLOCK_REGS_ROWS;
+  __shared__ T xs[RELAX_BLOCK_REGS_ROWS + 1], other[RELAX_BLOCK_REGS_ROWS];
+  __shared__ int placed[RELAX_BLOCK_REGS_ROWS];
+  __shared__ int counts[8 * WAVES];
+  const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // relaxes level d from xs; residual: afterwards rhs - A x goes to other
+  auto relax = [&](const BaseLevel<T>& L, bool forward, bool residual) {
+    const int R = L.R;
+    int colour = -1, pre = 0;
+    if (tid < R) {
+      const int64_t key = L.keys[tid];
+      colour = (key_x(key) & 1) + 2 * (key_y(key) & 1) + 4 * (key_z(key) & 1);
+    }
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const unsigned long long m = __ballot(colour == g);
+      if (colour == g) pre = __popcll(m & ((1ull << lane) - 1ull));
+      if (lane == 0) counts[g * WAVES + wave] = __popcll(m);
+    }
+    __syncthreads();
+    if (wave == 0) {  // exclusive scan of the 128 counts, two a lane
+      const int c0 = counts[2 * lane], c1 = counts[2 * lane + 1];
+      int sum = c0 + c1;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int l = __shfl_up(sum, o);
+        if (lane >= o) sum += l;
+      }
+      counts[2 * lane] = sum - c0 - c1;
+      counts[2 * lane + 1] = sum - c1;
+    }
+    __syncthreads();
+    if (colour >= 0) placed[counts[colour * WAVES + wave] + pre] = tid | (colour << 16);
+    __syncthreads();
+    const bool mine = tid < R;
+    const int p = mine ? placed[tid] : 0, row = p & 0xffff;  // row 0 exists (clamped loads)
+    const int group = mine ? p >> 16 : -1;
+    int at[27];
+    T v[27];
+    if (R > 0) {
+#pragma unroll
+      for (int k = 0; k < 27; ++k) {
+        at[k] = L.cols[k * R + row];
+        v[k] = L.vals[k * R + row];
+      }
+    }
+    T diagonal = T(0);
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+      const bool present = R > 0 && at[k] >= 0;
+      v[k] = present ? v[k] : T(0);
+      at[k] = present ? at[k] : ABSENT;
+      diagonal = at[k] == row ? v[k] : diagonal;
+    }
+    const T b = R > 0 ? L.rhs[row] : T(0);
+    const bool has = diagonal != T(0);
+    const T inv = has ? T(1) / diagonal : T(0);
+    const bool small = R <= 64;  // one wave holds the rows: its LDS accesses are in order
+    if (!small || wave == 0)
+      for (int it = 0; it < a.iters; ++it)
+        for (int c = 0; c < 8; ++c) {
+          if (group == (forward ? c : 7 - c)) {
+            T r = b;
+#pragma unroll
+            for (int k = 0; k < 27; ++k) r = r - xs[at[k]] * v[k];
+            if (has) xs[row] = xs[row] + r * inv;
+          }
+          if (small)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          else
+            __syncthreads();
+        }
+    if (small) __syncthreads();
+    if (residual) {
+      if (mine) {
+        T r = T(0);
+#pragma unroll
+        for (int k = 0; k < 27; ++k) r = r + v[k] * xs[at[k]];
+        r = r * T(-1);
+        other[row] = r + T(1) * b;
+      }
+      __syncthreads();
+    }
+    if (mine) L.x[tid] = xs[tid];
+  };
+  if (tid == 0) xs[ABSENT] = T(0);
+  for (int d = a.top; d > 0; --d) {
+    const BaseLevel<T>&L = a.level[d], &C = a.level[d - 1];
+    if (tid < L.R) xs[tid] = d < a.top || a.zero_top ? T(0) : L.x[tid];
+    relax(L, true, true);
+    if (tid < C.R) {
+      T v = T(0);
+#pragma unroll
+      for (int k = 0; k < 27; ++k) {
+        const int c = C.restr[k * C.R + tid];
+        const T t = v + T(restriction_weight(k)) * other[c >= 0 ? c : 0];
+        v = c >= 0 ? t : v;
+      }
+      C.rhs[tid] = v;
+    }
+    __syncthreads();
+  }
+  const BaseLevel<T>& root = a.level[0];
+  if (tid < root.R) {
+    root.x[tid] = T(0);
+    a.root_b[tid] = root.rhs[tid];
+    a.root_x[tid] = T(0);
+  }
+  __syncthreads();
+  if (tid == 0)
+    root_solve<T>(root.cols, root.vals, root.R, root.keys, root.rhs, root.x, (T*)nullptr, other, 0, a.base, a.cycle, a.acc, root.R,
+                  a.ran);
+  __syncthreads();
+  for (int d = 1; d <= a.top; ++d) {
+    const BaseLevel<T>&L = a.level[d], &C = a.level[d - 1];
+    if (tid < C.R) other[tid] = C.x[tid];
+    __syncthreads();
+    if (tid < L.R) {
+      T v = T(0);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int c = L.pcols[k * L.R + tid];
+        const T t = v + L.pvals[k * L.R + tid] * other[c >= 0 ? c : 0];
+        v = c >= 0 ? t : v;
+      }
+      v = v * T(1);
+      xs[tid] = v + T(1) * L.x[tid];
+    }
+    relax(L, false, false);
+    __syncthreads();
+  }
+}
+
 template <class T>
 void relax_colored(const GsOperator<T>& op, const Schedule<T>& sc, T* x, int iters, bool forward, hipStream_t s,
                    T* snap = nullptr) {
@@ -2771,28 +2861,6 @@ void relax_colored(const GsOperator<T>& op, const Schedule<T>& sc, T* x, int ite
                      (const int*)op.cols.data(), (const T*)op.vals.data(), (const T*)op.b.data(), (const T*)op.inv_diag.data(),
                      (const unsigned char*)op.has_diag.data(), x, op.R, iters, forward ? 1 : 0);
   KERNEL_CHECK();
-}
-
-// row_order (optional, device): output position j holds row row_order[j]
-template <class T> static Stencil<double> assemble_stiffness(const Result<T>& r, int depth, int trial_depth, hipStream_t s,
-                                                             const int* row_order = nullptr) {
-  const LevelState<T>&rowsL = r.levels[depth], &colsL = r.levels[trial_depth];
-  Stencil<double> m;
-  const int R = rowsL.basis_count;
-  m.rows = R;
-  m.cols_count = colsL.basis_count;
-  m.cols.reset(27 * (size_t)R, s);
-  m.vals.reset(27 * (size_t)R, s);
-  const int res = 1 << depth;
-  DArray<D2> table((res + 1) * 3, s);
-  hipLaunchKernelGGL(k_hat_table, dim3(blocks_for((res + 1) * 3, 256)), dim3(256), 0, s, depth, trial_depth, table.data());
-  KERNEL_CHECK();
-  if (R) {
-    hipLaunchKernelGGL(k_stiffness, dim3(blocks_for(R, 256)), dim3(256), 0, s, (const int64_t*)rowsL.basis_keys.data(), R,
-                       row_order, level_nodes(r, trial_depth), depth, trial_depth, (const D2*)table.data(), m.cols.data(), m.vals.data());
-    KERNEL_CHECK();
-  }
-  return m;
 }
 
 template <class T> struct PointSet {
@@ -2851,29 +2919,6 @@ template <class T> static PointBins<T> point_bins(const PointSet<T>& ps) {
                       ps.cell_start.empty() ? (const int*)nullptr : (const int*)ps.cell_start.data(),
                       ps.cell_end.empty() ? (const int*)nullptr : (const int*)ps.cell_end.data(), (const T*)ps.pos.data(),
                       (const T*)ps.w.data()};
-}
-
-template <class T>
-static void add_screening(Stencil<double>& m, const DArray<int64_t>& rows, const PointSet<T>& ps, int depth, int trial_depth,
-                          double* load, hipStream_t s, const int* row_order = nullptr) {
-  if (!m.rows) return;
-  hipLaunchKernelGGL(k_screening<T>, dim3(blocks_for(m.rows, 128)), dim3(128), 0, s, (const int64_t*)rows.data(), m.rows,
-                     row_order, depth, trial_depth, point_bins(ps), (const int*)m.cols.data(), m.vals.data(), load);
-  KERNEL_CHECK();
-}
-
-template <class T> static Stencil<T> cast_stencil(Stencil<double>&& m, hipStream_t s) {
-  Stencil<T> out;
-  out.rows = m.rows;
-  out.cols_count = m.cols_count;
-  out.cols = std::move(m.cols);
-  out.vals.reset(m.vals.size(), s);
-  if (m.vals.size()) {
-    hipLaunchKernelGGL(k_cast<T>, dim3(blocks_for(m.vals.size(), 256)), dim3(256), 0, s, (const double*)m.vals.data(),
-                       out.vals.data(), (int64_t)m.vals.size());
-    KERNEL_CHECK();
-  }
-  return out;
 }
 
 // LDS that a launch of the large assembly kernels (k_level_operator,
@@ -3339,84 +3384,102 @@ static void regular_multigrid(Result<T>& r, std::vector<DArray<int>>& restr, hip
                               const std::function<void()>& rhs_ready = {}) {
   const int base = r.prm.base_depth;
   LevelState<T>& B = r.levels[base];
-  std::vector<DArray<int>> mcols(base + 1);
-  std::vector<DArray<T>> mvals(base + 1);
+  // operators of levels 0..base: the base level's own, the others' products R A P
+  std::vector<DArray<int>> gcols(base);
+  std::vector<DArray<T>> gvals(base);
   std::vector<int> Rn(base + 1);
   for (int d = 0; d <= base; ++d) Rn[d] = r.levels[d].basis_count;
-  mcols[base].reset(27 * (size_t)Rn[base], s);
-  mvals[base].reset(27 * (size_t)Rn[base], s);
-  if (Rn[base]) {
-    HIP_CHECK(hipMemcpyAsync(mcols[base].data(), B.A.cols.data(), sizeof(int) * 27 * Rn[base], hipMemcpyDeviceToDevice, s));
-    HIP_CHECK(hipMemcpyAsync(mvals[base].data(), B.A.vals.data(), sizeof(T) * 27 * Rn[base], hipMemcpyDeviceToDevice, s));
-  }
+  auto mcols = [&](int d) { return (const int*)(d == base ? B.A.cols.data() : gcols[d].data()); };
+  auto mvals = [&](int d) { return (const T*)(d == base ? B.A.vals.data() : gvals[d].data()); };
   for (int d = base; d > 0; --d) {
     const int C = Rn[d - 1], F = Rn[d];
-    mcols[d - 1].reset(27 * (size_t)C, s);
-    mvals[d - 1].reset(27 * (size_t)C, s);
+    gcols[d - 1].reset(27 * (size_t)C, s);
+    gvals[d - 1].reset(27 * (size_t)C, s);
     if (C) {
-      hipLaunchKernelGGL(k_galerkin<T>, dim3(C), dim3(128), 0, s, (const int*)restr[d - 1].data(), C,
-                         (const int*)mcols[d].data(), (const T*)mvals[d].data(), F, (const int*)r.levels[d].P.cols.data(),
-                         (const T*)r.levels[d].P.vals.data(), mcols[d - 1].data(), mvals[d - 1].data(),
-                         (const int64_t*)r.levels[d - 1].basis_keys.data());
+      hipLaunchKernelGGL(k_galerkin<T>, dim3(C), dim3(128), 0, s, (const int*)restr[d - 1].data(), C, mcols(d), mvals(d), F,
+                         (const int*)r.levels[d].P.cols.data(), (const T*)r.levels[d].P.vals.data(), gcols[d - 1].data(),
+                         gvals[d - 1].data(), (const int64_t*)r.levels[d - 1].basis_keys.data());
       KERNEL_CHECK();
     }
   }
+  // levels 0..top run in one workgroup (k_base_cycle), the larger ones launch by launch
+  int top = 0;
+  while (top < base && Rn[top + 1] <= RELAX_BLOCK_REGS_ROWS) ++top;
+  if (Rn[0] > RELAX_BLOCK_REGS_ROWS) throw PsrError(1, "the root level has at most 8 nodes");
   std::vector<DArray<T>> rhs(base + 1), x(base + 1);
   for (int d = 0; d <= base; ++d) {
-    rhs[d].reset(Rn[d], s);
-    rhs[d].zero();
+    if (d < base) rhs[d].reset(Rn[d], s);
     x[d].reset(Rn[d], s);
-    x[d].zero();
+    if (d > top || base == 0) x[d].zero();
   }
-  std::vector<Schedule<T>> sched;
-  std::vector<GsOperator<T>> ops;
-  for (int d = 0; d <= base; ++d) {  // (the gathered b is replaced before each relaxation)
-    sched.push_back(make_schedule<T>(r.levels[d].basis_keys, Rn[d], d, false, s, false));
-    ops.push_back(gather_operator<T>(sched[d], mcols[d], mvals[d], rhs[d].data(), Rn[d], s));
+  std::vector<Schedule<T>> sched(base + 1);
+  std::vector<GsOperator<T>> ops(base + 1);
+  for (int d = top + 1; d <= base; ++d) {  // (the gathered b is replaced before each relaxation)
+    sched[d] = make_schedule<T>(r.levels[d].basis_keys, Rn[d], d, false, s, false);
+    ops[d] = gather_operator<T>(sched[d], mcols(d), mvals(d), (const T*)nullptr, Rn[d], s);
   }
   if (rhs_ready) rhs_ready();
-  if (Rn[base]) HIP_CHECK(hipMemcpyAsync(rhs[base].data(), B.rhs.data(), sizeof(T) * Rn[base], hipMemcpyDeviceToDevice, s));
+  auto rhs_of = [&](int d) { return d == base ? B.rhs.data() : rhs[d].data(); };
   const int dc = (base == 0 && r.prm.point_weight == 0.0) ? 1 : 0;
-  DArray<T> pad_x(64, s), work(256, s), residual;
-  pad_x.zero();
+  DArray<T> pad_x, work, residual;
+  if (base == 0) {
+    pad_x.reset(64, s);
+    pad_x.zero();
+    work.reset(256, s);
+  }
   r.cg_ran.reset((size_t)std::max(0, r.prm.base_v_cycles), s);
   const int iters = r.prm.iters;
   for (int cycle = 0; cycle < r.prm.base_v_cycles; ++cycle) {
-    for (int d = base; d > 0; --d) {
-      refresh_rhs(ops[d], sched[d], rhs[d].data(), s);
+    for (int d = base; d > top; --d) {
+      refresh_rhs(ops[d], sched[d], (const T*)rhs_of(d), s);
       relax_colored(ops[d], sched[d], x[d].data(), iters, true, s);
       residual.reset(Rn[d], s);
-      hipLaunchKernelGGL(k_spmv<T>, dim3(blocks_for(Rn[d], 256)), dim3(256), 0, s, (const int*)mcols[d].data(),
-                         (const T*)mvals[d].data(), Rn[d], 27, (const T*)x[d].data(), residual.data(), T(-1), T(1),
-                         (const T*)rhs[d].data());
+      hipLaunchKernelGGL(k_spmv<T>, dim3(blocks_for(Rn[d], 256)), dim3(256), 0, s, mcols(d), mvals(d), Rn[d], 27,
+                         (const T*)x[d].data(), residual.data(), T(-1), T(1), (const T*)rhs_of(d));
       KERNEL_CHECK();
       if (Rn[d - 1]) {
         hipLaunchKernelGGL(k_restrict_apply<T>, dim3(blocks_for(Rn[d - 1], 256)), dim3(256), 0, s,
                            (const int*)restr[d - 1].data(), Rn[d - 1], (const T*)residual.data(), rhs[d - 1].data(), 0);
         KERNEL_CHECK();
       }
-      x[d - 1].zero();
+      if (d - 1 > top) x[d - 1].zero();
     }
-    {  // the root solve's inputs, for the reverse pass
-      DArray<T> rb(std::max(Rn[0], 1), s), rx(64, s);
-      if (Rn[0]) HIP_CHECK(hipMemcpyAsync(rb.data(), rhs[0].data(), sizeof(T) * Rn[0], hipMemcpyDeviceToDevice, s));
+    // the root solve's inputs, for the reverse pass
+    DArray<T> rb(std::max(Rn[0], 1), s), rx(64, s);
+    if (base == 0) {
+      if (Rn[0]) HIP_CHECK(hipMemcpyAsync(rb.data(), B.rhs.data(), sizeof(T) * Rn[0], hipMemcpyDeviceToDevice, s));
       HIP_CHECK(hipMemcpyAsync(rx.data(), dc ? pad_x.data() : x[0].data(), sizeof(T) * (dc ? 64 : Rn[0]), hipMemcpyDeviceToDevice, s));
-      r.root_b.push_back(std::move(rb));
-      r.root_x.push_back(std::move(rx));
+      hipLaunchKernelGGL(k_root_solve<T>, dim3(1), dim3(64), 0, s, mcols(0), mvals(0), Rn[0],
+                         (const int64_t*)B.basis_keys.data(), (const T*)B.rhs.data(), x[0].data(), pad_x.data(), work.data(), dc,
+                         base, cycle, r.prm.cg_accuracy, Rn[0], r.cg_ran.data() + cycle);
+    } else {
+      BaseCycle<T> a{};
+      for (int d = 0; d <= top; ++d)
+        a.level[d] = BaseLevel<T>{r.levels[d].basis_keys.data(), mcols(d), mvals(d), r.levels[d].P.cols.data(),
+                                  r.levels[d].P.vals.data(), d < base ? restr[d].data() : nullptr, rhs_of(d), x[d].data(), Rn[d]};
+      a.top = top;
+      a.base = base;
+      a.cycle = cycle;
+      a.iters = iters;
+      a.zero_top = top < base || cycle == 0;
+      a.acc = r.prm.cg_accuracy;
+      a.ran = r.cg_ran.data() + cycle;
+      a.root_b = rb.data();
+      a.root_x = rx.data();
+      hipLaunchKernelGGL(k_base_cycle<T>, dim3(1), dim3(RELAX_BLOCK_REGS_ROWS), 0, s, a);
     }
-    hipLaunchKernelGGL(k_root_solve<T>, dim3(1), dim3(64), 0, s, (const int*)mcols[0].data(), (const T*)mvals[0].data(), Rn[0],
-                       (const int64_t*)r.levels[0].basis_keys.data(), (const T*)rhs[0].data(), x[0].data(), pad_x.data(),
-                       work.data(), dc, base, cycle, r.prm.cg_accuracy, Rn[0], r.cg_ran.data() + cycle);
     KERNEL_CHECK();
-    for (int d = 1; d <= base; ++d) {
+    r.root_b.push_back(std::move(rb));
+    r.root_x.push_back(std::move(rx));
+    for (int d = top + 1; d <= base; ++d) {
       hipLaunchKernelGGL(k_spmv<T>, dim3(blocks_for(Rn[d], 256)), dim3(256), 0, s, (const int*)r.levels[d].P.cols.data(),
                          (const T*)r.levels[d].P.vals.data(), Rn[d], 8, (const T*)x[d - 1].data(), x[d].data(), T(1), T(1),
                          (const T*)nullptr);
       KERNEL_CHECK();
-      x[d - 1].zero();
       relax_colored(ops[d], sched[d], x[d].data(), iters, false, s);
     }
   }
+  if (base > 0 && r.prm.base_v_cycles <= 0 && top == base) x[base].zero();
   if (dc && Rn[0]) {
     hipLaunchKernelGGL(k_root_extract<T>, dim3(1), dim3(64), 0, s, (const int64_t*)r.levels[0].basis_keys.data(), Rn[0],
                        (const T*)pad_x.data(), x[0].data());
@@ -3724,7 +3787,7 @@ template <class T, class V> class FinerAssembly {
 // The base solve, then each finer level once its operators and load are ready.
 template <class T, class V>
 static void solve_cascade(Result<T>& r, std::vector<DArray<int>>& restr, bool screened, FinerAssembly<T, V>& finer,
-                          hipEvent_t loads_ready, hipStream_t s) {
+                          const std::function<void()>& base_loads, hipEvent_t loads_ready, hipStream_t s) {
   const int base = r.prm.base_depth;
   DArray<T> cumulative;
   PreparedLevel<T> next;  // the coming finer level's buffers and graph
@@ -3734,17 +3797,18 @@ static void solve_cascade(Result<T>& r, std::vector<DArray<int>>& restr, bool sc
     if (!R) break;
     if (d == base) {
       L.point_load.reset(R, s);
-      L.point_load.zero();
       L.rhs.reset(R, s);
-      Stencil<double> A = assemble_stiffness(r, d, d, s);
-      if (screened) {
-        PointSet<T> pts = point_constraints(r, d, s);
-        add_screening(A, L.basis_keys, pts, d, d, L.point_load.data(), s);
-      }
-      L.A = cast_stencil<T>(std::move(A), s);
+      PointSet<T> pts;
+      if (screened)
+        pts = point_constraints(r, d, s);
+      else
+        L.point_load.zero();
+      level_operator<T, T>(r, d, d, screened ? &pts : nullptr, L.point_load.data(), (const int*)nullptr, (const int*)nullptr, L.A,
+                           (GsOperator<T, T>*)nullptr, (RowRecord<T, T>*)nullptr, (unsigned long long*)nullptr, s);
       // the base operators are set up while the normal loads finish on
       // their own stream; the right-hand side waits for them
       regular_multigrid(r, restr, s, [&] {
+        base_loads();
         HIP_CHECK(hipStreamWaitEvent(s, loads_ready, 0));
         hipLaunchKernelGGL(k_rhs<T>, dim3(blocks_for(R, 256)), dim3(256), 0, s, (const double*)L.normal_load.data(),
                            (const double*)L.point_load.data(), R, L.rhs.data());
@@ -3785,13 +3849,20 @@ static void solve_levels(Result<T>& r, std::vector<DArray<int>>& restr, bool scr
   HIP_CHECK(hipStreamWaitEvent(h, start, 0));
   {
     FinerAssembly<T, V> finer(r, base + 1, r.prm.solve_depth, screened, s);
-    normal_loads_base(r, restr, plan, h);
-    HIP_CHECK(hipEventRecord(loads_ready, h));
-    finer.set_loads(&plan);
-    solve_cascade<T, V>(r, restr, screened, finer, loads_ready, s);
+    // enqueued once the base operators' launches are, which need no loads
+    bool loads = false;
+    auto base_loads = [&] {
+      if (loads) return;
+      loads = true;
+      normal_loads_base(r, restr, plan, h);
+      HIP_CHECK(hipEventRecord(loads_ready, h));
+      finer.set_loads(&plan);
+    };
+    solve_cascade<T, V>(r, restr, screened, finer, base_loads, loads_ready, s);
+    base_loads();  // also when the cascade stopped before the base level
   }  // the solve stream is ordered after the assembly stream here
   group_finish();
-  HIP_CHECK(hipStreamWaitEvent(s, loads_ready, 0));  // also when the cascade stopped before the base level
+  HIP_CHECK(hipStreamWaitEvent(s, loads_ready, 0));
   (void)hipEventDestroy(start);
   (void)hipEventDestroy(loads_ready);
   normal_loads_rest(r, plan, s);
@@ -3883,7 +3954,7 @@ void relax_sliced_csr(const int64_t* keys, int R, const int* offsets, const int*
   KERNEL_CHECK();
   if (read_int(flag.data(), s)) throw PsrError(2, "relaxation rows hold at most 27 entries");
   Schedule<T> sc = make_schedule<T>(k, R, depth, true, s);
-  GsOperator<T> op = gather_operator<T>(sc, cols, vals, b, R, s);
+  GsOperator<T> op = gather_operator<T>(sc, cols.data(), vals.data(), b, R, s);
   (void)relax_sliced_any(op, sc, x, depth, iters, s);
 }
 
@@ -3907,7 +3978,7 @@ void relax_scheduled_csr(const int64_t* keys, int R, const int* offsets, const i
   KERNEL_CHECK();
   if (read_int(flag.data(), s)) throw PsrError(2, "relaxation rows hold at most 27 entries");
   Schedule<T> sc = make_schedule<T>(k, R, depth, z >= 0, s);
-  GsOperator<T> op = gather_operator<T>(sc, cols, vals, b, R, s);
+  GsOperator<T> op = gather_operator<T>(sc, cols.data(), vals.data(), b, R, s);
   if (z < 0 && R <= 65536) {
     relax_colored(op, sc, x, iters, forward != 0, s);
     return;
@@ -5014,15 +5085,12 @@ template <class T> void solve_backward(Result<T>& r, const double* gcoef, double
           KERNEL_CHECK();
         }
       }
-      // gather_operator reads b over each level's rows
-      DArray<T> zero_b(std::max(1, *std::max_element(Rn.begin(), Rn.end())), s);
-      zero_b.zero();
       std::vector<Schedule<T>> sched;
       std::vector<GsOperator<T>> ops;
       std::vector<DArray<T>> tvals(base + 1);
       for (int d = 0; d <= base; ++d) {
         sched.push_back(make_schedule<T>(r.levels[d].basis_keys, Rn[d], d, false, s, false));
-        ops.push_back(gather_operator<T>(sched[d], mcols[d], mvals[d], zero_b.data(), Rn[d], s));
+        ops.push_back(gather_operator<T>(sched[d], mcols[d].data(), mvals[d].data(), (const T*)nullptr, Rn[d], s));
         if (Rn[d] && Rn[d] <= RELAX_BLOCK_REGS_ROWS) {
           tvals[d].reset(27 * (size_t)Rn[d], s);
           hipLaunchKernelGGL(k_transpose_operator<T>, dim3(blocks_for(Rn[d], 256)), dim3(256), 0, s,
