@@ -3479,7 +3479,6 @@ static void regular_multigrid(Result<T>& r, std::vector<DArray<int>>& restr, hip
       relax_colored(ops[d], sched[d], x[d].data(), iters, false, s);
     }
   }
-  if (base > 0 && r.prm.base_v_cycles <= 0 && top == base) x[base].zero();
   if (dc && Rn[0]) {
     hipLaunchKernelGGL(k_root_extract<T>, dim3(1), dim3(64), 0, s, (const int64_t*)r.levels[0].basis_keys.data(), Rn[0],
                        (const T*)pad_x.data(), x[0].data());
